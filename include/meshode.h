@@ -174,9 +174,9 @@ typedef struct mo_lm_options {
   int32_t max_successful_steps;          /* > 0: stop after that many accepted steps (0) */
   int32_t team_vertices;                 /* pairs on the multi-workgroup kernel: vertices per
                                             workgroup of a pair's team (0: 4 * block_threads);
-                                            mo_deform_rot(_batch): > 0 puts each problem on a
-                                            team of that many vertices per workgroup (0: one
-                                            workgroup per problem) */
+                                            mo_deform_rot(_batch): largest chunk of a problem per
+                                            workgroup, at most 256 (512 above 16384 vertices; 0:
+                                            that) */
 } mo_lm_options;
 
 typedef struct mo_lm_stats {
@@ -434,13 +434,16 @@ int mo_linear_estimation(double* V, int64_t nv, const int32_t* F, int64_t nf, co
  * device array in the template's normalized frame: the rest shape in, the
  * solution out.  rot [nv,3] FP64 device array or null: the start rotations
  * (zeros when null, as the reference) in, the final ones out.  F [nf,3]
- * device.  opt.block_threads above 256 is clamped to 256.  Synchronizes
- * `stream`. */
+ * device.  A problem of up to 32768 vertices is solved on chip by one
+ * workgroup per chunk of 256 (512 above 16384) vertices; larger ones, hubs
+ * whose adjacency exceeds a chunk's LDS and devices that refuse a
+ * cooperative grid take one workgroup of opt.block_threads (at most 256)
+ * threads.  Synchronizes `stream`. */
 int mo_deform_rot(int32_t param_id, double* V, int64_t nv, const int32_t* F, int64_t nf, double lambda,
                   const mo_lm_options* opt, double* rot, mo_lm_stats* stats, void* stream);
 
-/* mo_deform_rot for a batch of independent problems in one launch (one
- * workgroup each): pair p deforms V[p] ([nv[p],3] FP64 device, normalized
+/* mo_deform_rot for a batch of independent problems, as many in one launch
+ * as are co-resident: pair p deforms V[p] ([nv[p],3] FP64 device, normalized
  * frame of template param_ids[p]) with faces F[p] ([nf[p],3]) and weight
  * lambda[p]; rot (nullable array, entries nullable) as in mo_deform_rot;
  * stats[p] per pair.  Each pair's result does not depend on the others. */

@@ -1888,64 +1888,22 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
     if (nf[p]) MO_HIP(hipMemcpyAsync(hF[p].data(), F[p], hF[p].size() * 4, hipMemcpyDeviceToHost, s));
   }
   MO_HIP(hipStreamSynchronize(s));
-  // per pair: half-edges in residual order (face, j), skipping a == b (Ceres
-  // rejects a residual block that names one parameter block twice), and
-  // each vertex's outgoing then incoming half-edges
-  std::vector<int2> hab;
-  std::vector<int4> vadj;
-  std::vector<int> vlist;
-  long long vtot = 0, htot = 0;
+  MO_CHECK(o.team_vertices >= 0, MO_ERR_ARG, "team_vertices must be >= 0");
+  long long vtot = 0;
   for (int p = 0; p < npairs; ++p) {
-    const int n = (int)nv[p];
     for (size_t k = 0; k < hF[p].size(); ++k)
-      MO_CHECK(hF[p][k] >= 0 && hF[p][k] < n, MO_ERR_ARG, "mo_deform_rot: pair %d: face index %d out of range", p,
+      MO_CHECK(hF[p][k] >= 0 && hF[p][k] < nv[p], MO_ERR_ARG, "mo_deform_rot: pair %d: face index %d out of range", p,
                hF[p][k]);
-    const size_t h0 = hab.size();
-    for (int64_t f = 0; f < nf[p]; ++f)
-      for (int j = 0; j < 3; ++j) {
-        const int a = hF[p][3 * f + j], b = hF[p][3 * f + (j + 1) % 3];
-        if (a != b) hab.push_back(make_int2(a, b));
-      }
-    const int nh = (int)(hab.size() - h0);
-    std::vector<int> nout(n, 0), nin(n, 0);
-    for (size_t h = h0; h < hab.size(); ++h) { nout[hab[h].x]++; nin[hab[h].y]++; }
-    const size_t v0 = vadj.size(), l0 = vlist.size();
-    int pos = 0;
-    for (int i = 0; i < n; ++i) {
-      vadj.push_back(make_int4(pos, nout[i], nin[i], 0));
-      pos += nout[i] + nin[i];
-    }
-    vlist.resize(l0 + (size_t)pos);
-    std::vector<int> fo(n), fi(n);
-    for (int i = 0; i < n; ++i) { fo[i] = vadj[v0 + i].x; fi[i] = vadj[v0 + i].x + vadj[v0 + i].y; }
-    for (int h = 0; h < nh; ++h) {
-      vlist[l0 + fo[hab[h0 + h].x]++] = h;
-      vlist[l0 + fi[hab[h0 + h].y]++] = h;
-    }
-    pd[p].nv = n;
-    pd[p].nh = nh;
+    pd[p].nv = (int)nv[p];
     pd[p].vbase = vtot;
-    pd[p].hbase = htot;
-    pd[p].lbase = (long long)l0;
-    vtot += n;
-    htot += nh;
+    vtot += nv[p];
   }
-  const long long hslots = htot ? htot : 1;
-  DevPtr d_x0, d_u, d_w, d_adj, d_list, d_hab, d_vw, d_hw, d_pair, d_res;
+  DevPtr d_x0, d_u, d_w, d_pair, d_res;
   if (int e_ = d_x0.alloc((size_t)vtot * 16)) return e_;
   if (int e_ = d_u.alloc((size_t)vtot * 16)) return e_;
   if (int e_ = d_w.alloc((size_t)vtot * 16)) return e_;
-  if (int e_ = d_adj.alloc((size_t)vtot * 16)) return e_;
-  if (int e_ = d_list.alloc(vlist.size() * 4)) return e_;
-  if (int e_ = d_hab.alloc((size_t)htot * 8)) return e_;
-  if (int e_ = d_vw.alloc((size_t)vtot * 16 * kRotVSlots)) return e_;
-  if (int e_ = d_hw.alloc((size_t)hslots * 16 * kRotHSlots)) return e_;
   if (int e_ = d_pair.alloc(npairs * sizeof(RotPairDesc))) return e_;
   if (int e_ = d_res.alloc(npairs * sizeof(LMResultDev))) return e_;
-  MO_HIP(hipMemcpyAsync(d_adj.p, vadj.data(), (size_t)vtot * 16, hipMemcpyHostToDevice, s));
-  if (!vlist.empty()) MO_HIP(hipMemcpyAsync(d_list.p, vlist.data(), vlist.size() * 4, hipMemcpyHostToDevice, s));
-  if (htot) MO_HIP(hipMemcpyAsync(d_hab.p, hab.data(), (size_t)htot * 8, hipMemcpyHostToDevice, s));
-  MO_HIP(hipMemcpyAsync(d_pair.p, pd.data(), npairs * sizeof(RotPairDesc), hipMemcpyHostToDevice, s));
   for (int p = 0; p < npairs; ++p) {
     const unsigned blocks = (unsigned)((nv[p] + 255) / 256);
     hipLaunchKernelGGL(k_rot_init, dim3(blocks), dim3(256), 0, s, V[p], rot ? rot[p] : nullptr, (int)nv[p],
@@ -1953,13 +1911,6 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
                        d_w.as<float4>() + pd[p].vbase);
   }
   MO_HIP(hipGetLastError());
-  RotArrays A{d_x0.as<float4>(), d_u.as<float4>(), d_w.as<float4>(), d_adj.as<int4>(), d_list.as<int>(),
-              d_hab.as<int2>(), d_vw.as<float4>(), d_hw.as<float4>()};
-  // team_vertices > 0: each problem on a team of ceil(nv / team_vertices)
-  // co-resident workgroups (k_lm_rot_team; at most lm_team_max()), packed
-  // largest first into cooperative launches, one such launch at a time in
-  // the process (team_launch_mutex); otherwise one workgroup per problem.
-  const int rbt = std::min(o.block_threads, 256);
   std::unique_lock<std::mutex> team_lock(team_launch_mutex(), std::defer_lock);
   struct TeamDrain {
     std::unique_lock<std::mutex>& lk;
@@ -1968,77 +1919,251 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
       if (lk.owns_lock()) (void)hipStreamSynchronize(s);
     }
   } team_drain{team_lock, s};
-  int path = MO_PATH_ONE_WORKGROUP;
+  std::vector<int> path(npairs, MO_PATH_ONE_WORKGROUP);
   std::vector<int> rot_wgs(npairs, 1);   // workgroups that solve each problem
-  DevPtr d_team;
+  std::vector<int> solo;                 // problems for the one-workgroup kernel in global memory
+  DevPtr d_chip[9];
   int* d_abort = nullptr;
   int rc;
-  MO_CHECK(o.team_vertices >= 0, MO_ERR_ARG, "team_vertices must be >= 0");
-  const int rcap = o.team_vertices > 0 ? lm_rot_team_capacity(rbt) : 0;
-  if (o.team_vertices > 0 && rcap >= lm_team_max()) {
-    std::vector<int> order(npairs);
-    std::iota(order.begin(), order.end(), 0);
-    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return nv[a] > nv[b]; });
-    std::vector<int> tc(npairs);
-    long long nwg_all = 0;
-    for (int t = 0; t < npairs; ++t) {
-      tc[t] = (int)std::min<long long>(std::max<long long>((nv[order[t]] + o.team_vertices - 1) / o.team_vertices, 1),
-                                       lm_team_max());
-      nwg_all += tc[t];
-      rot_wgs[order[t]] = tc[t];
+
+  // On-chip solver: chunks of at most 256 vertices (512 where 64 of those
+  // are not enough; options.team_vertices > 0 asks for smaller ones), one
+  // workgroup each.  A problem's chunks depend on the problem alone, so its
+  // result is the same in any batch.  A chunk whose records and adjacency
+  // do not fit the LDS (a halo or a vertex degree of thousands), or a
+  // problem above 64 x 512 vertices, takes the one-workgroup kernel.
+  const size_t lds_cap = 150 * 1024;
+  std::vector<int2> c_row((size_t)vtot);
+  std::vector<unsigned> c_ent;
+  std::vector<int> c_halo;
+  struct Plan { int threads; size_t lds; std::vector<RotChunk> chunks; };
+  std::vector<Plan> plan(npairs);
+  for (int p = 0; p < npairs; ++p) {
+    const int n = (int)nv[p];
+    const int threads = n <= 256 * kRotChipTeam ? 256 : kRotChip;
+    int c = (n + threads - 1) / threads;
+    if (o.team_vertices > 0) c = std::max(c, std::min(kRotChipTeam, (n + o.team_vertices - 1) / o.team_vertices));
+    if (c > kRotChipTeam) {
+      solo.push_back(p);
+      continue;
     }
-    std::vector<int4> wg;
-    std::vector<int> chunk_team{0}, chunk_wg{0};
-    int used = 0;
-    for (int t = 0; t < npairs; ++t) {
-      if (used + tc[t] > rcap) {
-        chunk_team.push_back(t);
-        chunk_wg.push_back((int)wg.size());
-        used = 0;
+    // neighbours of each vertex with the half-edges leaving to and arriving
+    // from it, merged; half-edges with a == b are skipped (Ceres rejects a
+    // residual block that names one parameter block twice)
+    std::vector<int> deg(n + 1, 0);
+    auto half_edges = [&](auto fn) {
+      for (int64_t f = 0; f < nf[p]; ++f)
+        for (int j = 0; j < 3; ++j) {
+          const int a = hF[p][3 * f + j], b = hF[p][3 * f + (j + 1) % 3];
+          if (a != b) fn(a, b);
+        }
+    };
+    half_edges([&](int a, int b) { deg[a + 1]++; deg[b + 1]++; });
+    for (int i = 0; i < n; ++i) deg[i + 1] += deg[i];
+    std::vector<int> list(deg[n]), fill(deg.begin(), deg.end() - 1);
+    half_edges([&](int a, int b) {
+      list[fill[a]++] = b << 1;          // leaves to b
+      list[fill[b]++] = (a << 1) | 1;    // arrives from a
+    });
+    Plan& L = plan[p];
+    L.threads = threads;
+    L.lds = 0;
+    const size_t ent0 = c_ent.size(), halo0 = c_halo.size();
+    std::vector<int> seen(n, -1), at(n, 0), record(n, -1);
+    const int ch = (n + c - 1) / c;
+    bool fits = true;
+    for (int r = 0; r < c && fits; ++r) {
+      RotChunk k{};
+      k.pid = p;
+      k.rank = r;
+      k.size = c;
+      k.lo = std::min(n, r * ch);
+      k.own = std::min(n, k.lo + ch) - k.lo;
+      k.ent = (long long)c_ent.size();
+      k.halo = (long long)c_halo.size();
+      for (int i = k.lo; i < k.lo + k.own; ++i) {
+        const int first = (int)(c_ent.size() - (size_t)k.ent);
+        for (int q = deg[i]; q < deg[i + 1]; ++q) {
+          const int j = list[q] >> 1;
+          const unsigned one = (list[q] & 1) ? 1u << 26 : 1u << 20;
+          const unsigned top = (list[q] & 1) ? c_ent.empty() ? 0u : c_ent[at[j]] >> 26
+                                             : c_ent.empty() ? 0u : (c_ent[at[j]] >> 20) & 63u;
+          if (seen[j] == i && top < (unsigned)kRotMaxMult) {
+            c_ent[at[j]] += one;
+            continue;
+          }
+          int rec = j - k.lo;
+          if (rec < 0 || rec >= k.own) {
+            if (record[j] < 0 || c_halo.size() <= (size_t)(k.halo + record[j]) || c_halo[k.halo + record[j]] != j) {
+              record[j] = (int)(c_halo.size() - (size_t)k.halo);
+              c_halo.push_back(j);
+            }
+            rec = threads + record[j];
+          }
+          seen[j] = i;
+          at[j] = (int)c_ent.size();
+          c_ent.push_back((unsigned)rec | one);
+        }
+        c_row[(size_t)pd[p].vbase + i] = make_int2(first, (int)(c_ent.size() - (size_t)k.ent) - first);
       }
-      for (int r = 0; r < tc[t]; ++r) wg.push_back(make_int4(t - chunk_team.back(), r, tc[t], 0));
-      used += tc[t];
+      k.nent = (int)(c_ent.size() - (size_t)k.ent);
+      k.nhalo = (int)(c_halo.size() - (size_t)k.halo);
+      L.lds = std::max(L.lds, lm_rot_chip_lds(threads, k.nhalo, k.nent));
+      fits = L.lds <= lds_cap && (size_t)threads + k.nhalo < (1u << 20);
+      L.chunks.push_back(k);
     }
-    chunk_team.push_back(npairs);
-    chunk_wg.push_back((int)wg.size());
-    const int per = lm_team_part_doubles();
-    const size_t b_tp = al(npairs * sizeof(int)), b_wg = al(nwg_all * sizeof(int4)),
-                 b_cnt = al(((size_t)npairs * 32 + 1) * sizeof(unsigned)), b_part = al((size_t)npairs * per * 8);
-    if (int e_ = d_team.alloc(b_tp + b_wg + b_cnt + b_part)) return e_;
-    char* base = d_team.as<char>();
-    int* d_tp = (int*)base;
-    int4* d_wg = (int4*)(base + b_tp);
-    unsigned* d_cnt = (unsigned*)(base + b_tp + b_wg);
-    double* d_part = (double*)(base + b_tp + b_wg + b_cnt);
-    d_abort = (int*)(d_cnt + (size_t)npairs * 32);
-    if ((rc = zero_fill(d_cnt, ((size_t)npairs * 32 + 1) * sizeof(unsigned), s))) return rc;
-    MO_HIP(hipMemcpyAsync(d_tp, order.data(), npairs * sizeof(int), hipMemcpyHostToDevice, s));
-    MO_HIP(hipMemcpyAsync(d_wg, wg.data(), wg.size() * sizeof(int4), hipMemcpyHostToDevice, s));
+    if (!fits) {
+      c_ent.resize(ent0);
+      c_halo.resize(halo0);
+      L.chunks.clear();
+      solo.push_back(p);
+      continue;
+    }
+    rot_wgs[p] = c;
+    path[p] = c > 1 ? MO_PATH_TEAM : MO_PATH_ONE_WORKGROUP;
+  }
+  // launches: largest problems first, as many as are co-resident together
+  // (teams wait for each other's members, so a launch with teams is
+  // cooperative; one such launch at a time in the process)
+  std::vector<int> order;
+  for (int p = 0; p < npairs; ++p)
+    if (!plan[p].chunks.empty()) order.push_back(p);
+  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return nv[a] > nv[b]; });
+  if (!order.empty()) {
+    struct Launch { int threads; size_t lds; bool coop; size_t c0, c1, p0; };
+    std::vector<Launch> launches;
+    std::vector<RotChunk> chunks;
+    int cap = 0;
+    size_t cap_lds = 0;
+    for (size_t q = 0; q < order.size(); ++q) {
+      const Plan& L = plan[order[q]];
+      const int c = (int)L.chunks.size();
+      Launch* cur = launches.empty() ? nullptr : &launches.back();
+      bool open = cur && cur->threads == L.threads;
+      if (open && L.lds > cap_lds) {
+        cap_lds = L.lds;
+        cap = lm_rot_chip_capacity(L.threads, cap_lds);
+      }
+      if (!open || (int)(chunks.size() - cur->c0) + c > cap) {
+        cap_lds = L.lds;
+        cap = lm_rot_chip_capacity(L.threads, cap_lds);
+        if (cap < c) {   // the team cannot be co-resident on this device
+          solo.push_back(order[q]);
+          path[order[q]] = MO_PATH_ONE_WORKGROUP;
+          rot_wgs[order[q]] = 1;
+          continue;
+        }
+        launches.push_back(Launch{L.threads, 0, false, chunks.size(), chunks.size(), q});
+        cur = &launches.back();
+      }
+      for (RotChunk k : L.chunks) {
+        k.team = (int)q;
+        chunks.push_back(k);
+      }
+      cur->lds = std::max(cur->lds, L.lds);
+      cur->coop = cur->coop || c > 1;
+      cur->c1 = chunks.size();
+    }
+    const size_t words = (size_t)lm_rot_chip_slot_words() * order.size();
+    enum { kRow, kEnt, kHalo, kEv, kEr, kEs, kPub, kSlots, kChunks };
+    const size_t ne = std::max<size_t>(c_ent.size(), 1);
+    const size_t bytes[9] = {(size_t)vtot * 8, ne * 4, c_halo.size() * 4, ne * 16, ne * 16, ne * 16,
+                             (size_t)vtot * 8 * kRotPubWords, words * 8 + 8, chunks.size() * sizeof(RotChunk)};
+    for (int k = 0; k < 9; ++k)
+      if (int e_ = d_chip[k].alloc(bytes[k])) return e_;
+    MO_HIP(hipMemcpyAsync(d_chip[kRow].p, c_row.data(), (size_t)vtot * 8, hipMemcpyHostToDevice, s));
+    if (!c_ent.empty())
+      MO_HIP(hipMemcpyAsync(d_chip[kEnt].p, c_ent.data(), c_ent.size() * 4, hipMemcpyHostToDevice, s));
+    if (!c_halo.empty())
+      MO_HIP(hipMemcpyAsync(d_chip[kHalo].p, c_halo.data(), c_halo.size() * 4, hipMemcpyHostToDevice, s));
+    MO_HIP(hipMemcpyAsync(d_chip[kChunks].p, chunks.data(), chunks.size() * sizeof(RotChunk), hipMemcpyHostToDevice, s));
+    MO_HIP(hipMemcpyAsync(d_pair.p, pd.data(), npairs * sizeof(RotPairDesc), hipMemcpyHostToDevice, s));
+    if ((rc = zero_fill(d_chip[kSlots].p, words * 8 + 8, s))) return rc;
     MO_HIP(hipStreamSynchronize(s));   // host vectors above go out of scope
-    team_lock.lock();
-    path = MO_PATH_TEAM;
-    for (size_t k = 0; k + 1 < chunk_team.size(); ++k) {
-      const int t0 = chunk_team[k];
-      rc = lm_rot_team_launch(d_pair.as<RotPairDesc>(), d_tp + t0, d_wg + chunk_wg[k], chunk_wg[k + 1] - chunk_wg[k],
-                              A, to_dev_options(o), d_res.as<LMResultDev>(), vtot, hslots, rbt,
-                              d_cnt + (size_t)t0 * 32, d_part + (size_t)t0 * per, d_abort, s);
+    const RotChipArrays CA{d_x0.as<float4>(), d_u.as<float4>(), d_w.as<float4>(), d_chip[kRow].as<int2>(),
+                           d_chip[kEnt].as<unsigned>(), d_chip[kHalo].as<int>(), d_chip[kEv].as<float4>(),
+                           d_chip[kEr].as<float4>(), d_chip[kEs].as<float4>(),
+                           d_chip[kPub].as<unsigned long long>()};
+    unsigned long long* slots = d_chip[kSlots].as<unsigned long long>();
+    d_abort = (int*)(slots + words);
+    for (size_t k = 0; k < launches.size(); ++k) {
+      const Launch& L = launches[k];
+      if (L.coop && !team_lock.owns_lock()) team_lock.lock();
+      rc = lm_rot_chip_launch(d_pair.as<RotPairDesc>(), d_chip[kChunks].as<RotChunk>() + L.c0, (int)(L.c1 - L.c0), CA,
+                              to_dev_options(o), d_res.as<LMResultDev>(), L.threads, L.lds, L.coop, slots, d_abort, s);
       if (rc == kCoopRefused && k == 0) {
         // the runtime refused the cooperative grid before any problem ran:
         // one workgroup per problem instead
-        if ((rc = lm_rot_launch(d_pair.as<RotPairDesc>(), npairs, A, to_dev_options(o), d_res.as<LMResultDev>(), vtot,
-                                hslots, rbt, s)))
-          return rc;
-        path = MO_PATH_COOP_REFUSED;
+        solo.resize(npairs);
+        std::iota(solo.begin(), solo.end(), 0);
+        std::fill(path.begin(), path.end(), MO_PATH_COOP_REFUSED);
         std::fill(rot_wgs.begin(), rot_wgs.end(), 1);
         break;
       }
       if (rc == kCoopRefused) return fail(MO_ERR_HIP, "DeformWithRot: cooperative launch refused after %zu chunks", k);
       if (rc) return rc;
     }
-  } else {
-    rc = lm_rot_launch(d_pair.as<RotPairDesc>(), npairs, A, to_dev_options(o), d_res.as<LMResultDev>(), vtot, hslots,
-                       rbt, s);
+  }
+  DevPtr d_adj, d_list, d_hab, d_vw, d_hw, d_pair1, d_res1;
+  if (!solo.empty()) {
+    // half-edges in residual order (face, j) and each vertex's outgoing then
+    // incoming half-edges
+    std::vector<int2> hab;
+    std::vector<int4> vadj((size_t)vtot);
+    std::vector<int> vlist;
+    std::vector<RotPairDesc> spd;
+    long long htot = 0;
+    for (int p : solo) {
+      const int n = (int)nv[p];
+      const size_t h0 = hab.size();
+      for (int64_t f = 0; f < nf[p]; ++f)
+        for (int j = 0; j < 3; ++j) {
+          const int a = hF[p][3 * f + j], b = hF[p][3 * f + (j + 1) % 3];
+          if (a != b) hab.push_back(make_int2(a, b));
+        }
+      const int nh = (int)(hab.size() - h0);
+      std::vector<int> nout(n, 0), nin(n, 0);
+      for (size_t h = h0; h < hab.size(); ++h) { nout[hab[h].x]++; nin[hab[h].y]++; }
+      const size_t v0 = (size_t)pd[p].vbase, l0 = vlist.size();
+      int pos = 0;
+      for (int i = 0; i < n; ++i) {
+        vadj[v0 + i] = make_int4(pos, nout[i], nin[i], 0);
+        pos += nout[i] + nin[i];
+      }
+      vlist.resize(l0 + (size_t)pos);
+      std::vector<int> fo(n), fi(n);
+      for (int i = 0; i < n; ++i) { fo[i] = vadj[v0 + i].x; fi[i] = vadj[v0 + i].x + vadj[v0 + i].y; }
+      for (int h = 0; h < nh; ++h) {
+        vlist[l0 + fo[hab[h0 + h].x]++] = h;
+        vlist[l0 + fi[hab[h0 + h].y]++] = h;
+      }
+      pd[p].nh = nh;
+      pd[p].hbase = htot;
+      pd[p].lbase = (long long)l0;
+      htot += nh;
+      spd.push_back(pd[p]);
+    }
+    const long long hslots = htot ? htot : 1;
+    if (int e_ = d_adj.alloc((size_t)vtot * 16)) return e_;
+    if (int e_ = d_list.alloc(vlist.size() * 4)) return e_;
+    if (int e_ = d_hab.alloc((size_t)htot * 8)) return e_;
+    if (int e_ = d_vw.alloc((size_t)vtot * 16 * kRotVSlots)) return e_;
+    if (int e_ = d_hw.alloc((size_t)hslots * 16 * kRotHSlots)) return e_;
+    if (int e_ = d_pair1.alloc(spd.size() * sizeof(RotPairDesc))) return e_;
+    if (int e_ = d_res1.alloc(spd.size() * sizeof(LMResultDev))) return e_;
+    MO_HIP(hipMemcpyAsync(d_adj.p, vadj.data(), (size_t)vtot * 16, hipMemcpyHostToDevice, s));
+    if (!vlist.empty()) MO_HIP(hipMemcpyAsync(d_list.p, vlist.data(), vlist.size() * 4, hipMemcpyHostToDevice, s));
+    if (htot) MO_HIP(hipMemcpyAsync(d_hab.p, hab.data(), (size_t)htot * 8, hipMemcpyHostToDevice, s));
+    MO_HIP(hipMemcpyAsync(d_pair1.p, spd.data(), spd.size() * sizeof(RotPairDesc), hipMemcpyHostToDevice, s));
+    MO_HIP(hipStreamSynchronize(s));   // host vectors above go out of scope
+    RotArrays A{d_x0.as<float4>(), d_u.as<float4>(), d_w.as<float4>(), d_adj.as<int4>(), d_list.as<int>(),
+                d_hab.as<int2>(), d_vw.as<float4>(), d_hw.as<float4>()};
+    rc = lm_rot_launch(d_pair1.as<RotPairDesc>(), (int)spd.size(), A, to_dev_options(o), d_res1.as<LMResultDev>(), vtot,
+                       hslots, std::min(o.block_threads, 256), s);
     if (rc) return rc;
+    for (size_t q = 0; q < solo.size(); ++q)
+      MO_HIP(hipMemcpyAsync(d_res.as<LMResultDev>() + solo[q], d_res1.as<LMResultDev>() + q, sizeof(LMResultDev),
+                            hipMemcpyDeviceToDevice, s));
   }
   if (d_abort) {
     // invalid solutions after a barrier wait ran out: raise before the
@@ -2072,7 +2197,7 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
       o2.pcg_iterations = r[p].pcg_iterations;
       o2.clock_start = r[p].clock_start;
       o2.clock_end = r[p].clock_end;
-      o2.solver_path = path;
+      o2.solver_path = path[p];
       o2.workgroups = rot_wgs[p];
     }
   return MO_OK;

@@ -1,6 +1,9 @@
 // Levenberg-Marquardt solve of Deformer::DeformWithRot (deformer.cc:94-171)
-// on gfx950: one workgroup per problem, the whole trust-region loop in one
-// persistent kernel (the loop of mo_lm_util.h).
+// on gfx950: the whole trust-region loop in one persistent kernel (the loop
+// of mo_lm_util.h), on chip on one workgroup per 256-vertex chunk of the
+// problem (k_lm_rot_chip below), or, for problems that kernel does not hold
+// and where the runtime refuses a cooperative grid, on one workgroup with
+// its vectors in global memory (k_lm_rot).
 //
 // Unknowns per vertex i: the position p_i = x0_i + u_i and an angle-axis
 // rotation w_i (zero at the start, deformer.cc:114).  Residuals:
@@ -14,7 +17,7 @@
 // G_h = dq/dw at (w_a, p_a - p_b)) and I (w_a), -I (w_b) for the last three.
 //
 // Per LM step, (J^T J + D^2) delta = -J^T f is solved by PCG with FP32
-// vectors and FP64 reductions; J^T J x is formed matrix-free in two passes
+// vectors and FP64 reductions; in k_lm_rot J^T J x is formed matrix-free in two passes
 // (per half-edge: t = lambda (A_a (x_pa - x_pb) + G_h x_wa) and
 // s = x_wa - x_wb and their transposed images; per vertex: the gather over
 // its outgoing and incoming half-edges), preconditioned by the inverse of
@@ -454,17 +457,391 @@ __global__ void __launch_bounds__(256) k_lm_rot(const RotPairDesc* __restrict__ 
   lm_rot_pair(pairs[pid], res + pid, A, opt, totalV, totalH, team, red);
 }
 
-// wg[b] = (team, rank, team size, -): team t solves problem plist[t].
-__global__ void __launch_bounds__(256) k_lm_rot_team(const RotPairDesc* __restrict__ pairs,
-                                                      const int* __restrict__ plist, const int4* __restrict__ wg,
-                                                      RotArrays A, LMOptionsDev opt, LMResultDev* __restrict__ res,
-                                                      long long totalV, long long totalH, unsigned* cnt, double* part,
-                                                      int* abort_flag, long long limit) {
-  __shared__ double red[2 * 8 * kMaxWaves];
-  const int4 m = wg[blockIdx.x];
-  const int pid = plist[m.x];
-  GridTeam team{m.y, m.z, cnt + (size_t)m.x * 32, part + (size_t)m.x * 2 * kMaxTeam * 8, abort_flag, limit, 0u, 0};
-  lm_rot_pair(pairs[pid], res + pid, A, opt, totalV, totalH, team, red);
+// ---------------------------------------------------------------------------
+// The on-chip solver.  With R = A_a (a rotation: A^T A = I) and J = the right
+// Jacobian of the exponential map at w_a, dq/dw x = R ((J x) x e), so for a
+// half-edge h = (a, b) with e = p_a - p_b the residual's directional
+// derivative is
+//     lambda R y,   y = x_pa - x_pb + omega_a x e,   omega_a = J x_wa,
+// and its transpose images are lambda^2 y at p_a, -lambda^2 y at p_b and
+// lambda^2 J^T (e x y) at w_a: no matrix per half-edge is left, and a vertex
+// needs nine floats of each neighbour (x_p, x_w, omega) and the edge vector.
+// (In the first-order branch, |w|^2 <= double epsilon, J = I and A = I + [w]x
+// is orthogonal to 1e-16.)
+//
+// One thread per vertex holds the vertex's whole PCG state in registers; a
+// workgroup holds a chunk of consecutive vertices, its LDS the chunk's
+// records and its halo's, and the adjacency with the edge vectors.  A PCG
+// iteration publishes z = M^-1 r once, loads the halo's records, forms
+// A z, p = z + beta p and A p = A z + beta A p_prev, and needs the two
+// reductions of CG and no other exchange; the team protocol is TagTeam.
+// What bounds it: the two exchanges and the halo load of an iteration, each
+// a round trip through memory shared by the XCDs, not arithmetic (about
+// 5.7 us an iteration).  One 5000-vertex problem (20 chunks, 4600 PCG
+// iterations): 26.3 ms, where k_lm_rot takes 990 ms on its one CU.  Chunks
+// of 256 put one wavefront on each SIMD of a CU; 21 VGPRs of the cold parts
+// spill at two workgroups per CU.
+__device__ inline float3 cross3(float3 a, float3 b) {
+  return make_float3(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x);
+}
+__device__ inline float dotf(float3 a, float3 b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+__device__ inline float3 madd(float3 a, float s, float3 b) {   // a + s b
+  return make_float3(a.x + s * b.x, a.y + s * b.y, a.z + s * b.z);
+}
+__device__ inline float3 m9v(const float (&m)[9], float3 v) {
+  return make_float3(m[0] * v.x + m[1] * v.y + m[2] * v.z, m[3] * v.x + m[4] * v.y + m[5] * v.z,
+                     m[6] * v.x + m[7] * v.y + m[8] * v.z);
+}
+__device__ inline float3 m9tv(const float (&m)[9], float3 v) {
+  return make_float3(m[0] * v.x + m[3] * v.y + m[6] * v.z, m[1] * v.x + m[4] * v.y + m[7] * v.z,
+                     m[2] * v.x + m[5] * v.y + m[8] * v.z);
+}
+
+// Right Jacobian of the rotation at w: I - a [w]x + b [w]x^2 with
+// a = (1 - cos t) / t^2 = 2 sin^2(t / 2) / t^2, b = (t - sin t) / t^3 (its
+// series below t = 1, where the difference cancels); I in the first-order
+// branch.
+__device__ inline void right_jacobian(const float3 w, float (&J)[9]) {
+  const float t2 = dotf(w, w);
+  float a = 0.f, b = 0.f;
+  if (t2 > kAngleAxisEps) {
+    const float t = sqrtf(t2);
+    const float h = sinf(0.5f * t);
+    a = 2.f * h * h / t2;
+    b = t2 < 1.f ? 1.f / 6.f + t2 * (-1.f / 120.f + t2 * (1.f / 5040.f + t2 * (-1.f / 362880.f + t2 / 39916800.f)))
+                 : (t - sinf(t)) / (t2 * t);
+  }
+  const float d = 1.f - b * t2;
+  J[0] = d + b * w.x * w.x;     J[1] = b * w.x * w.y + a * w.z; J[2] = b * w.x * w.z - a * w.y;
+  J[3] = b * w.x * w.y - a * w.z; J[4] = d + b * w.y * w.y;     J[5] = b * w.y * w.z + a * w.x;
+  J[6] = b * w.x * w.z + a * w.y; J[7] = b * w.y * w.z - a * w.x; J[8] = d + b * w.z * w.z;
+}
+
+__device__ inline unsigned long long pack2(float a, float b) {
+  return (unsigned long long)__float_as_uint(a) | ((unsigned long long)__float_as_uint(b) << 32);
+}
+
+template <int T>
+__global__ void __launch_bounds__(T, T == 256 ? 2 : 1) k_lm_rot_chip(
+    const RotPairDesc* __restrict__ pairs, const RotChunk* __restrict__ chunks, RotChipArrays A, LMOptionsDev opt,
+    LMResultDev* __restrict__ res, unsigned long long* slots, int* abort_flag, long long limit) {
+  extern __shared__ __align__(16) float4 smem4[];
+  __shared__ double red[kTagRed];
+  const RotChunk C = chunks[blockIdx.x];
+  const RotPairDesc P = pairs[C.pid];
+  float4* __restrict__ REC = smem4;                                // 3 float4 per record
+  float4* __restrict__ LE = smem4 + 3 * (T + C.nhalo);             // edge vector and packed entry
+  const int tid = threadIdx.x;
+  const bool mine = tid < C.own;
+  const int i = C.lo + (mine ? tid : 0);
+  const long long vi = P.vbase + i;
+  const float lam = P.lambda, l2 = lam * lam;
+  TagTeam team{C.rank, C.size, slots + (size_t)C.team * kTagSlotWords, abort_flag, limit, red, 0u, 0};
+  const long long clock_start = wall_clock64();
+  const int2 row = A.row[vi];
+  const int e0 = mine ? row.x : 0, e1 = mine ? row.x + row.y : 0;
+  const unsigned* __restrict__ ENT = A.ent + C.ent;
+  float4* __restrict__ EV = A.ev + C.ent;
+  float4* __restrict__ ER = A.er + C.ent;
+  float4* __restrict__ ES = A.es + C.ent;
+  const int* __restrict__ HALO = A.halo + C.halo;
+  unsigned long long* PUB = A.pub + P.vbase * kRotPubWords;
+
+  const float3 x0 = f3(A.x0[vi]);
+  float3 u = f3(A.u[vi]), w = f3(A.w[vi]);
+  float3 g = make_float3(0.f, 0.f, 0.f), gp = g, gw = g;
+  float dist = 0.f;
+  float J[9];                       // right Jacobian at w
+  double S1[3], S2[6];              // sums over outgoing edges: e, |e|^2 I - e e^T
+  float cnt = 0.f;                  // half-edges at the vertex
+  float sc[6], dg[6], dt[6], Mi[21];
+  float3 zp, zw, zo, pp, pw, qp, qw, rp, rw, dlp, dlw;
+  dlp = dlw = pp = pw = qp = qw = rp = rw = zp = zw = zo = make_float3(0.f, 0.f, 0.f);
+  for (int k = 0; k < 6; ++k) sc[k] = dg[k] = dt[k] = 0.f;
+
+  // this vertex's nine published floats, to LDS and, for teams, to memory
+  auto publish = [&](float3 a, float3 b, float3 c) {
+    if (!mine) return;
+    REC[3 * tid] = make_float4(a.x, a.y, a.z, b.x);
+    REC[3 * tid + 1] = make_float4(b.y, b.z, c.x, c.y);
+    REC[3 * tid + 2].x = c.z;
+    if (C.size > 1) {
+      unsigned long long* d = PUB + (size_t)i * kRotPubWords;
+      const unsigned long long v[kRotPubWords] = {pack2(a.x, a.y), pack2(a.z, b.x), pack2(b.y, b.z), pack2(c.x, c.y),
+                                                  pack2(c.z, 0.f)};
+      for (int k = 0; k < kRotPubWords; ++k)
+        __hip_atomic_store(d + k, v[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  };
+  // the halo's records, after the exchange that ended their publication
+  auto stage = [&]() {
+    for (int k = tid; k < C.nhalo; k += T) {
+      unsigned long long* d = PUB + (size_t)HALO[k] * kRotPubWords;
+      unsigned long long v[kRotPubWords];
+      for (int q = 0; q < kRotPubWords; ++q) v[q] = __hip_atomic_load(d + q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      float f[2 * kRotPubWords];
+      for (int q = 0; q < kRotPubWords; ++q) {
+        f[2 * q] = __uint_as_float((unsigned)v[q]);
+        f[2 * q + 1] = __uint_as_float((unsigned)(v[q] >> 32));
+      }
+      float4* R = REC + 3 * (T + k);
+      R[0] = make_float4(f[0], f[1], f[2], f[3]);
+      R[1] = make_float4(f[4], f[5], f[6], f[7]);
+      R[2].x = f[8];
+    }
+    if (C.nhalo) __syncthreads();
+  };
+  auto record = [&](unsigned e, float3& a, float3& b, float3& c) {
+    const float4* R = REC + 3 * (e & 0xFFFFFu);
+    const float4 r0 = R[0], r1 = R[1];
+    a = make_float3(r0.x, r0.y, r0.z);
+    b = make_float3(r0.w, r1.x, r1.y);
+    c = make_float3(r1.z, r1.w, R[2].x);
+  };
+  auto out_mult = [](unsigned e) { return (float)((e >> 20) & 63u); };
+  auto in_mult = [](unsigned e) { return (float)(e >> 26); };
+
+  // ---- residuals, gradient J^T f, edge vectors and block sums, cost --------
+  auto eval = [&](bool first, double& cv, double& ce, double& gmax) {
+    publish(u, w, x0);
+    team.barrier();
+    stage();
+    double v[3] = {0.0, 0.0, 0.0};
+    if (mine) {
+      const JetF L = lookup_jet(P.grid, P.N, x0.x + u.x, x0.y + u.y, x0.z + u.z);
+      g = make_float3(L.v0, L.v1, L.v2);
+      dist = L.a;
+      v[0] = 0.5 * (double)dist * (double)dist;
+      const float wv[3] = {w.x, w.y, w.z};
+      float Am[9];
+      rotation_point_jacobian(wv, Am);
+      right_jacobian(w, J);
+      gp = mul(g, dist);
+      gw = make_float3(0.f, 0.f, 0.f);
+      float3 tor = gw;
+      cnt = 0.f;
+      for (int k = 0; k < 3; ++k) S1[k] = 0.0;
+      for (int k = 0; k < 6; ++k) S2[k] = 0.0;
+      for (int k = e0; k < e1; ++k) {
+        const unsigned pk = ENT[k];
+        float3 un, wn, xn;
+        record(pk, un, wn, xn);
+        const float mo = out_mult(pk), mi = in_mult(pk);
+        const float3 vh = sub(x0, xn);
+        const float3 e = add(vh, sub(u, un));
+        const float3 sg = sub(w, wn);
+        LE[k] = make_float4(e.x, e.y, e.z, __uint_as_float(pk));
+        float3 cr = make_float3(0.f, 0.f, 0.f);
+        if (mo > 0.f) {
+          const float3 r = mul(sub(m9v(Am, e), vh), lam);
+          const float3 t = mul(m9tv(Am, r), lam);
+          cr = t;
+          gp = madd(gp, mo, t);
+          tor = madd(tor, mo, cross3(e, t));
+          v[1] += 0.5 * (double)mo * (dot3(r, r) + dot3(sg, sg));
+          const double ex = e.x, ey = e.y, ez = e.z, m = mo;
+          S1[0] += m * ex; S1[1] += m * ey; S1[2] += m * ez;
+          S2[0] += m * (ey * ey + ez * ez); S2[1] -= m * ex * ey; S2[2] -= m * ex * ez;
+          S2[3] += m * (ex * ex + ez * ez); S2[4] -= m * ey * ez; S2[5] += m * (ex * ex + ey * ey);
+        }
+        if (mi > 0.f) {          // half-edge (j, i): its edge vector is -e, its rest edge -vh
+          const float wj[3] = {wn.x, wn.y, wn.z};
+          float Aj[9];
+          rotation_point_jacobian(wj, Aj);
+          const float3 r = mul(sub(vh, m9v(Aj, e)), lam);
+          gp = madd(gp, -mi * lam, m9tv(Aj, r));
+        }
+        gw = madd(gw, mo + mi, sg);
+        cnt += mo + mi;
+        EV[k] = f4(vh);
+        ER[k] = f4(cr);
+        ES[k] = f4(sg);
+      }
+      gw = add(gw, m9tv(J, tor));
+      const float3 m1 = absmax3(gp), m2 = absmax3(gw);
+      v[2] = (double)fmaxf(fmaxf(fmaxf(m1.x, m1.y), fmaxf(m1.z, m2.x)), fmaxf(m2.y, m2.z));
+    }
+    team.template reduce<2, 1>(v);
+    cv = v[0]; ce = v[1]; gmax = v[2];
+    (void)first;
+  };
+
+  // J^T J diagonal block (6x6, p then w): g g^T + l2 cnt I, -l2 [S1]x J, l2 J^T S2 J + cnt I
+  auto block = [&](double (&M)[6][6]) {
+    const double gv[3] = {g.x, g.y, g.z};
+    const double K1[3][3] = {{0.0, -S1[2], S1[1]}, {S1[2], 0.0, -S1[0]}, {-S1[1], S1[0], 0.0}};
+    const double K2[3][3] = {{S2[0], S2[1], S2[2]}, {S2[1], S2[3], S2[4]}, {S2[2], S2[4], S2[5]}};
+    for (int r = 0; r < 3; ++r)
+      for (int c = 0; c < 3; ++c) {
+        M[r][c] = gv[r] * gv[c] + (r == c ? (double)l2 * cnt : 0.0);
+        double pwv = 0.0, wwv = 0.0;
+        for (int m = 0; m < 3; ++m) {
+          pwv -= K1[r][m] * (double)J[3 * m + c];
+          double t = 0.0;
+          for (int q = 0; q < 3; ++q) t += K2[m][q] * (double)J[3 * q + c];
+          wwv += (double)J[3 * m + r] * t;
+        }
+        M[r][3 + c] = l2 * pwv;
+        M[3 + c][r] = l2 * pwv;
+        M[3 + r][3 + c] = l2 * wwv + (r == c ? (double)cnt : 0.0);
+      }
+  };
+  auto minv = [&](float3 a, float3 b, float3& ya, float3& yb) {
+    const float r[6] = {a.x, a.y, a.z, b.x, b.y, b.z};
+    float y[6];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) {
+      float t = 0.f;
+#pragma unroll
+      for (int n = 0; n < 6; ++n) t += Mi[sym6(m, n)] * r[n];
+      y[m] = t;
+    }
+    ya = make_float3(y[0], y[1], y[2]);
+    yb = make_float3(y[3], y[4], y[5]);
+  };
+
+  bool scaled = false;
+  // ---- LM diagonal, preconditioner, PCG ------------------------------------
+  auto solve = [&](bool reuse, double radius) -> int {
+    double v[2] = {0.0, 0.0};
+    if (mine) {
+      const double inv_radius = 1.0 / radius;
+      double M[6][6];
+      block(M);
+      if (!scaled)
+        for (int k = 0; k < 6; ++k) sc[k] = (float)(1.0 / (1.0 + sqrt(M[k][k])));
+      if (!reuse)
+        for (int k = 0; k < 6; ++k) {
+          double t = (double)sc[k] * sc[k] * M[k][k];
+          t = t < opt.min_lm_diagonal ? opt.min_lm_diagonal : (t > opt.max_lm_diagonal ? opt.max_lm_diagonal : t);
+          dg[k] = (float)t;
+        }
+      for (int k = 0; k < 6; ++k) {
+        const double t = (double)dg[k] / ((double)sc[k] * sc[k]) * inv_radius;
+        dt[k] = (float)(t < 1e30 ? t : 1e30);
+        M[k][k] += dt[k];
+      }
+      if (!spd6_inverse(M, Mi)) {
+        for (int k = 0; k < 21; ++k) Mi[k] = 0.f;
+        for (int k = 0; k < 6; ++k) Mi[sym6(k, k)] = M[k][k] > 0.0 ? (float)(1.0 / M[k][k]) : 0.f;
+      }
+      rp = mul(gp, -1.f);
+      rw = mul(gw, -1.f);
+      minv(rp, rw, zp, zw);
+      zo = m9v(J, zw);
+      dlp = dlw = pp = pw = qp = qw = make_float3(0.f, 0.f, 0.f);
+      v[0] = dot3(rp, zp) + dot3(rw, zw);
+      v[1] = dot3(rp, rp) + dot3(rw, rw);
+    }
+    scaled = true;
+    publish(zp, zw, zo);
+    team.template reduce<2, 0>(v);
+    double rz = v[0];
+    const double tol2 = (double)opt.pcg_relative_tolerance * opt.pcg_relative_tolerance * v[1];
+    if (!(v[1] > 0.0)) return 0;
+    float beta = 0.f;
+    int k = 0;
+    for (; k < opt.pcg_max_iterations; ++k) {
+      stage();
+      double v1[1] = {0.0};
+      if (mine) {
+        const float gd = dotf(g, zp);
+        float3 ap = make_float3(0.f, 0.f, 0.f), aw = ap, tor = ap;
+        for (int n = e0; n < e1; ++n) {
+          const float4 le = LE[n];
+          const unsigned pk = __float_as_uint(le.w);
+          const float3 e = f3(le);
+          float3 a, b, c;
+          record(pk, a, b, c);
+          const float mo = out_mult(pk), mi = in_mult(pk);
+          const float3 d = sub(zp, a);
+          const float3 y = add(d, cross3(zo, e));
+          const float3 om = make_float3(mo * zo.x + mi * c.x, mo * zo.y + mi * c.y, mo * zo.z + mi * c.z);
+          ap = add(ap, madd(cross3(om, e), mo + mi, d));
+          aw = madd(aw, mo + mi, sub(zw, b));
+          tor = madd(tor, mo, cross3(e, y));
+        }
+        tor = m9tv(J, tor);
+        ap = make_float3(l2 * ap.x + g.x * gd + dt[0] * zp.x, l2 * ap.y + g.y * gd + dt[1] * zp.y,
+                         l2 * ap.z + g.z * gd + dt[2] * zp.z);
+        aw = make_float3(aw.x + l2 * tor.x + dt[3] * zw.x, aw.y + l2 * tor.y + dt[4] * zw.y,
+                         aw.z + l2 * tor.z + dt[5] * zw.z);
+        pp = madd(zp, beta, pp);
+        pw = madd(zw, beta, pw);
+        qp = madd(ap, beta, qp);
+        qw = madd(aw, beta, qw);
+        v1[0] = dot3(pp, qp) + dot3(pw, qw);
+      }
+      team.template reduce<1, 0>(v1);
+      if (!(v1[0] > 0.0)) break;
+      const float fa = (float)(rz / v1[0]);
+      double v2[2] = {0.0, 0.0};
+      if (mine) {
+        dlp = madd(dlp, fa, pp);
+        dlw = madd(dlw, fa, pw);
+        rp = madd(rp, -fa, qp);
+        rw = madd(rw, -fa, qw);
+        minv(rp, rw, zp, zw);
+        zo = m9v(J, zw);
+        v2[0] = dot3(rp, zp) + dot3(rw, zw);
+        v2[1] = dot3(rp, rp) + dot3(rw, rw);
+      }
+      publish(zp, zw, zo);
+      team.template reduce<2, 0>(v2);
+      beta = (float)(v2[0] / rz);
+      rz = v2[0];
+      if (v2[1] <= tol2) { ++k; break; }
+    }
+    return k;
+  };
+
+  // ---- model cost change, candidate cost, step and parameter norms ---------
+  auto candidate = [&]() -> LMCandidate {
+    publish(dlp, dlw, dlw);
+    team.barrier();
+    stage();
+    double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if (mine) {
+      const float gd = dotf(g, dlp);
+      v[0] = (double)gd * ((double)dist + 0.5 * (double)gd);
+      const float dc = lookup_f32(P.grid, P.N, x0.x + (u.x + dlp.x), x0.y + (u.y + dlp.y), x0.z + (u.z + dlp.z));
+      v[1] = 0.5 * (double)dc * (double)dc;
+      v[3] = dot3(dlp, dlp) + dot3(dlw, dlw);
+      const float3 x = add(x0, u);
+      v[4] = dot3(x, x) + dot3(w, w);
+      const float3 om = m9v(J, dlw);
+      const float wv[3] = {w.x + dlw.x, w.y + dlw.y, w.z + dlw.z};
+      float Am[9];
+      rotation_point_jacobian(wv, Am);
+      for (int n = e0; n < e1; ++n) {
+        const float4 le = LE[n];
+        const unsigned pk = __float_as_uint(le.w);
+        const float mo = out_mult(pk);
+        if (!(mo > 0.f)) continue;
+        const float3 e = f3(le);
+        float3 a, b, c;
+        record(pk, a, b, c);
+        const float3 d = sub(dlp, a), ms = sub(dlw, b);
+        const float3 y = add(d, cross3(om, e));
+        const float3 sg = f3(ES[n]);
+        v[0] += (double)mo * (dot3(y, f3(ER[n])) + 0.5 * (double)l2 * dot3(y, y) + dot3(ms, madd(sg, 0.5f, ms)));
+        const float3 rc = mul(sub(m9v(Am, add(e, d)), f3(EV[n])), lam);
+        const float3 s2 = add(sg, ms);
+        v[2] += 0.5 * (double)mo * (dot3(rc, rc) + dot3(s2, s2));
+      }
+    }
+    team.template reduce<5, 0>(v);
+    return LMCandidate{-v[0], v[1] + v[2], sqrt(v[3]), sqrt(v[4])};
+  };
+  auto accept = [&]() {
+    u = add(u, dlp);
+    w = add(w, dlw);
+  };
+  lm_trust_region_loop(opt, eval, solve, candidate, accept, team.leader() ? res + C.pid : nullptr, clock_start);
+  if (mine) {
+    A.u[vi] = f4(u);
+    A.w[vi] = f4(w);
+  }
 }
 
 }  // namespace
@@ -481,39 +858,53 @@ int lm_rot_launch(const RotPairDesc* pairs_dev, int npairs, const RotArrays& arr
   return MO_OK;
 }
 
-int lm_rot_team_capacity(int block_threads) {
+size_t lm_rot_chip_lds(int threads, int nhalo, int nent) {
+  return 48 * ((size_t)threads + (size_t)nhalo) + 16 * (size_t)nent;
+}
+
+int lm_rot_chip_slot_words() { return kTagSlotWords; }
+
+static const void* chip_kernel(int threads) {
+  return threads == 256 ? (const void*)k_lm_rot_chip<256> : (const void*)k_lm_rot_chip<512>;
+}
+
+int lm_rot_chip_capacity(int threads, size_t lds_bytes) {
   int dev = 0, cus = 0, per = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
+  if (hipFuncSetAttribute(chip_kernel(threads), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) !=
+          hipSuccess ||
+      hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_lm_rot_team, block_threads, 0) != hipSuccess)
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, chip_kernel(threads), threads, lds_bytes) != hipSuccess) {
+    (void)hipGetLastError();
     return 0;
+  }
   return per * cus;
 }
 
-int lm_rot_team_launch(const RotPairDesc* pairs_dev, const int* plist, const int4* wg_dev, int nwg,
-                       const RotArrays& arrays, const LMOptionsDev& opt, LMResultDev* results_dev,
-                       long long total_vertices, long long total_half_edges, int block_threads, unsigned* cnt,
-                       double* part, int* abort_flag, hipStream_t s) {
-  if (nwg <= 0) return MO_OK;
-  MO_CHECK(block_threads >= 64 && block_threads <= 256 && block_threads % 64 == 0, MO_ERR_ARG,
-           "block_threads must be a multiple of 64 in [64, 256] (got %d)", block_threads);
+int lm_rot_chip_launch(const RotPairDesc* pairs_dev, const RotChunk* chunks_dev, int nchunks, const RotChipArrays& a,
+                       const LMOptionsDev& opt, LMResultDev* results_dev, int threads, size_t lds_bytes, bool coop,
+                       unsigned long long* slots, int* abort_flag, hipStream_t s) {
+  if (nchunks <= 0) return MO_OK;
+  MO_HIP(hipFuncSetAttribute(chip_kernel(threads), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
   int dev = 0, khz = 0;
   MO_HIP(hipGetDevice(&dev));
   MO_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
   long long limit = (long long)std::max(khz, 1) * 1000LL * 20;   // a 20 s bound on any one wait
   if (const char* w = getenv("MO_LM_TEAM_WAIT_US")) limit = atoll(w) * (long long)std::max(khz, 1) / 1000LL;
-  RotArrays a = arrays;
+  RotChipArrays arr = a;
   LMOptionsDev o = opt;
-  LMResultDev* r = results_dev;
-  long long tv = total_vertices, th = total_half_edges;
-  void* args[] = {(void*)&pairs_dev, (void*)&plist, (void*)&wg_dev, (void*)&a, (void*)&o, (void*)&r, (void*)&tv,
-                  (void*)&th, (void*)&cnt, (void*)&part, (void*)&abort_flag, (void*)&limit};
+  void* args[] = {(void*)&pairs_dev, (void*)&chunks_dev, (void*)&arr,        (void*)&o,
+                  (void*)&results_dev, (void*)&slots,    (void*)&abort_flag, (void*)&limit};
+  if (!coop) {
+    MO_HIP(hipLaunchKernel(chip_kernel(threads), dim3(nchunks), dim3(threads), args, lds_bytes, s));
+    return MO_OK;
+  }
   // MO_LM_COOP_REFUSE=1 treats the launch as refused without trying it (the
   // fallback path's test hook; the runtime refuses cooperative grids while
   // another process holds the GPU)
   if (const char* f = getenv("MO_LM_COOP_REFUSE"))
     if (f[0] == '1') return kCoopRefused;
-  if (hipLaunchCooperativeKernel((const void*)k_lm_rot_team, dim3(nwg), dim3(block_threads), args, 0, s) !=
+  if (hipLaunchCooperativeKernel(chip_kernel(threads), dim3(nchunks), dim3(threads), args, (unsigned)lds_bytes, s) !=
       hipSuccess) {
     (void)hipGetLastError();   // the runtime refused the cooperative grid: nothing was launched
     return kCoopRefused;

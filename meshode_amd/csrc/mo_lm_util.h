@@ -291,6 +291,96 @@ struct CoherentTeam {
   }
 };
 
+// TagTeam: CoherentTeam's contract with one round trip fewer per exchange.
+// There a member stores its partials, waits for them, bumps the arrival
+// counter, polls it and then loads the partials; here every 64-bit word of
+// a member's slot carries the exchange's sequence number beside 32 bits of
+// data, so the members poll the c slots themselves: a slot whose words all
+// show the sequence number is complete.  Each wave waits for its own
+// published stores (s_waitcnt vmcnt(0)) before the workgroup barrier that
+// precedes the slot's stores, so published data is visible to whoever sees
+// the slot.  Two slot buffers alternate; a member can only overwrite a
+// buffer after every other member has posted the exchange in between, which
+// it does after it has read this one.  Wave 0 polls and combines, the others
+// get the totals through LDS: all threads of a workgroup hold the same bits
+// also when a wait ran out, so they leave the solver's loops together.
+constexpr int kTagWords = 16;                                     // words of a slot: 8 doubles in halves
+constexpr int kTagRed = 2 * (8 * kMaxWaves + 8);                  // doubles of a workgroup's reduction buffer
+constexpr int kTagSlotWords = 2 * kMaxTeam * kTagWords;           // 64-bit words of a team's slots (zeroed)
+
+struct TagTeam {
+  int r, c;
+  unsigned long long* slots;   // [2][kMaxTeam][kTagWords], zero before the launch
+  int* abort_flag;
+  long long limit;
+  double* red;                 // LDS, kTagRed doubles
+  unsigned seq;
+  int sel;
+  __device__ bool leader() const { return r == 0; }
+  __device__ void barrier() {
+    double z[1] = {0.0};
+    reduce<1, 0>(z);
+  }
+  template <int K, int M>
+  __device__ void reduce(double (&v)[K + M]) {
+    constexpr int kV = K + M;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    double* buf = red + sel * (8 * kMaxWaves + 8);
+    sel ^= 1;
+    for (int k = 0; k < K; ++k) v[k] = wave_sum_f64(v[k]);
+    for (int k = K; k < kV; ++k) v[k] = wave_max_f64(v[k]);
+    if (lane == 0)
+      for (int k = 0; k < kV; ++k) buf[k * kMaxWaves + w] = v[k];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (c > 1) ++seq;
+    if (c == 1 || w == 0) {
+      for (int k = 0; k < K; ++k) v[k] = readlane_f64(row_sum_f64(lane < nw ? buf[k * kMaxWaves + lane] : 0.0), 0);
+      for (int k = K; k < kV; ++k)
+        v[k] = readlane_f64(row_max_f64(lane < nw ? buf[k * kMaxWaves + lane] : -INFINITY), 0);
+    }
+    if (c == 1) return;
+    if (w == 0) {
+      unsigned long long* base = slots + (size_t)(seq & 1u) * (kMaxTeam * kTagWords);
+      unsigned half = 0;
+      for (int k = 0; k < kV; ++k) {
+        const unsigned long long b = __builtin_bit_cast(unsigned long long, v[k]);
+        if (lane == 2 * k) half = (unsigned)b;
+        if (lane == 2 * k + 1) half = (unsigned)(b >> 32);
+      }
+      if (lane < 2 * kV)
+        __hip_atomic_store(base + (size_t)r * kTagWords + lane, ((unsigned long long)seq << 32) | half,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      // lane q polls member q (c <= kMaxTeam = 64)
+      const unsigned long long* mine = base + (size_t)(lane < c ? lane : 0) * kTagWords;
+      unsigned long long word[2 * kV];
+      const long long t0 = wall_clock64();
+      while (true) {
+        bool ok = true;
+        const int aborted = __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (int k = 0; k < 2 * kV; ++k)
+          word[k] = __hip_atomic_load(const_cast<unsigned long long*>(mine) + k, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+        for (int k = 0; k < 2 * kV; ++k) ok = ok && (unsigned)(word[k] >> 32) == seq;
+        if (__all(ok) || aborted) break;
+        if (wall_clock64() - t0 > limit) {
+          __hip_atomic_store(abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          break;
+        }
+      }
+      for (int k = 0; k < kV; ++k) {
+        const double x = __builtin_bit_cast(
+            double, (word[2 * k] & 0xFFFFFFFFull) | (word[2 * k + 1] << 32));
+        v[k] = k < K ? wave_sum_f64(lane < c ? x : 0.0) : wave_max_f64(lane < c ? x : -INFINITY);
+      }
+      if (lane == 0)
+        for (int k = 0; k < kV; ++k) buf[8 * kMaxWaves + k] = v[k];
+    }
+    __syncthreads();
+    for (int k = 0; k < kV; ++k) v[k] = buf[8 * kMaxWaves + k];
+  }
+};
+
 // Candidate evaluation of one trust-region step.
 struct LMCandidate {
   double model_change;   // model_cost_change = -(J delta).(f + J delta / 2)

@@ -1,0 +1,68 @@
+"""The on-chip DeformWithRot solver (k_lm_rot_chip) at the edges of its
+chunks: one vertex below, at and above a 256-vertex chunk, a last chunk that
+is short, a last chunk of one vertex, merged parallel half-edges beyond an
+entry's multiplicity, vertices in no face, and a hub whose adjacency does not
+fit the LDS (which takes the one-workgroup kernel).  The bar is the one of
+the other DeformWithRot tests: the final energy, evaluated by the oracle's
+cost at the GPU's result, within 1e-3 of the oracle's exact-step solve."""
+import numpy as np
+import pytest
+import torch
+
+from meshode_amd import deform, pyDeform, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _fan(n):
+    """A hub joined to a rim of n vertices."""
+    a = 2 * np.pi * np.arange(n) / n
+    V = np.concatenate([[[0.0, 0.0, 0.3]], np.stack([np.cos(a), np.sin(a), 0 * a], 1)])
+    k = np.arange(n)
+    return V, np.stack([0 * k, 1 + k, 1 + (k + 1) % n], 1).astype(np.int32)
+
+
+def _case(name):
+    if name.startswith("boxes"):
+        sV, sF, tV, tF = synth.box_union_pair(3, n_boxes=3, n_verts=int(name[5:]) // 2 * 2)
+        if int(name[5:]) % 2:        # a vertex in no face
+            sV = np.concatenate([sV, sV.mean(0, keepdims=True)])
+        return sV, sF, tV, tF
+    _, _, tV, tF = synth.displaced_sphere_pair(5, src_level=1, tgt_level=2)
+    if name == "repeated":           # 70 copies of every half-edge: two entries per neighbour
+        sV, sF = synth.icosphere(1)
+        return sV * 0.9, np.tile(sF, (70, 1)), tV, tF
+    sV, sF = _fan(int(name[3:]))
+    return sV, sF, tV, tF
+
+
+@pytest.mark.parametrize("name,workgroups", [("boxes254", 1), ("boxes256", 1), ("boxes257", 2), ("boxes512", 2),
+                                             ("boxes600", 3), ("repeated", 1), ("fan300", 2)])
+def test_chip_energy_parity(gpu, oracle, name, workgroups):
+    print(f"[rot chip] {name}", flush=True)
+    sV, sF, tV, tF = _case(name)
+    pid = deform.template_f64(tV, tF, 16)
+    _, scale, trans = pyDeform.TemplateInfo(pid)
+    grid = pyDeform.TemplateGrid(pid)[0].cpu().numpy().reshape(-1)
+    sn = (sV - trans) / scale
+    V = torch.from_numpy(sn).to(gpu).contiguous()
+    st, W = deform.deform_rot(pid, V, sF, 1.0)
+    assert st["workgroups"] == workgroups
+    _, _, so = oracle.lm_rot_solve(grid, 16, sn, sF, 1.0)
+    eg = oracle.lm_rot_cost(grid, 16, V.cpu().numpy(), W.cpu().numpy(), sn, sF, 1.0)[0]
+    print(f"[rot chip]   gpu {eg:.6e} oracle {so['final_cost']:.6e} ({st['iterations']}/{so['iterations']} it)",
+          flush=True)
+    assert st["initial_cost"] == pytest.approx(so["initial_cost"], rel=1e-4)
+    assert abs(eg - so["final_cost"]) <= 1e-3 * so["final_cost"]
+
+
+def test_hub_beyond_lds(gpu):
+    """A hub of 6000 neighbours does not fit a chunk's LDS: one workgroup."""
+    print("[rot chip] fan6000", flush=True)
+    sV, sF, tV, tF = _case("fan6000")
+    pid = deform.template_f64(tV, tF, 16)
+    _, scale, trans = pyDeform.TemplateInfo(pid)
+    V = torch.from_numpy((sV - trans) / scale).to(gpu).contiguous()
+    opt = deform.default_options(max_num_iterations=2, pcg_max_iterations=20)
+    st, _ = deform.deform_rot(pid, V, sF, 1.0, options=opt)
+    assert st["workgroups"] == 1 and st["final_cost"] <= st["initial_cost"]
