@@ -502,7 +502,7 @@ int mo_ode_rk4_backward(const float* y0, int64_t n, const float* params, const f
                         const float* zsave, const float* gy1, float* gy0, float* gparams, void* work,
                         int64_t work_bytes, void* stream);
 
-/* ---- config-3 velocity field: one RK4 step on FP32 MFMA -------------------
+/* ---- config-3 velocity field: one RK4 step on MFMA ------------------------
  * The field v(y) = MLP(y - 0.5), 3 -> 256 -> 256 -> 256 -> 3 with softplus
  * (torch's threshold 20), the widened ODEFunc of neuralode_fast.py:7-33,
  * and the 3/8-rule step of odeint(method="rk4") (neuralode_fast.py:55-60):
@@ -511,12 +511,32 @@ int mo_ode_rk4_backward(const float* y0, int64_t n, const float* params, const f
  * mo_flow256_pack: the module's tensors (W0 [256,3], b0 [256], W1 [256,256],
  * b1, W2 [256,256], b2, W3 [3,256], b3 [3]; FP32 device, row-major) into
  * `packed` (mo_flow256_packed_floats() floats, device, 16-byte aligned).
- * mo_flow256_step: y0, y1 [n,3] FP32 device (distinct buffers). */
+ * mo_flow256_step: y0, y1 [n,3] FP32 device (distinct buffers); the
+ * 256 x 256 products on bf16 MFMA with every FP32 number split exactly into
+ * three bf16, at the accuracy of FP32 products (a non-finite activation
+ * gives NaN). */
 int64_t mo_flow256_packed_floats(void);
 int mo_flow256_pack(const float* W0, const float* b0, const float* W1, const float* b1, const float* W2,
                     const float* b2, const float* W3, const float* b3, float* packed, void* stream);
 int mo_flow256_step(const float* y0, int64_t n, const float* packed, float h, float* y1, void* stream);
-/* The adjoint of a step (the reference differentiates odeint by autograd).
+/* The adjoint of an integration (the reference differentiates odeint by
+ * autograd).  Forward: mo_flow256_step_stages is mo_flow256_step that also
+ * writes the stage inputs Zs [4][n][3] (or null).  Backward, per step, last
+ * first: mo_flow256_adjoint_step takes the step's Zs and gy1 = dL/dy1 to
+ * gy0 = dL/dy0 and adds the step's part of the parameter gradients to the
+ * partial sums in `work` (mo_flow256_adjoint_work_floats(n) floats, device,
+ * 16-byte aligned; `first` nonzero starts them).  mo_flow256_adjoint_grads
+ * writes the gradients (laid out as mo_flow256_pack's tensors; workgroup
+ * partials added in a fixed order in FP64).  gy0 and gy1 are distinct;
+ * n <= 2^25. */
+int mo_flow256_step_stages(const float* y0, int64_t n, const float* packed, float h, float* y1, float* Zs,
+                           void* stream);
+int64_t mo_flow256_adjoint_work_floats(int64_t n);
+int mo_flow256_adjoint_step(int64_t n, const float* packed, float h, const float* Zs, const float* gy1, float* gy0,
+                            float* work, int32_t first, void* stream);
+int mo_flow256_adjoint_grads(int64_t n, const float* work, float* W0, float* b0, float* W1, float* b1, float* W2,
+                             float* b2, float* W3, float* b3, void* stream);
+/* The adjoint of one step on FP32 MFMA, with its intermediates handed out.
  * mo_flow256_step_save: mo_flow256_step that also writes the stage inputs
  * x = z - 0.5 to Xs [4][n][3] and the activations H1, H2, H3 to
  * Hs [3][4][n][256] (layer, stage, point).  mo_flow256_step_backward: from

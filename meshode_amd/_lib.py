@@ -30,7 +30,8 @@ SYMBOLS = [
     "mo_ode_rk4_workspace_bytes", "mo_ode_rk4_forward", "mo_ode_rk4_backward",
     "mo_flow256_packed_floats", "mo_flow256_pack", "mo_flow256_step", "mo_flow256_step_save",
     "mo_flow256_step_backward", "mo_flow256_small_grad_floats", "mo_flow256_small_grads",
-    "mo_flow256_dw_work_floats", "mo_flow256_dw_grads",
+    "mo_flow256_dw_work_floats", "mo_flow256_dw_grads", "mo_flow256_step_stages", "mo_flow256_adjoint_work_floats",
+    "mo_flow256_adjoint_step", "mo_flow256_adjoint_grads",
     "mo_deform_batch_noalloc_max_bytes", "mo_deform_batch_noalloc", "mo_template_rebuild_f64",
     "mo_last_grid_stats", "mo_rigid_deform_batch_graph", "mo_batch_graph_launch", "mo_batch_graph_destroy",
     "mo_rigid_deform_batch_async", "mo_batch_wait",
@@ -157,6 +158,10 @@ _SIGS = {
     "mo_flow256_small_grad_floats": (_i64, []),
     "mo_flow256_small_grads": (C.c_int, [_i64, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "mo_flow256_dw_work_floats": (_i64, []),
+    "mo_flow256_step_stages": (C.c_int, [_vp, _i64, _vp, C.c_float, _vp, _vp, _vp]),
+    "mo_flow256_adjoint_work_floats": (_i64, [_i64]),
+    "mo_flow256_adjoint_step": (C.c_int, [_i64, _vp, C.c_float, _vp, _vp, _vp, _vp, C.c_int32, _vp]),
+    "mo_flow256_adjoint_grads": (C.c_int, [_i64] + [_vp] * 10),
     "mo_flow256_dw_grads": (C.c_int, [_i64, _vp, _vp, _vp, _vp, _vp]),
     "mo_ode_rk4_forward": (C.c_int, [_vp, _i64, _vp, _vp, C.c_float, C.c_float, _vp, _vp, _vp]),
     "mo_ode_rk4_backward": (C.c_int, [_vp, _i64, _vp, _vp, C.c_float, C.c_float, _vp, _vp, _vp, _vp, _vp, _i64,

@@ -1,4 +1,7 @@
-// One RK4 step of the config-3 velocity field on FP32 MFMA: the MLP
+// One RK4 step of the config-3 velocity field on FP32 MFMA, with its
+// activations handed to the caller, and its backward from them (the plain
+// step and the adjoint the Python layer runs are in mo_flow256_split.hip):
+// the MLP
 // 3 -> 256 -> 256 -> 256 -> 3 with softplus, v(y) = MLP(y - 0.5)
 // (meshode_amd/neuralode.py's VelocityMLP; the reference's ODEFunc layout,
 // neuralode_fast.py:7-33, widened as the config-3 workload specifies), and
@@ -23,6 +26,7 @@
 #include <algorithm>
 
 #include "mo_common.h"
+#include "mo_flow256.h"
 
 #define MO_EXPORT extern "C" __attribute__((visibility("default")))
 
@@ -31,23 +35,9 @@ namespace {
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-constexpr int kH = 256;
 constexpr int kPts = 64;
 constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
-// packed parameter layout (floats)
-constexpr int kPW0 = 0;                 // W0 [256][4] (k = 3 padded with 0)
-constexpr int kPB0 = kPW0 + kH * 4;     // b0 [256]
-constexpr int kPW1 = kPB0 + kH;         // W1 fragments [8 col blocks][32 groups][64 lanes][4]
-constexpr int kPB1 = kPW1 + kH * kH;
-constexpr int kPW2 = kPB1 + kH;
-constexpr int kPB2 = kPW2 + kH * kH;
-constexpr int kPW3 = kPB2 + kH;         // W3 [3][256]
-constexpr int kPB3 = kPW3 + 3 * kH;     // b3 [3] (+1 pad)
-constexpr int kPW1T = kPB3 + 4;         // W1^T fragments (backward: dH1 = dA2 W1)
-constexpr int kPW2T = kPW1T + kH * kH;  // W2^T fragments (backward: dH2 = dA3 W2)
-constexpr int kPacked = kPW2T + kH * kH;
-
 // Activation tile: [128 unit pairs][64 points][2], the point index XOR-ed
 // with the unit pair (mod 32) so that the epilogue's writes (32 units, 2
 // point rows per wave) spread over the banks; a 32-point block stays a
@@ -92,6 +82,19 @@ __global__ void k_flow256_pack(const float* __restrict__ W0, const float* __rest
     P[kPW2 + e] = W2[row * kH + col];
     P[kPW1T + e] = W1[col * kH + row];
     P[kPW2T + e] = W2[col * kH + row];
+    // split planes: element e of a fragment plane
+    const int j8 = e & 7, ls = (e >> 3) & 63, ks = (e >> 9) & 15, rb = e >> 13;
+    const int sr = 32 * rb + (ls & 31), sk = 16 * ks + 8 * (ls >> 5) + j8;
+    const float v[4] = {W1[sr * kH + sk], W2[sr * kH + sk], W1[sk * kH + sr], W2[sk * kH + sr]};
+    for (int m = 0; m < 4; ++m) {
+      unsigned short* S = reinterpret_cast<unsigned short*>(P + kPSplit + m * kSplitLayer);
+      float x = v[m];
+      for (int pl = 0; pl < 3; ++pl) {
+        const __bf16 h = (__bf16)x;
+        S[pl * kH * kH + e] = __builtin_bit_cast(unsigned short, h);
+        x -= (float)h;
+      }
+    }
   }
   if (e < 3 * kH) P[kPW3 + e] = W3[e];
   if (e < 4) P[kPB3 + e] = e < 3 ? b3[e] : 0.f;
@@ -210,11 +213,10 @@ __device__ __forceinline__ void store_tile(const float* __restrict__ T, float* _
 
 // Workgroup b of G takes points [n b / G, n (b + 1) / G) in chunks of 64
 // (G = one per CU: the shares differ by at most one point, and a chunk of
-// at most 32 points skips the second 32-point MFMA block).  With kSave the
-// stage inputs x = z - 0.5 go to Xs [4][n][3] and the activations H1, H2, H3
+// at most 32 points skips the second 32-point MFMA block).  The stage
+// inputs x = z - 0.5 go to Xs [4][n][3] and the activations H1, H2, H3
 // to Hs [3][4][n][256] (layer, stage, point) for the backward.
-template <bool kSave>
-__global__ __launch_bounds__(kThreads) void k_flow256_step(const float* __restrict__ y0, int n,
+__global__ __launch_bounds__(kThreads) void k_flow256_step_save(const float* __restrict__ y0, int n,
                                                            const float* __restrict__ P, float h,
                                                            float* __restrict__ y1, float* __restrict__ Hs,
                                                            float* __restrict__ Xs) {
@@ -244,7 +246,7 @@ __global__ __launch_bounds__(kThreads) void k_flow256_step(const float* __restri
                     : s == 1 ? y + h * K[0][tid][c] / 3.0f
                     : s == 2 ? y + h * (K[1][tid][c] - K[0][tid][c] / 3.0f)
                              : y + h * (K[0][tid][c] - K[1][tid][c] + K[2][tid][c]);
-          if (kSave && tid < nvalid) Xs[((size_t)s * n + base + tid) * 3 + c] = Z[tid][c] - 0.5f;
+          if (tid < nvalid) Xs[((size_t)s * n + base + tid) * 3 + c] = Z[tid][c] - 0.5f;
         }
       }
       __syncthreads();
@@ -259,18 +261,18 @@ __global__ __launch_bounds__(kThreads) void k_flow256_step(const float* __restri
       }
       __syncthreads();
       {
-        float* d1 = kSave ? Hs + (0 * 4 + s) * plane + (size_t)base * kH : nullptr;
-        if (nvalid > 32) hidden_layer<true, kSave>(P + kPW1, P + kPB1, TA, TB, w, l, d1, nvalid);
-        else hidden_layer<false, kSave>(P + kPW1, P + kPB1, TA, TB, w, l, d1, nvalid);
+        float* d1 = Hs + (0 * 4 + s) * plane + (size_t)base * kH;
+        if (nvalid > 32) hidden_layer<true, true>(P + kPW1, P + kPB1, TA, TB, w, l, d1, nvalid);
+        else hidden_layer<false, true>(P + kPW1, P + kPB1, TA, TB, w, l, d1, nvalid);
       }
       __syncthreads();
       {
-        float* d2 = kSave ? Hs + (1 * 4 + s) * plane + (size_t)base * kH : nullptr;
-        if (nvalid > 32) hidden_layer<true, kSave>(P + kPW2, P + kPB2, TB, TA, w, l, d2, nvalid);
-        else hidden_layer<false, kSave>(P + kPW2, P + kPB2, TB, TA, w, l, d2, nvalid);
+        float* d2 = Hs + (1 * 4 + s) * plane + (size_t)base * kH;
+        if (nvalid > 32) hidden_layer<true, true>(P + kPW2, P + kPB2, TB, TA, w, l, d2, nvalid);
+        else hidden_layer<false, true>(P + kPW2, P + kPB2, TB, TA, w, l, d2, nvalid);
       }
       __syncthreads();
-      if (kSave) store_tile(TA, Hs + (2 * 4 + s) * plane + (size_t)base * kH, nvalid);
+      store_tile(TA, Hs + (2 * 4 + s) * plane + (size_t)base * kH, nvalid);
       // layer 3 (VALU): wave w sums units [32 w, 32 w + 32) for point l
       {
         float o0 = 0.f, o1 = 0.f, o2 = 0.f;
@@ -425,7 +427,6 @@ __global__ __launch_bounds__(kThreads) void k_flow256_step_bwd(int n, const floa
 // workgroup b sums rows [R b / G, R (b + 1) / G) for unit u (coalesced rows
 // of dA1, dA2, dA3, H3) and writes the workgroup's partial row;
 // k_flow256_rows_reduce adds the rows in a fixed order (FP64).
-constexpr int kSmallGrad = 3 * kH + 3 * kH + 3 * kH + 3;   // 2307
 __global__ __launch_bounds__(kH) void k_flow256_grad_small(int rows, const float* __restrict__ dA1,
                                                            const float* __restrict__ dA2,
                                                            const float* __restrict__ dA3,
@@ -571,6 +572,11 @@ int cu_count() {
 }
 
 }  // namespace
+
+void flow256_rows_reduce(const float* partial, int nblocks, int len, int ny, float* out, hipStream_t s) {
+  hipLaunchKernelGGL(k_flow256_rows_reduce, dim3((len + 63) / 64, ny), dim3(512), 0, s, partial, nblocks, len, out);
+}
+
 }  // namespace mo
 
 using namespace mo;
@@ -586,17 +592,6 @@ MO_EXPORT int mo_flow256_pack(const float* W0, const float* b0, const float* W1,
   return MO_OK;
 }
 
-MO_EXPORT int mo_flow256_step(const float* y0, int64_t n, const float* packed, float h, float* y1, void* stream) {
-  MO_CHECK(packed && n >= 0 && n <= (1LL << 30) && (n == 0 || (y0 && y1)), MO_ERR_ARG,
-           "mo_flow256_step: bad arguments");
-  if (n == 0) return MO_OK;
-  const int grid = (int)std::min<int64_t>((n + kPts - 1) / kPts, cu_count());
-  hipLaunchKernelGGL(k_flow256_step<false>, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, y0, (int)n, packed, h,
-                     y1, nullptr, nullptr);
-  MO_HIP(hipGetLastError());
-  return MO_OK;
-}
-
 MO_EXPORT int mo_flow256_step_save(const float* y0, int64_t n, const float* packed, float h, float* y1, float* Hs,
                                    float* Xs, void* stream) {
   MO_CHECK(packed && n >= 0 && n <= (1LL << 30) / 12 && (n == 0 || (y0 && y1 && Hs && Xs)), MO_ERR_ARG,
@@ -604,7 +599,7 @@ MO_EXPORT int mo_flow256_step_save(const float* y0, int64_t n, const float* pack
   MO_CHECK(((uintptr_t)Hs & 15) == 0, MO_ERR_ARG, "mo_flow256_step_save: Hs not 16-byte aligned");
   if (n == 0) return MO_OK;
   const int grid = (int)std::min<int64_t>((n + kPts - 1) / kPts, cu_count());
-  hipLaunchKernelGGL(k_flow256_step<true>, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, y0, (int)n, packed, h,
+  hipLaunchKernelGGL(k_flow256_step_save, dim3(grid), dim3(kThreads), 0, (hipStream_t)stream, y0, (int)n, packed, h,
                      y1, Hs, Xs);
   MO_HIP(hipGetLastError());
   return MO_OK;
@@ -637,8 +632,7 @@ MO_EXPORT int mo_flow256_small_grads(int64_t n, const float* dAs, const float* H
   const int nb = 256;
   hipLaunchKernelGGL(k_flow256_grad_small, dim3(nb), dim3(kH), 0, s, rows, dAs, dAs + plane4, dAs + 2 * plane4,
                      Hs + 2 * plane4, Xs, Gs, work);
-  hipLaunchKernelGGL(k_flow256_rows_reduce, dim3((kSmallGrad + 63) / 64, 1), dim3(512), 0, s, work, nb, kSmallGrad,
-                     out);
+  flow256_rows_reduce(work, nb, kSmallGrad, 1, out, s);
   MO_HIP(hipGetLastError());
   return MO_OK;
 }
@@ -658,7 +652,7 @@ MO_EXPORT int mo_flow256_dw_grads(int64_t n, const float* dAs, const float* Hs, 
   const int G = cu_count();
   hipLaunchKernelGGL(k_flow256_dw, dim3(G, 2), dim3(kThreads), 0, s, (int)(4 * n), dAs + plane4, Hs,
                      dAs + 2 * plane4, Hs + plane4, work);
-  hipLaunchKernelGGL(k_flow256_rows_reduce, dim3(kH * kH / 64, 2), dim3(512), 0, s, work, G, kH * kH, out);
+  flow256_rows_reduce(work, G, kH * kH, 2, out, s);
   MO_HIP(hipGetLastError());
   return MO_OK;
 }

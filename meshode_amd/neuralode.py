@@ -90,14 +90,16 @@ def flow256_pack(func):
     return out
 
 
-def flow256_step(packed, y, h):
-    """One fused RK4 step (FP32, GPU) of the packed 256-wide field."""
+def flow256_step(packed, y, h, stages=None):
+    """One fused RK4 step (FP32, GPU) of the packed 256-wide field; stages:
+    a [4, n, 3] tensor that receives the stage inputs."""
     import ctypes as C
     from . import _lib
     y = y.contiguous()
     y1 = torch.empty_like(y)
-    _lib.call("mo_flow256_step", C.c_void_p(y.data_ptr()), y.shape[0], C.c_void_p(packed.data_ptr()), float(h),
-              C.c_void_p(y1.data_ptr()), pyDeform._stream())
+    _lib.call("mo_flow256_step_stages", C.c_void_p(y.data_ptr()), y.shape[0], C.c_void_p(packed.data_ptr()), float(h),
+              C.c_void_p(y1.data_ptr()), C.c_void_p(stages.data_ptr() if stages is not None else 0),
+              pyDeform._stream())
     return y1
 
 
@@ -108,66 +110,51 @@ class RK4Adjoint(Function):
     @staticmethod
     def forward(ctx, y0, steps, func, *params):
         h = 1.0 / steps
-        ys = [y0.detach()]
+        y = y0.detach()
         with torch.no_grad():
-            y = y0.detach()
             packed = flow256_pack(func) if _fused_field(func, y) else None
-            for _ in range(steps):
-                y = flow256_step(packed, y, h) if packed is not None else rk4_step(func, y, h)
-                ys.append(y)
+            if packed is not None:
+                # the fused adjoint starts from the stage inputs: 48 B a point and step
+                keep = any(ctx.needs_input_grad)
+                saved = [torch.empty((steps, 4) + tuple(y.shape), dtype=torch.float32, device=y.device)] if keep else []
+                for k in range(steps):
+                    y = flow256_step(packed, y, h, saved[0][k] if keep else None)
+            else:
+                saved = [y]
+                for _ in range(steps):
+                    y = rk4_step(func, y, h)
+                    saved.append(y)
+                saved.pop()
         ctx.func, ctx.steps, ctx.h, ctx.packed = func, steps, h, packed
-        ctx.save_for_backward(*ys[:-1])
+        ctx.save_for_backward(*saved)
         ctx.n_params = len(params)
         return y
 
     @staticmethod
     def _fused_backward(ctx, gy):
-        """Per step, last first: the fused step again, saving its stage
-        inputs and activations (mo_flow256_step_save), the fused backward
-        through its four stages (mo_flow256_step_backward: dL/dy and the
-        pre-activation gradients), and the parameter gradients as sums over
-        the step's 4 n stage points: a split-K MFMA kernel for W1 and W2
-        (mo_flow256_dw_grads), one reduction kernel for W0, W3 and the
-        biases (mo_flow256_small_grads)."""
+        """Per step, last first, mo_flow256_adjoint_step: back through its
+        four stages from their inputs (dL/dy), with the weight-gradient
+        products over its 4 n stage points added to the integration's partial
+        sums; mo_flow256_adjoint_grads turns those into the gradients."""
         import ctypes as C
         from . import _lib
-        ys = ctx.saved_tensors
-        n, dev, h = ys[0].shape[0], ys[0].device, ctx.h
-        params = list(ctx.func.parameters())
-        gp = [torch.zeros_like(p) for p in params]
-        Hs = torch.empty(3 * 4 * n * 256, dtype=torch.float32, device=dev)
-        dAs = torch.empty_like(Hs)
-        Xs = torch.empty(4 * n * 3, dtype=torch.float32, device=dev)
-        Gs = torch.empty_like(Xs)
-        y1 = torch.empty(n, 3, dtype=torch.float32, device=dev)
-        nsmall = int(_lib.load().mo_flow256_small_grad_floats())
-        small = torch.empty(nsmall, dtype=torch.float32, device=dev)
-        work = torch.empty(256 * nsmall, dtype=torch.float32, device=dev)
-        dw = torch.empty(2, 256, 256, dtype=torch.float32, device=dev)
-        dwork = torch.empty(int(_lib.load().mo_flow256_dw_work_floats()), dtype=torch.float32, device=dev)
-        H, dA = Hs.view(3, 4 * n, 256), dAs.view(3, 4 * n, 256)
-        X, G = Xs.view(4 * n, 3), Gs.view(4 * n, 3)
+        zs = ctx.saved_tensors[0].contiguous()
+        n, dev = zs.shape[2], zs.device
+        gp = [torch.zeros(p.shape, dtype=torch.float32, device=dev) for p in ctx.func.parameters()]
         g = gy.contiguous().to(torch.float32)
+        if n == 0:
+            return (g, None, None, *gp)
+        work = torch.empty(int(_lib.load().mo_flow256_adjoint_work_floats(n)), dtype=torch.float32, device=dev)
         ptr = lambda t: C.c_void_p(t.data_ptr())      # noqa: E731
         for k in reversed(range(ctx.steps)):
-            _lib.call("mo_flow256_step_save", ptr(ys[k].contiguous()), n, ptr(ctx.packed), float(h), ptr(y1),
-                      ptr(Hs), ptr(Xs), pyDeform._stream())
             gnew = torch.empty(n, 3, dtype=torch.float32, device=dev)
-            _lib.call("mo_flow256_step_backward", n, ptr(ctx.packed), float(h), ptr(Hs), ptr(g), ptr(gnew),
-                      ptr(dAs), ptr(Gs), pyDeform._stream())
-            # weights[0..3], biases[0..3]: W0 [256,3], W1, W2 [256,256], W3 [3,256]
-            _lib.call("mo_flow256_dw_grads", n, ptr(dAs), ptr(Hs), ptr(dw), ptr(dwork), pyDeform._stream())
-            gp[1].add_(dw[0])
-            gp[2].add_(dw[1])
-            _lib.call("mo_flow256_small_grads", n, ptr(dAs), ptr(Hs), ptr(Xs), ptr(Gs), ptr(small), ptr(work),
-                      pyDeform._stream())
-            gp[0].add_(small[0:768].view(256, 3))
-            gp[4].add_(small[768:1024])
-            gp[5].add_(small[1024:1280])
-            gp[6].add_(small[1280:1536])
-            gp[3].add_(small[1536:2304].view(3, 256))
-            gp[7].add_(small[2304:2307])
+            _lib.call("mo_flow256_adjoint_step", n, ptr(ctx.packed), float(ctx.h), ptr(zs[k]), ptr(g), ptr(gnew),
+                      ptr(work), int(k == ctx.steps - 1), pyDeform._stream())
             g = gnew
+        if ctx.steps > 0:
+            # weights[0..3], biases[0..3]
+            order = [gp[i] for pair in zip(range(4), range(4, 8)) for i in pair]
+            _lib.call("mo_flow256_adjoint_grads", n, ptr(work), *[ptr(t) for t in order], pyDeform._stream())
         return (g, None, None, *gp)
 
     @staticmethod
