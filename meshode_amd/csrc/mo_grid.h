@@ -5,21 +5,28 @@
 
 namespace mo {
 
-// FP64 face record for the point-triangle distance (240 bytes).
+// FP64 face record for the point-triangle distance (192 bytes).
 struct GFace {
   double ax, ay, az, bx, by, bz, cx, cy, cz;   // positions in face order
   double nx, ny, nz, inv_nn;                   // n = (b-a) x (c-a), 1/(n.n)
   double d00, d01, d11, denom;                 // Gram entries of (b-a, c-a)
   double ll0, ll1, ll2, il0, il1, il2;         // |edge j|^2 and its reciprocal
-  double lox, loy, loz, hix, hiy, hiz;         // face AABB (culling only)
   int flip;                                    // bit j: edge j endpoints swapped (index order)
   int face;                                    // original face index
 };
 
-// Compact culling record of a face (112 bytes): AABB and plane.
+// FP32 culling record of a face (48 bytes): its AABB rounded outward, and its
+// plane as unit normal n, offset c = n . a and an absolute error bound e of
+// n . q - c in FP32 for q in the unit box (all 0 for slivers: no bound).
 struct GCull {
-  double lox, loy, loz, hix, hiy, hiz;
-  double nx, ny, nz, ax, ay, az, inv_nn, pad;
+  float lox, loy, loz, hix, hiy, hiz;
+  float nx, ny, nz, c, e, pad;
+};
+
+// Bricks handed from the grid build to its second kernel.
+struct GridQueue {
+  int count, next;
+  int2 item[1];        // (job, brick) [every brick of the launch]
 };
 
 // One distance grid to build: normalized FP64 target vertices [nv,3] and
@@ -69,9 +76,9 @@ struct GridJob {
   GCull* cull;
   unsigned* bin;
   int* perm;
-  double* tb;
+  float* tb;          // tile AABBs [ntiles][6], rounded outward
   long long nsuper;   // super-tiles: kSuperTiles consecutive tiles each
-  double* sb;         // their AABBs [nsuper][6]
+  float* sb;          // their AABBs [nsuper][6]
   double* dist64;
   float* dist32;
   int* nearest;

@@ -18,9 +18,10 @@
 //   2. k_bin_sort    : one workgroup counting-sorts face indices by bin (LDS
 //                      histogram + scan) so tiles of consecutive faces are
 //                      spatially tight.
-//   3. k_face_prep   : FP64 face record per face, written in sorted order.
-//   4. k_tile_bounds : AABB per tile of kTile (8) sorted faces;
-//      k_super_bounds: AABB per super-tile of kSuperTiles (16) tiles.
+//   3. k_face_prep   : FP64 face record and FP32 culling record per face,
+//                      written in sorted order.
+//   4. k_tile_bounds : AABB per tile of kTile (8) sorted faces and per
+//                      super-tile of kSuperTiles (16) tiles.
 //   5. k_grid_build  : one wavefront per 4x4x8 brick of grid points (two
 //                      points per lane, 4 apart in z).  The
 //                      wave first evaluates the 6 tiles nearest its brick's
@@ -80,17 +81,16 @@ __device__ inline unsigned spread3(unsigned v) {
 
 __device__ inline double dmin(double a, double b) { return b < a ? b : a; }
 __device__ inline double dmax(double a, double b) { return b > a ? b : a; }
-// One-instruction v_max_f64 / v_min_f64 for the culling bounds and the
-// minimum of the three edge distances: the operands are never NaN there, and
-// where two operands are equal (including +0 / -0) either result gives the
-// same squared distance and the same comparisons.
-__device__ inline double vmax(double a, double b) { return __builtin_fmax(a, b); }
+// One-instruction v_min_f64 for the minimum of the three edge distances: the
+// operands are never NaN there, and where two operands are equal (including
+// +0 / -0) either result gives the same comparisons.
 __device__ inline double vmin(double a, double b) { return __builtin_fmin(a, b); }
 
 // Pass 1: validate indices and compute the centroid bin (Morton order of a
 // 16^3 lattice over [0,1]^3, clamped).  blockIdx.y = job.
-__global__ void k_face_bins(const GridJob* __restrict__ jobs, int* __restrict__ err) {
+__global__ void k_face_bins(const GridJob* __restrict__ jobs, int* __restrict__ err, GridQueue* __restrict__ queue) {
   const GridJob J = jobs[blockIdx.y];
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) queue->count = queue->next = 0;
   for (long long f = (long long)blockIdx.x * blockDim.x + threadIdx.x; f < J.nf;
        f += (long long)gridDim.x * blockDim.x) {
     double c[3] = {0.0, 0.0, 0.0};
@@ -156,7 +156,17 @@ __global__ void __launch_bounds__(kSortT) k_bin_sort(const GridJob* __restrict__
   }
 }
 
-// Pass 3: FP64 face record of face perm[pos], written at its sorted position.
+__device__ inline float round_down(double x) {
+  const float f = (float)x;
+  return (double)f > x ? nextafterf(f, -INFINITY) : f;
+}
+__device__ inline float round_up(double x) {
+  const float f = (float)x;
+  return (double)f < x ? nextafterf(f, INFINITY) : f;
+}
+
+// Pass 3: FP64 face record of face perm[pos] and its FP32 culling record,
+// written at its sorted position.
 // At most 64 VGPRs (8 wavefronts per SIMD): the kernel then fits beside a
 // running grid build's wavefronts (85 VGPRs, 5 per SIMD), so a second
 // batch's face preparation is not held back until that build ends.
@@ -204,53 +214,54 @@ __global__ void __launch_bounds__(256, 8) k_face_prep(const GridJob* __restrict_
   }
   g.ll0 = ll[0]; g.ll1 = ll[1]; g.ll2 = ll[2];
   g.il0 = il[0]; g.il1 = il[1]; g.il2 = il[2];
-  g.lox = dmin(g.ax, dmin(g.bx, g.cx)); g.hix = dmax(g.ax, dmax(g.bx, g.cx));
-  g.loy = dmin(g.ay, dmin(g.by, g.cy)); g.hiy = dmax(g.ay, dmax(g.by, g.cy));
-  g.loz = dmin(g.az, dmin(g.bz, g.cz)); g.hiz = dmax(g.az, dmax(g.bz, g.cz));
   g.flip = flip;
   g.face = (int)f;
   J.faces[pos] = g;
-  J.cull[pos] = GCull{g.lox, g.loy, g.loz, g.hix, g.hiy, g.hiz, g.nx, g.ny, g.nz, g.ax, g.ay, g.az, g.inv_nn, 0.0};
+  GCull q;
+  q.lox = round_down(dmin(g.ax, dmin(g.bx, g.cx))); q.hix = round_up(dmax(g.ax, dmax(g.bx, g.cx)));
+  q.loy = round_down(dmin(g.ay, dmin(g.by, g.cy))); q.hiy = round_up(dmax(g.ay, dmax(g.by, g.cy)));
+  q.loz = round_down(dmin(g.az, dmin(g.bz, g.cz))); q.hiz = round_up(dmax(g.az, dmax(g.bz, g.cz)));
+  q.nx = q.ny = q.nz = q.c = q.e = q.pad = 0.f;
+  // FP32 error of n . q - c for |q_i| <= 1: 3 products and sums of terms
+  // below 3 + |c|, their operands rounded to 2^-24: under 1e-6 (1 + |c|).
+  // n itself is good to 1e-10 where the triangle's sine exceeds 1e-6.
+  if (nn > 1e-12 * g.d00 * g.d11) {
+    const double inv = 1.0 / sqrt(nn);
+    const double ux = g.nx * inv, uy = g.ny * inv, uz = g.nz * inv;
+    const double c = ux * g.ax + uy * g.ay + uz * g.az;
+    q.nx = (float)ux; q.ny = (float)uy; q.nz = (float)uz;
+    q.c = (float)c;
+    q.e = (float)(1e-6 * (1.0 + (c < 0.0 ? -c : c)));
+  }
+  J.cull[pos] = q;
   }
 }
 
-// One wavefront per tile: lanes read the face AABBs, wave min/max.
+// One thread per tile: the union of its faces' AABBs; the 16 lanes of a
+// super-tile then combine theirs.  (A wavefront per tile took 1.6 ms for 512
+// targets of 9952 faces.)
 __global__ void __launch_bounds__(256) k_tile_bounds(const GridJob* __restrict__ jobs) {
   const GridJob J = jobs[blockIdx.y];
-  const int lane = threadIdx.x & 63;
-  const long long t = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= J.ntiles) return;
-  const long long f = t * kTile + lane;
-  double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-  if (lane < kTile && f < J.nf) {
-    const GCull* g = J.cull + f;
-    v[0] = g->lox; v[1] = g->loy; v[2] = g->loz; v[3] = g->hix; v[4] = g->hiy; v[5] = g->hiz;
-  }
-  for (int o = 32; o > 0; o >>= 1)
-    for (int a = 0; a < 6; ++a) {
-      double y = __shfl_xor(v[a], o, 64);
-      v[a] = a < 3 ? dmin(v[a], y) : dmax(v[a], y);
-    }
-  if (lane < 6) {
-    double out = v[0];
-    for (int a = 1; a < 6; ++a) out = lane == a ? v[a] : out;
-    J.tb[t * 6 + lane] = out;
-  }
-}
-
-// One thread per super-tile: the union of its tiles' AABBs.
-__global__ void k_super_bounds(const GridJob* __restrict__ jobs) {
-  const GridJob J = jobs[blockIdx.y];
-  const long long s = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= J.nsuper) return;
-  double v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
-  const long long t1 = (s + 1) * kSuperTiles < J.ntiles ? (s + 1) * kSuperTiles : J.ntiles;
-  for (long long t = s * kSuperTiles; t < t1; ++t)
+  const long long t = (long long)blockIdx.x * 256 + threadIdx.x;
+  float v[6] = {INFINITY, INFINITY, INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  const long long f1 = (t + 1) * kTile < J.nf ? (t + 1) * kTile : J.nf;
+  for (long long f = t * kTile; f < f1; ++f) {
+    const float* g = &J.cull[f].lox;
     for (int a = 0; a < 3; ++a) {
-      v[a] = dmin(v[a], J.tb[t * 6 + a]);
-      v[3 + a] = dmax(v[3 + a], J.tb[t * 6 + 3 + a]);
+      v[a] = fminf(v[a], g[a]);
+      v[3 + a] = fmaxf(v[3 + a], g[3 + a]);
     }
-  for (int a = 0; a < 6; ++a) J.sb[s * 6 + a] = v[a];
+  }
+  if (t < J.ntiles)
+    for (int a = 0; a < 6; ++a) J.tb[t * 6 + a] = v[a];
+  for (int o = 1; o < kSuperTiles; o <<= 1)
+    for (int a = 0; a < 3; ++a) {
+      v[a] = fminf(v[a], __shfl_xor(v[a], o, 64));
+      v[3 + a] = fmaxf(v[3 + a], __shfl_xor(v[3 + a], o, 64));
+    }
+  const long long sp = t / kSuperTiles;
+  if (sp < J.nsuper && (t & (kSuperTiles - 1)) == 0)
+    for (int a = 0; a < 6; ++a) J.sb[sp * 6 + a] = v[a];
 }
 
 // Canonical edge squared distance (endpoints ordered by vertex index).
@@ -320,140 +331,173 @@ __device__ inline unsigned dpp_u32(unsigned v) {
   return (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
 }
 template <int CTRL>
-__device__ inline double dpp_f64(double v) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = dpp_u32<CTRL>((unsigned)b), hi = dpp_u32<CTRL>((unsigned)(b >> 32));
-  return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+__device__ inline float dpp_f32(float v) {
+  return __uint_as_float(dpp_u32<CTRL>(__float_as_uint(v)));
 }
-__device__ inline double readlane_f64(double v, int l) {
-  const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)b, l);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b >> 32), l);
-  return __builtin_bit_cast(double, (unsigned long long)lo | ((unsigned long long)hi << 32));
+__device__ inline float readlane_f32(float v, int l) {
+  return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(v), l));
 }
-
-__device__ inline double wave_max(double v) {
-  v = vmax(v, dpp_f64<0xB1>(v));
-  v = vmax(v, dpp_f64<0x4E>(v));
-  v = vmax(v, dpp_f64<0x141>(v));
-  v = vmax(v, dpp_f64<0x140>(v));
-  return vmax(vmax(readlane_f64(v, 0), readlane_f64(v, 16)), vmax(readlane_f64(v, 32), readlane_f64(v, 48)));
+__device__ inline float wave_max(float v) {
+  v = fmaxf(v, dpp_f32<0xB1>(v));
+  v = fmaxf(v, dpp_f32<0x4E>(v));
+  v = fmaxf(v, dpp_f32<0x141>(v));
+  v = fmaxf(v, dpp_f32<0x140>(v));
+  return fmaxf(fmaxf(readlane_f32(v, 0), readlane_f32(v, 16)), fmaxf(readlane_f32(v, 32), readlane_f32(v, 48)));
 }
-
-// (value, index) with the smaller value, ties to the smaller non-negative
-// index (-1: none)
-__device__ inline void argmin_step(double& ol, int& ot, double xl, int xt) {
-  if (xl < ol || (xl == ol && xt >= 0 && (ot < 0 || xt < ot))) { ol = xl; ot = xt; }
+__device__ inline unsigned wave_min_u32(unsigned v) {
+  v = min(v, dpp_u32<0xB1>(v));
+  v = min(v, dpp_u32<0x4E>(v));
+  v = min(v, dpp_u32<0x141>(v));
+  v = min(v, dpp_u32<0x140>(v));
+  const unsigned a = (unsigned)__builtin_amdgcn_readlane((int)v, 0), b = (unsigned)__builtin_amdgcn_readlane((int)v, 16),
+                 c = (unsigned)__builtin_amdgcn_readlane((int)v, 32), d = (unsigned)__builtin_amdgcn_readlane((int)v, 48);
+  return min(min(a, b), min(c, d));
 }
-template <int CTRL>
-__device__ inline void argmin_dpp(double& ol, int& ot) {
-  argmin_step(ol, ot, dpp_f64<CTRL>(ol), (int)dpp_u32<CTRL>((unsigned)ot));
-}
-// the wave's argmin (the same in every lane)
-__device__ inline void wave_argmin(double& ol, int& ot) {
-  argmin_dpp<0xB1>(ol, ot);
-  argmin_dpp<0x4E>(ol, ot);
-  argmin_dpp<0x141>(ol, ot);
-  argmin_dpp<0x140>(ol, ot);
-  double rl = readlane_f64(ol, 0);
-  int rt = __builtin_amdgcn_readlane(ot, 0);
-  for (int r = 16; r < 64; r += 16) argmin_step(rl, rt, readlane_f64(ol, r), __builtin_amdgcn_readlane(ot, r));
-  ol = rl;
-  ot = rt;
+// the lane holding the (nearly) smallest non-negative key, -1 when every
+// lane is out: the low bits of the key give way to the lane number
+__device__ inline int nearest_lane(float key, bool in) {
+  const unsigned k = in ? (__float_as_uint(key) & ~63u) | (threadIdx.x & 63u) : 0xFFFFFFFFu;
+  const unsigned m = wave_min_u32(k);
+  return m == 0xFFFFFFFFu ? -1 : (int)(m & 63u);
 }
 
-__device__ inline double box_gap2(const MO_GLOBAL double* __restrict__ tb, long long t, double lx, double ly, double lz,
-                                  double hx, double hy, double hz) {
-  double tl[3] = {tb[t * 6 + 0], tb[t * 6 + 1], tb[t * 6 + 2]};
-  double th[3] = {tb[t * 6 + 3], tb[t * 6 + 4], tb[t * 6 + 5]};
-  double ql[3] = {lx, ly, lz}, qh[3] = {hx, hy, hz};
-  double s = 0.0;
-  for (int a = 0; a < 3; ++a) {
-    double g = vmax(0.0, vmax(tl[a] - qh[a], ql[a] - th[a]));
-    s += g * g;
-  }
-  return s;
+// Culling in FP32.  A lower bound of a squared distance is formed from
+// outward-rounded AABBs; beside the real gap D it is at most
+// (D + 5.2e-8)^2 (1 + 5e-7): the grid point's coordinates in [0, 1) are
+// rounded by 2^-25 an axis, and the subtractions and fused sums by 2^-24
+// relative.  cut_of(best) is above that for every D <= sqrt(best), so a
+// bound beyond it shows that the face can neither improve nor tie the best.
+// (FP64 bounds, 18 operations without contraction where FP32 needs 11, on
+// records of twice the size: 36.7 ms against 31.2 for 512 box-union grids.)
+__device__ inline float cut_of(double best) {
+  const float r = __builtin_sqrtf((float)best) * 1.000002f + 2e-7f;
+  return r * r * 1.000002f;
+}
+__device__ inline float gap1(float lo, float hi, float a, float b) {   // [lo, hi] against [a, b]
+  return fmaxf(fmaxf(lo - b, a - hi), 0.f);
+}
+__device__ inline float box_gap2(const MO_GLOBAL float* __restrict__ tb, long long t, float lx, float ly, float lz,
+                                 float hx, float hy, float hz) {
+  const MO_GLOBAL float* b = tb + t * 6;
+  const float gx = gap1(b[0], b[3], lx, hx), gy = gap1(b[1], b[4], ly, hy), gz = gap1(b[2], b[5], lz, hz);
+  return __builtin_fmaf(gz, gz, __builtin_fmaf(gy, gy, gx * gx));
 }
 
-// One wavefront (64 lanes) per 4x4x8 brick: lane l holds the two grid
-// points (x, y, z) and (x, y, z + 4) of it.  The two points share the
-// brick's culling, the staged face records, every LDS read of a record and
-// the x / y parts of their bounds.
-constexpr int kZPts = 2;   // points per lane, 4 apart in z
-__global__ void __launch_bounds__(64) k_grid_build(const GridJob* __restrict__ jobs) {
-  // survivors of a tile's brick-level cull: their full records, copied with
-  // coalesced vector loads, then read by the whole wave at one LDS address
-  __shared__ GFace s_face[kTile];
-  __shared__ int s_list[kTile];
-  const GridJob& JJ = jobs[blockIdx.y];
+// LDS of one wavefront: the survivors of a tile's brick-level cull, culling
+// records and full records
+struct WaveTile {
+  GFace face[kTile];
+  float4 cull[3 * kTile];
+  int list[kTile];
+};
+// orders a wavefront's own LDS accesses (the hardware keeps their order)
+__device__ inline void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+constexpr int kZPts = 2;          // points per lane, 4 apart in z
+constexpr int kHeavyWaves = 16;   // wavefronts of a brick in the second kernel
+
+// LDS the wavefronts of one brick share in the second kernel
+struct BrickShare {
+  unsigned cut[kZPts][64];                  // culling thresholds, FP32 bits (non-negative: integer order)
+  double best[kHeavyWaves][kZPts][64];
+  int idx[kHeavyWaves][kZPts][64];
+};
+
+// One 4x4x8 brick: lane l holds the two grid points (x, y, z) and
+// (x, y, z + 4) of it.  The two points share the brick's culling, the staged
+// face records, every LDS read of a record and the x / y parts of their
+// bounds.  With kWaves > 1 the tiles are dealt out to the wavefronts by their
+// number, every wavefront holding all points; they share their culling
+// thresholds through LDS and merge their bests at the end.  With one
+// wavefront, a brick that has walked max_tiles tiles is given up (false).
+template <int kWaves>
+__device__ inline bool grid_brick(const GridJob& JJ, int b, int max_tiles, WaveTile& L, BrickShare* S) {
   const MO_GLOBAL GFace* __restrict__ faces = gptr(JJ.faces);
   const MO_GLOBAL GCull* __restrict__ cull = gptr(JJ.cull);
   const long long nf = JJ.nf;
-  const MO_GLOBAL double* __restrict__ tb = gptr(JJ.tb);
+  const MO_GLOBAL float* __restrict__ tb = gptr(JJ.tb);
   const long long ntiles = JJ.ntiles;
-  const MO_GLOBAL double* __restrict__ sb = gptr(JJ.sb);
+  const MO_GLOBAL float* __restrict__ sb = gptr(JJ.sb);
   const long long nsuper = JJ.nsuper;
   const int N = JJ.N;
-  const int bpa = (N + 3) / 4, bpz = (N + 4 * kZPts - 1) / (4 * kZPts);
+  const int bpa = (N + 3) / 4;
   MO_GLOBAL double* __restrict__ dist64 = gptr(JJ.dist64);
   MO_GLOBAL float* __restrict__ dist32 = gptr(JJ.dist32);
   MO_GLOBAL int* __restrict__ nearest = gptr(JJ.nearest);
-  const int lane = threadIdx.x;
-  long long b = blockIdx.x;
-  if (b >= (long long)bpa * bpa * bpz) return;
-  const int bx = (int)(b % bpa);
-  const int by = (int)((b / bpa) % bpa);
-  const int bz = (int)(b / ((long long)bpa * bpa));
+  const int lane = threadIdx.x & 63, wv = kWaves > 1 ? (int)(threadIdx.x >> 6) : 0;
+  const int bx = b % bpa;
+  const int by = (b / bpa) % bpa;
+  const int bz = b / (bpa * bpa);
   const int k = bx * 4 + (lane & 3), j = by * 4 + ((lane >> 2) & 3);
   int ip[kZPts];
   bool valid[kZPts];
   double qz[kZPts];
   const double qx = (double)k / (double)N, qy = (double)j / (double)N;
+  float fz[kZPts];
+  const float fx = (float)qx, fy = (float)qy;
 #pragma unroll
   for (int s = 0; s < kZPts; ++s) {
     ip[s] = bz * 4 * kZPts + (lane >> 4) + 4 * s;
     valid[s] = (k < N) && (j < N) && (ip[s] < N);
     qz[s] = (double)ip[s] / (double)N;
+    fz[s] = (float)qz[s];
   }
   // brick AABB over valid points
   const int k1 = min(bx * 4 + 3, N - 1), j1 = min(by * 4 + 3, N - 1), i1 = min(bz * 4 * kZPts + 4 * kZPts - 1, N - 1);
-  const double lx = (double)(bx * 4) / N, ly = (double)(by * 4) / N, lz = (double)(bz * 4 * kZPts) / N;
-  const double hx = (double)k1 / N, hy = (double)j1 / N, hz = (double)i1 / N;
+  const float lx = (float)((double)(bx * 4) / N), ly = (float)((double)(by * 4) / N),
+              lz = (float)((double)(bz * 4 * kZPts) / N);
+  const float hx = (float)((double)k1 / N), hy = (float)((double)j1 / N), hz = (float)((double)i1 / N);
 
-  // points farther than the band only need to be shown farther (GridSpec)
-  double best[kZPts], bcut[kZPts];   // bcut: the culling threshold, kept with best
+  // points farther than the band only need to be shown farther (GridSpec);
+  // cut: the FP32 culling threshold kept with best (-1: no point here, below
+  // every bound)
+  double best[kZPts];
+  float cut[kZPts];
   int bidx[kZPts];
 #pragma unroll
   for (int s = 0; s < kZPts; ++s) {
     best[s] = JJ.band2;
-    bcut[s] = best[s] * (1.0 + 1e-9);
+    cut[s] = valid[s] ? cut_of(best[s]) : -1.f;
     bidx[s] = INT_MAX;
   }
-  // the wave's worst best over its valid points
-  auto worst = [&]() {
-    double m = -INFINITY;
+  if (kWaves > 1) {
+    if (wv == 0)
 #pragma unroll
-    for (int s = 0; s < kZPts; ++s) m = valid[s] ? vmax(m, best[s]) : m;
-    return wave_max(m);
+      for (int s = 0; s < kZPts; ++s) S->cut[s][lane] = __float_as_uint(valid[s] ? cut[s] : 0.f);
+    __syncthreads();
+  }
+  // the thresholds the brick's other wavefronts have reached
+  auto refresh = [&]() {
+    if (kWaves > 1)
+#pragma unroll
+      for (int s = 0; s < kZPts; ++s)
+        if (valid[s]) cut[s] = fminf(cut[s], __uint_as_float(*(volatile unsigned*)&S->cut[s][lane]));
   };
+  // the wave's worst threshold over its valid points
+  auto worst = [&]() { return wave_max(fmaxf(cut[0], cut[1])); };
+  static_assert(kZPts == 2, "worst() takes two points");
   // work counters (wave-uniform): exact evaluations (one point per lane),
   // lanes that needed one, face bound checks (per point), staged tiles
   unsigned long long n_exact = 0, n_needed = 0, n_bound = 0, n_tiles = 0;
 
-  // bound: an upper bound of every valid point's best (the wave's worst
-  // best when it was taken; bests only shrink, so an older value stays valid)
-  auto process_tile = [&](int t, double bound) {
+  // bound: an upper bound of every valid point's threshold (the wave's worst
+  // when it was taken; thresholds only shrink, so an older value stays valid)
+  auto process_tile = [&](int t, float bound) {
     const long long f0 = (long long)t * kTile;
     const int cnt = (int)((nf - f0) < kTile ? (nf - f0) : kTile);
     // stage 1, one face per lane: drop faces whose AABB is farther from the
     // brick AABB than the wave's worst best distance
     bool cand = false;
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    f32x4 c0, c1, c2;
     if (lane < cnt) {
-      const MO_GLOBAL GCull* gp = cull + f0 + lane;
-      const double ax = vmax(0.0, vmax(gp->lox - hx, lx - gp->hix));
-      const double ay = vmax(0.0, vmax(gp->loy - hy, ly - gp->hiy));
-      const double az = vmax(0.0, vmax(gp->loz - hz, lz - gp->hiz));
-      cand = !(ax * ax + ay * ay + az * az > bound * (1.0 + 1e-9));
+      const MO_GLOBAL f32x4* gp = reinterpret_cast<const MO_GLOBAL f32x4*>(cull + f0 + lane);
+      c0 = gp[0]; c1 = gp[1]; c2 = gp[2];
+      const float ax = gap1(c0.x, c0.w, lx, hx), ay = gap1(c0.y, c1.x, ly, hy), az = gap1(c0.z, c1.y, lz, hz);
+      cand = !(__builtin_fmaf(az, az, __builtin_fmaf(ay, ay, ax * ax)) > bound);
     }
     const unsigned long long m = __ballot(cand);
     const int ns = __popcll(m);
@@ -462,42 +506,46 @@ __global__ void __launch_bounds__(64) k_grid_build(const GridJob* __restrict__ j
     n_bound += (unsigned long long)ns * kZPts;
     // compact the survivors (in face order) and stage their records in LDS
     const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-    if (cand) s_list[rank] = lane;
-    __syncthreads();
+    wave_sync();   // the last tile's records have been read
+    if (cand) {
+      L.list[rank] = lane;
+      f32x4* d = reinterpret_cast<f32x4*>(L.cull) + 3 * rank;
+      d[0] = c0; d[1] = c1; d[2] = c2;
+    }
+    wave_sync();
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     constexpr int kChunks = (int)(sizeof(GFace) / sizeof(u32x4));
-    static_assert(sizeof(GFace) % sizeof(u32x4) == 0, "face records are copied in 16-byte chunks");
+    static_assert(sizeof(GFace) % sizeof(u32x4) == 0 && sizeof(GCull) == 48, "records are copied in 16-byte chunks");
     const MO_GLOBAL u32x4* __restrict__ src = reinterpret_cast<const MO_GLOBAL u32x4*>(faces + f0);
-    u32x4* dst = reinterpret_cast<u32x4*>(s_face);
+    u32x4* dst = reinterpret_cast<u32x4*>(L.face);
     for (int c = lane; c < ns * kChunks; c += 64) {
       const int r = c / kChunks, w = c - r * kChunks;
-      dst[c] = src[s_list[r] * kChunks + w];
+      dst[c] = src[L.list[r] * kChunks + w];
     }
-    __syncthreads();
+    wave_sync();
+    refresh();
     // stage 2, per surviving face: every point's own AABB bound, then (when
     // it leaves some point) the plane bound, then the exact test when some
-    // lane's point can still improve or tie its best.  The bounds are summed
-    // in the order x, y, z as for a single point.
+    // lane's point can still improve or tie its best
     for (int r = 0; r < ns; ++r) {
-      const GFace& g = s_face[r];
-      const double gx = vmax(0.0, vmax(g.lox - qx, qx - g.hix));
-      const double gy = vmax(0.0, vmax(g.loy - qy, qy - g.hiy));
-      const double gxy = gx * gx + gy * gy;
+      const float4 r0 = L.cull[3 * r], r1 = L.cull[3 * r + 1], r2 = L.cull[3 * r + 2];
+      const float gx = gap1(r0.x, r0.w, fx, fx), gy = gap1(r0.y, r1.x, fy, fy);
+      const float gxy = __builtin_fmaf(gy, gy, gx * gx);
       bool mine[kZPts];
       bool any = false;
 #pragma unroll
       for (int s = 0; s < kZPts; ++s) {
-        const double gz = vmax(0.0, vmax(g.loz - qz[s], qz[s] - g.hiz));
-        mine[s] = valid[s] && !(gxy + gz * gz > bcut[s]);
+        const float gz = gap1(r0.z, r1.y, fz[s], fz[s]);
+        mine[s] = !(__builtin_fmaf(gz, gz, gxy) > cut[s]);
         any = any || mine[s];
       }
       if (!__ballot(any)) continue;
-      // the face plane is a second lower bound (0 for degenerate faces)
-      const double dxy = g.nx * (qx - g.ax) + g.ny * (qy - g.ay);
+      // the face plane is a second lower bound
+      const float dxy = __builtin_fmaf(r1.z, fx, __builtin_fmaf(r1.w, fy, -r2.y));
 #pragma unroll
       for (int s = 0; s < kZPts; ++s) {
-        const double dp = dxy + g.nz * (qz[s] - g.az);
-        mine[s] = mine[s] && !((dp * dp) * g.inv_nn > bcut[s]);
+        const float dp = fmaxf(fabsf(__builtin_fmaf(r2.x, fz[s], dxy)) - r2.z, 0.f);
+        mine[s] = mine[s] && !(dp * dp > cut[s]);
       }
 #pragma unroll
       for (int s = 0; s < kZPts; ++s) {
@@ -509,16 +557,17 @@ __global__ void __launch_bounds__(64) k_grid_build(const GridJob* __restrict__ j
         // its best cannot improve or tie it), so the face-region / edge
         // branches diverge over those lanes alone
         if (mine[s]) {
+          const GFace& g = L.face[r];
           const double d = face_d2(g, qx, qy, qz[s]);
           if (d < best[s] || (d == best[s] && g.face < bidx[s])) {
             best[s] = d;
-            bcut[s] = d * (1.0 + 1e-9);
+            cut[s] = fminf(cut[s], cut_of(d));
             bidx[s] = g.face;
+            if (kWaves > 1) atomicMin(&S->cut[s][lane], __float_as_uint(cut[s]));
           }
         }
       }
     }
-    __syncthreads();  // the next tile overwrites s_face / s_list
   };
 
   // 1. seeds: the kSupPass super-tiles nearest to the brick's centre (one
@@ -526,35 +575,32 @@ __global__ void __launch_bounds__(64) k_grid_build(const GridJob* __restrict__ j
   //    kSeedTiles nearest of their 64 tiles, are evaluated first.  They give
   //    every point a near-exact distance, which makes the culling below
   //    tight (the choice of seeds affects speed only).
-  int seeds[kSeedTiles];
-  int nseed = 0;
+  int seedv = -1, nseed = 0;   // lane r holds the r-th seed
   {
     // ranked by the AABB gap from the brick's centre (a brick inside
     // several AABBs has gap 0 to all of them)
-    const double cx = 0.5 * (lx + hx), cy = 0.5 * (ly + hy), cz = 0.5 * (lz + hz);
-    double slb = INFINITY;
+    const float cx = 0.5f * (lx + hx), cy = 0.5f * (ly + hy), cz = 0.5f * (lz + hz);
+    float slb = INFINITY;
     int ss = -1;
     for (long long c = 0; c < nsuper; c += 64) {
       const long long sidx = c + lane;
       if (sidx >= nsuper) continue;
-      const double lb = box_gap2(sb, sidx, cx, cy, cz, cx, cy, cz);
+      const float lb = box_gap2(sb, sidx, cx, cy, cz, cx, cy, cz);
       if (lb < slb) { slb = lb; ss = (int)sidx; }
     }
     int sp[kSupPass];
     for (int u = 0; u < kSupPass; ++u) sp[u] = -1;
     for (int u = 0; u < kSupPass; ++u) {
-      double ol = slb;
-      int os = ss;
-      wave_argmin(ol, os);
-      if (os < 0) break;
-      if (ss == os) { slb = INFINITY; ss = -1; }
-      sp[u] = os;
+      const int at = nearest_lane(slb, ss >= 0);
+      if (at < 0) break;
+      sp[u] = __builtin_amdgcn_readlane(ss, at);
+      if (lane == at) ss = -1;
     }
     const int q = lane / kSuperTiles;
     int sq = -1;
 #pragma unroll
     for (int u = 0; u < kSupPass; ++u) sq = q == u ? sp[u] : sq;
-    double mlb = INFINITY;
+    float mlb = INFINITY;
     int mt = -1;
     if (sq >= 0) {
       const long long t = (long long)sq * kSuperTiles + (lane & (kSuperTiles - 1));
@@ -564,15 +610,14 @@ __global__ void __launch_bounds__(64) k_grid_build(const GridJob* __restrict__ j
       }
     }
     for (int r = 0; r < kSeedTiles; ++r) {
-      double ol = mlb;
-      int ot = mt;
-      wave_argmin(ol, ot);
-      if (ot < 0) break;
-      if (mt == ot) { mlb = INFINITY; mt = -1; }
-      seeds[nseed++] = ot;
+      const int at = nearest_lane(mlb, mt >= 0);
+      if (at < 0) break;
+      const int st = __builtin_amdgcn_readlane(mt, at);
+      if (lane == r) seedv = st;
+      ++nseed;
+      if (lane == at) mt = -1;
     }
   }
-  for (int r = 0; r < nseed; ++r) process_tile(seeds[r], worst());
 
   // 2. every other tile that can still improve (or tie) some point's best:
   //    super-tiles whose AABB is within the wave's worst best of the brick
@@ -580,48 +625,93 @@ __global__ void __launch_bounds__(64) k_grid_build(const GridJob* __restrict__ j
   //    on tile j of the q-th) their tiles by the same test, and each such
   //    tile is kept only if some point's own point-to-AABB bound reaches its
   //    own best.
-  for (long long c = 0; c < nsuper; c += 64) {
-    const long long sidx = c + lane;
-    const double slb = sidx < nsuper ? box_gap2(sb, sidx, lx, ly, lz, hx, hy, hz) : INFINITY;
-    const double sbound = worst();
-    unsigned long long smask = __ballot(sidx < nsuper && !(slb > sbound * (1.0 + 1e-9)));
-    while (smask) {
-      int sp[kSupPass];
-      for (int u = 0; u < kSupPass; ++u) {
-        sp[u] = smask ? (int)c + __ffsll((long long)smask) - 1 : -1;
-        smask &= smask - 1;
+  //    (One loop for both, so that the face tests are compiled in once.)
+  int walked = 0, seed = 0;
+  long long c = 0, t = -1;
+  unsigned long long smask = 0, tmask = 0;
+  float bound = 0.f;
+  while (true) {
+    int tt;
+    if (seed < nseed) {
+      const int r = seed++;
+      if (kWaves > 1 && r % kWaves != wv) continue;
+      tt = __builtin_amdgcn_readlane(seedv, r);
+      bound = worst();
+    } else {
+      if (seed == nseed) {      // after the seeds
+        ++seed;
+        if (kWaves > 1) __syncthreads();
       }
-      const int q = lane / kSuperTiles;
-      int sq = -1;
+      if (!tmask) {
+        refresh();
+        bound = worst();
+        if (!smask) {
+          if (c >= nsuper) break;
+          const long long sidx = c + lane;
+          const float slb = sidx < nsuper ? box_gap2(sb, sidx, lx, ly, lz, hx, hy, hz) : INFINITY;
+          smask = __ballot(sidx < nsuper && !(slb > bound));
+          c += 64;
+          if (!smask) continue;
+        }
+        const long long first = c - 64;
+        const int q = lane / kSuperTiles;
+        int sq = -1;
 #pragma unroll
-      for (int u = 0; u < kSupPass; ++u) sq = q == u ? sp[u] : sq;
-      const long long t = sq < 0 ? -1 : (long long)sq * kSuperTiles + (lane & (kSuperTiles - 1));
-      const double bound = worst();
-      bool need = false;
-      if (t >= 0 && t < ntiles) {
-        bool taken = false;
-        for (int r = 0; r < nseed; ++r) taken |= (seeds[r] == (int)t);
-        need = !taken && !(box_gap2(tb, t, lx, ly, lz, hx, hy, hz) > bound * (1.0 + 1e-9));
-      }
-      unsigned long long tmask = __ballot(need);
-      while (tmask) {
-        const int l = __ffsll((long long)tmask) - 1;
-        tmask &= tmask - 1;
-        const int tt = __builtin_amdgcn_readlane((int)t, l);
-        bool reach = false;
+        for (int u = 0; u < kSupPass; ++u) {
+          const int sp = smask ? (int)first + __ffsll((long long)smask) - 1 : -1;
+          smask &= smask - 1;
+          sq = q == u ? sp : sq;
+        }
+        t = sq < 0 ? -1 : (long long)sq * kSuperTiles + (lane & (kSuperTiles - 1));
+        bool need = false;
+        if (t >= 0 && t < ntiles && (kWaves == 1 || (lane & (kWaves - 1)) == wv))
+          need = !(box_gap2(tb, t, lx, ly, lz, hx, hy, hz) > bound);
 #pragma unroll
-        for (int s = 0; s < kZPts; ++s)
-          reach = reach || (valid[s] && !(box_gap2(tb, tt, qx, qy, qz[s], qx, qy, qz[s]) > bcut[s]));
-        if (!__ballot(reach)) continue;
-        process_tile(tt, bound);
+        for (int r = 0; r < kSeedTiles; ++r) need = need && __builtin_amdgcn_readlane(seedv, r) != (int)t;
+        tmask = __ballot(need);
+        continue;
       }
+      const int l = __ffsll((long long)tmask) - 1;
+      tmask &= tmask - 1;
+      tt = __builtin_amdgcn_readlane((int)t, l);
+      const MO_GLOBAL float* tbb = tb + (long long)tt * 6;
+      const float gx = gap1(tbb[0], tbb[3], fx, fx), gy = gap1(tbb[1], tbb[4], fy, fy);
+      const float gxy = __builtin_fmaf(gy, gy, gx * gx);
+      bool reach = false;
+#pragma unroll
+      for (int s = 0; s < kZPts; ++s) {
+        const float gz = gap1(tbb[2], tbb[5], fz[s], fz[s]);
+        reach = reach || !(__builtin_fmaf(gz, gz, gxy) > cut[s]);
+      }
+      if (!__ballot(reach)) continue;
+      if (kWaves == 1 && ++walked > max_tiles) return false;
     }
+    process_tile(tt, bound);
   }
+  static_assert(kWaves == 1 || kSuperTiles % kWaves == 0, "tiles are dealt by their number in a super-tile");
   if (JJ.stats && lane == 0) {
     atomicAdd(JJ.stats + kGridStatExact, n_exact * 64ull);
     atomicAdd(JJ.stats + kGridStatExactNeeded, n_needed);
     atomicAdd(JJ.stats + kGridStatBound, n_bound * 64ull);
     atomicAdd(JJ.stats + kGridStatTiles, n_tiles);
+  }
+  if (kWaves > 1) {
+#pragma unroll
+    for (int s = 0; s < kZPts; ++s) {
+      S->best[wv][s][lane] = best[s];
+      S->idx[wv][s][lane] = bidx[s];
+    }
+    __syncthreads();
+    if (wv == 0)
+#pragma unroll
+      for (int s = 0; s < kZPts; ++s)
+        for (int w = 1; w < kWaves; ++w) {
+          const double d = S->best[w][s][lane];
+          const int i = S->idx[w][s][lane];
+          if (d < best[s] || (d == best[s] && i < bidx[s])) { best[s] = d; bidx[s] = i; }
+        }
+    __syncthreads();   // the next brick overwrites the shared arrays
+    if (wv != 0) return true;
   }
 #pragma unroll
   for (int s = 0; s < kZPts; ++s) {
@@ -631,6 +721,45 @@ __global__ void __launch_bounds__(64) k_grid_build(const GridJob* __restrict__ j
     if (dist64) dist64[cell] = sq;
     if (dist32) dist32[cell] = (float)sq;
     if (nearest) nearest[cell] = bidx[s] == INT_MAX ? -1 : bidx[s];
+  }
+  return true;
+}
+
+__device__ inline int brick_count(int N) {
+  const int bpa = (N + 3) / 4, bpz = (N + 4 * kZPts - 1) / (4 * kZPts);
+  return bpa * bpa * bpz;
+}
+
+// One wavefront per brick.  Most bricks walk a few tiles; one near the
+// target's medial surface can walk hundreds (1400 of a 81,920-face sphere at
+// 128^3, 8.4 ms, where the median brick takes 37 us), and a launch of few
+// bricks lasts as long as its worst.  A brick past max_tiles goes to the
+// queue (which holds every brick), and k_grid_heavy starts it again on 16
+// wavefronts.
+__global__ void __launch_bounds__(64, 5) k_grid_build(const GridJob* __restrict__ jobs, GridQueue* __restrict__ queue,
+                                                   int max_tiles) {
+  __shared__ WaveTile L;
+  const GridJob& JJ = jobs[blockIdx.y];
+  const int b = blockIdx.x;
+  if (b >= brick_count(JJ.N)) return;
+  if (grid_brick<1>(JJ, b, max_tiles, L, nullptr)) return;
+  if (threadIdx.x == 0) queue->item[atomicAdd(&queue->count, 1)] = make_int2((int)blockIdx.y, b);
+}
+
+__global__ void __launch_bounds__(64 * kHeavyWaves) k_grid_heavy(const GridJob* __restrict__ jobs,
+                                                                 GridQueue* __restrict__ queue) {
+  __shared__ WaveTile L[kHeavyWaves];
+  __shared__ BrickShare S;
+  __shared__ int s_item;
+  const int n = queue->count;
+  while (true) {
+    if (threadIdx.x == 0) s_item = atomicAdd(&queue->next, 1);
+    __syncthreads();
+    const int q = s_item;
+    if (q >= n) return;
+    const int2 it = queue->item[q];
+    grid_brick<kHeavyWaves>(jobs[it.x], it.y, INT_MAX, L[threadIdx.x >> 6], &S);
+    __syncthreads();
   }
 }
 
@@ -697,9 +826,15 @@ size_t grid_job_workspace_bytes(long long nf) {
   const long long ntiles = (nf + kTile - 1) / kTile;
   const long long nsuper = (ntiles + kSuperTiles - 1) / kSuperTiles;
   return al256((size_t)nf * sizeof(GFace)) + al256((size_t)nf * sizeof(GCull)) + al256((size_t)nf * sizeof(unsigned)) +
-         al256((size_t)nf * sizeof(int)) + al256((size_t)ntiles * 6 * sizeof(double)) +
-         al256((size_t)nsuper * 6 * sizeof(double));
+         al256((size_t)nf * sizeof(int)) + al256((size_t)ntiles * 6 * sizeof(float)) +
+         al256((size_t)nsuper * 6 * sizeof(float));
 }
+
+static long long brick_total(long long N) {
+  const long long bpa = (N + 3) / 4, bpz = (N + 4 * kZPts - 1) / (4 * kZPts);
+  return bpa * bpa * bpz;
+}
+static size_t queue_bytes(long long bricks) { return al256(sizeof(GridQueue) + (size_t)bricks * sizeof(int2)); }
 
 int grid_build_batch_launch(const GridSpec* specs, int n, void* workspace, hipStream_t stream, int* err_dev,
                             hipEvent_t build_after) {
@@ -708,7 +843,11 @@ int grid_build_batch_launch(const GridSpec* specs, int n, void* workspace, hipSt
   char* w = (char*)workspace;
   GridJob* d_jobs = (GridJob*)w;
   w += al256((size_t)n * sizeof(GridJob));
-  long long max_nf = 0, max_tiles = 0, max_bricks = 0, max_super = 0;
+  long long bricks = 0;
+  for (int q = 0; q < n; ++q) bricks += brick_total(specs[q].N);
+  GridQueue* queue = (GridQueue*)w;
+  w += queue_bytes(bricks);
+  long long max_nf = 0, max_tiles = 0, max_bricks = 0;
   for (int q = 0; q < n; ++q) {
     const GridSpec& sp = specs[q];
     MO_CHECK(sp.N >= 2 && sp.N <= 2048, MO_ERR_ARG, "grid resolution %d out of range [2, 2048]", sp.N);
@@ -720,38 +859,51 @@ int grid_build_batch_launch(const GridSpec* specs, int n, void* workspace, hipSt
     J.cull = (GCull*)w; w += al256((size_t)sp.nf * sizeof(GCull));
     J.bin = (unsigned*)w; w += al256((size_t)sp.nf * sizeof(unsigned));
     J.perm = (int*)w; w += al256((size_t)sp.nf * sizeof(int));
-    J.tb = (double*)w; w += al256((size_t)J.ntiles * 6 * sizeof(double));
+    J.tb = (float*)w; w += al256((size_t)J.ntiles * 6 * sizeof(float));
     J.nsuper = (J.ntiles + kSuperTiles - 1) / kSuperTiles;
-    J.sb = (double*)w; w += al256((size_t)J.nsuper * 6 * sizeof(double));
+    J.sb = (float*)w; w += al256((size_t)J.nsuper * 6 * sizeof(float));
     J.dist64 = sp.dist64; J.dist32 = sp.dist32; J.nearest = sp.nearest;
     MO_CHECK(sp.band2 > 0.0, MO_ERR_ARG, "grid band must be positive");
     J.band2 = sp.band2;
     J.stats = sp.stats;
-    const long long bpa = (sp.N + 3) / 4, bpz = (sp.N + 4 * kZPts - 1) / (4 * kZPts);
     max_nf = std::max(max_nf, sp.nf);
     max_tiles = std::max(max_tiles, J.ntiles);
-    max_super = std::max(max_super, J.nsuper);
-    max_bricks = std::max(max_bricks, bpa * bpa * bpz);
+    max_bricks = std::max(max_bricks, brick_total(sp.N));
   }
   int rc = chain_h2d(d_jobs, jobs.data(), (size_t)n * sizeof(GridJob), stream);
   if (rc) return rc;
   const int T = 256;
   const unsigned fb = (unsigned)std::min<long long>((max_nf + T - 1) / T, 1024);
-  hipLaunchKernelGGL(k_face_bins, dim3(fb, n), dim3(T), 0, stream, d_jobs, err_dev);
+  hipLaunchKernelGGL(k_face_bins, dim3(fb, n), dim3(T), 0, stream, d_jobs, err_dev, queue);
   hipLaunchKernelGGL(k_bin_sort, dim3(n), dim3(kSortT), 0, stream, d_jobs);
   hipLaunchKernelGGL(k_face_prep, dim3(fb, n), dim3(T), 0, stream, d_jobs);
-  hipLaunchKernelGGL(k_tile_bounds, dim3((unsigned)((max_tiles + 3) / 4), n), dim3(256), 0, stream, d_jobs);
-  hipLaunchKernelGGL(k_super_bounds, dim3((unsigned)((max_super + 63) / 64), n), dim3(64), 0, stream, d_jobs);
+  hipLaunchKernelGGL(k_tile_bounds, dim3((unsigned)((max_tiles + 255) / 256), n), dim3(256), 0, stream, d_jobs);
   if (build_after) MO_HIP(hipStreamWaitEvent(stream, build_after, 0));
-  hipLaunchKernelGGL(k_grid_build, dim3((unsigned)max_bricks, n), dim3(64), 0, stream, d_jobs);
+  // Where a brick is handed over: the tail matters the more the fewer bricks
+  // share the chip, the work done twice the more the more there are: a
+  // multiple of the square root of the launch's bricks (34 tiles for one 64^3
+  // grid, 96 for one 128^3 grid, 768 for 512 64^3 grids).  Multiples 0.25,
+  // 0.5, 1, 2, 4: a 642-vertex pair 3.15, 3.15, 3.22, 3.43, 3.80 ms, a
+  // 128^3 template 4.90, 5.25, 4.69, 4.87, 5.68 ms, 48 mixed pairs 125, 116,
+  // 114, 115, 116 ms; with 4 or 8 wavefronts in the second kernel each of
+  // the three is slower.
+  const int max_tiles_brick = std::max(16, (int)(0.75 * std::sqrt((double)bricks)));
+  hipLaunchKernelGGL(k_grid_build, dim3((unsigned)max_bricks, n), dim3(64), 0, stream, d_jobs, queue,
+                     max_tiles_brick);
+  hipLaunchKernelGGL(k_grid_heavy, dim3((unsigned)std::min<long long>(512, bricks)), dim3(64 * kHeavyWaves), 0, stream,
+                     d_jobs, queue);
   MO_HIP(hipGetLastError());
   return MO_OK;
 }
 
 size_t grid_batch_workspace_bytes(const GridSpec* specs, int n) {
   size_t b = al256((size_t)n * sizeof(GridJob));
-  for (int q = 0; q < n; ++q) b += grid_job_workspace_bytes(specs[q].nf);
-  return b + 256;
+  long long bricks = 0;
+  for (int q = 0; q < n; ++q) {
+    b += grid_job_workspace_bytes(specs[q].nf);
+    bricks += brick_total(specs[q].N);
+  }
+  return b + queue_bytes(bricks) + 256;
 }
 
 size_t xform_workspace_bytes(int n) { return al256((size_t)n * sizeof(XformJob)) + 256; }
