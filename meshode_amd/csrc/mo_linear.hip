@@ -14,9 +14,9 @@
 // Here the same energy is minimized with products that never form the
 // assembled rows: A p = 1e-6 p + sum_j w_ij (p_i - p_j) + w_g^2 sum_{k in g} p_k,
 // so the equal and opposite edge forces cancel exactly in the common motion
-// of a stiff pair.  One workgroup runs preconditioned conjugate gradients in
-// FP64 on the three columns in lockstep; the preconditioner inverts exactly
-// the blocks of vertices joined by stiff edges (weight > 1e4 x the median)
+// of a stiff pair.  One workgroup or a team of them runs preconditioned
+// conjugate gradients in FP64 on the three columns in lockstep; the
+// preconditioner inverts exactly the blocks of vertices joined by stiff edges (weight > 1e4 x the median)
 // and the diagonal elsewhere.  B is assembled on the host in the
 // reference's order (linear.cc:38-89).
 //
@@ -48,12 +48,14 @@
 namespace mo {
 namespace {
 
-constexpr int kCGThreads = 1024;
-constexpr int kTeamRows = 4096;   // systems this large run on a team of workgroups
+constexpr int kCGThreads = 1024;      // one workgroup
+constexpr int kCGTeamThreads = 512;   // each workgroup of a team
+constexpr int kTeamRows = 4096;       // systems this large run on a team of workgroups
 constexpr int kMaxBlock = 64;
 
 struct CGArgs {
   int n, ng;            // ng = 0: no cluster term
+  int blocks;           // nonzero: some preconditioner block has more than one row
   double c0;            // diagonal coefficient (1e-6 LinearEstimation, 1 WithRot)
   const double* dg;     // [n] per-row diagonal coefficients, or null for c0
   const int* rp;        // [n+1] Laplacian rows
@@ -70,166 +72,240 @@ struct CGArgs {
   const double* binv;
   const double* B;      // [n,3]
   double* X;            // [n,3] in: rest positions, out: solution
-  double* R;
-  double* Z;
+  double* R;            // exchanged where blocks
+  double* Z;            // exchanged
   double* P;
   double* Q;
-  double* S;            // [ng,3] cluster sums
+  double* S;            // [ng,3] cluster sums, exchanged
   int max_iter;
   double rtol;
   int* info;
 };
 
-__device__ inline void cluster_sums(const CGArgs& a, const double* __restrict__ Y, int g0, int gstride) {
+// What the members of a team exchange (Z, S, and R where a block spans rows)
+// moves only through device-coherent accesses, as TagTeam asks; one
+// workgroup uses plain ones.
+template <bool kTeam>
+__device__ inline double ld(const double* p) { return kTeam ? load_coherent(p) : *p; }
+template <bool kTeam>
+__device__ inline void st(double* p, double v) {
+  if (kTeam) store_coherent(p, v);
+  else *p = v;
+}
+
+template <bool kTeam>
+__device__ inline void cluster_sums(const CGArgs& a, int g0, int gstride) {
   for (int g = g0; g < a.ng; g += gstride) {
     double s0 = 0, s1 = 0, s2 = 0;
     for (int k = a.cp[g]; k < a.cp[g + 1]; ++k) {
-      const int m = a.cm[k];
-      s0 += Y[3 * m];
-      s1 += Y[3 * m + 1];
-      s2 += Y[3 * m + 2];
+      const double* z = a.Z + 3 * (size_t)a.cm[k];
+      s0 += ld<kTeam>(z);
+      s1 += ld<kTeam>(z + 1);
+      s2 += ld<kTeam>(z + 2);
     }
-    a.S[3 * g] = s0;
-    a.S[3 * g + 1] = s1;
-    a.S[3 * g + 2] = s2;
+    double* S = a.S + 3 * (size_t)g;
+    st<kTeam>(S, s0);
+    st<kTeam>(S + 1, s1);
+    st<kTeam>(S + 2, s2);
   }
 }
 
-// (A y)_i from edge differences, the cluster sums and the c0 diagonal
-__device__ inline void apply_row(const CGArgs& a, const double* __restrict__ Y, int i, double* out) {
-  const double yi[3] = {Y[3 * i], Y[3 * i + 1], Y[3 * i + 2]};
+// (A z)_i from edge differences, the cluster sums and the diagonal; four
+// neighbours' values are in flight at once (each is a trip to memory)
+template <bool kTeam>
+__device__ inline void apply_row(const CGArgs& a, int i, const double (&zi)[3], double (&out)[3]) {
   double acc[3] = {0, 0, 0};
-  for (int e = a.rp[i]; e < a.rp[i + 1]; ++e) {
-    const int j = a.ci[e];
-    const double we = a.w[e];
-    for (int c = 0; c < 3; ++c) acc[c] += we * (yi[c] - Y[3 * j + c]);
+  const int e1 = a.rp[i + 1];
+  for (int e = a.rp[i]; e < e1; e += 4) {
+    double z[4][3], we[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int f = e + k < e1 ? e + k : e1 - 1;
+      const double* zj = a.Z + 3 * (size_t)a.ci[f];
+      we[k] = e + k < e1 ? a.w[f] : 0.0;
+      for (int c = 0; c < 3; ++c) z[k][c] = ld<kTeam>(zj + c);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (e + k < e1)
+        for (int c = 0; c < 3; ++c) acc[c] += we[k] * (zi[c] - z[k][c]);
   }
   double cl[3] = {0, 0, 0};
   if (a.ng) {
     const int g = a.cid[i];
-    for (int c = 0; c < 3; ++c) cl[c] = a.cw2[g] * a.S[3 * g + c];
+    for (int c = 0; c < 3; ++c) cl[c] = a.cw2[g] * ld<kTeam>(a.S + 3 * (size_t)g + c);
   }
   const double d0 = a.dg ? a.dg[i] : a.c0;
-  for (int c = 0; c < 3; ++c) out[c] = d0 * yi[c] + acc[c] + cl[c];
+  for (int c = 0; c < 3; ++c) out[c] = d0 * zi[c] + acc[c] + cl[c];
 }
 
-__device__ inline void precond_row(const CGArgs& a, const double* __restrict__ Rv, int i, double* out) {
-  const int s = a.pstart[i], m = a.psize[i], row = a.prow[i];
-  double z[3] = {0, 0, 0};
+// (M^-1 r)_i; own: the row's residual
+template <bool kTeam>
+__device__ inline void precond_row(const CGArgs& a, int i, const double (&own)[3], double (&z)[3]) {
+  const int m = a.psize[i], row = a.prow[i];
+  if (m == 1) {
+    const double b = a.binv[row];
+    for (int c = 0; c < 3; ++c) z[c] = b * own[c];
+    return;
+  }
+  const int s = a.pstart[i];
+  for (int c = 0; c < 3; ++c) z[c] = 0.0;
   for (int k = 0; k < m; ++k) {
     const double b = a.binv[row + k];
-    const int j = a.bmem[s + k];
-    for (int c = 0; c < 3; ++c) z[c] += b * Rv[3 * j + c];
+    const double* r = a.R + 3 * (size_t)a.bmem[s + k];
+    for (int c = 0; c < 3; ++c) z[c] += b * ld<kTeam>(r + c);
   }
-  for (int c = 0; c < 3; ++c) out[c] = z[c];
 }
 
-// Preconditioned CG on the three right-hand sides, by one workgroup
-// (SoloTeam) or by all workgroups of a cooperative grid (GridTeam: rows
-// split as in the LM team solver, FP64 partials summed in rank order).
-template <class Team>
-__device__ inline void cg3_body(const CGArgs& a, Team& team, double* red) {
-  int sel = 0;
+// Preconditioned CG on the three right-hand sides, by one workgroup or by
+// the workgroups of a cooperative grid (rows dealt out by workgroup, FP64
+// partials exchanged through TagTeam).  As in the LM solver an iteration
+// publishes z = M^-1 r once and forms A p as A z + beta A p_prev, so it has
+// two exchanges (three with multi-row blocks or clusters).  kOne: no thread
+// has more than one row, whose vectors then stay in registers.
+//
+// What bounds it: the exchanges and the gather of z, trips through memory
+// shared by the XCDs.  21982 rows: see run_cg.
+template <bool kTeam, bool kOne>
+__device__ inline void cg3_body(const CGArgs& a, TagTeam& team) {
   const int tid = threadIdx.x, n = a.n;
-  const int i0 = team.rank() * blockDim.x + tid, nt = team.size() * blockDim.x;
+  const int i0 = team.r * blockDim.x + tid, nt = team.c * blockDim.x;
+  double x[3], r[3], p[3], q[3], z[3];
+  auto load = [&](const double* src, int i, double (&v)[3]) {
+    if (!kOne)
+      for (int c = 0; c < 3; ++c) v[c] = src[3 * (size_t)i + c];
+  };
+  auto keep = [&](double* dst, int i, const double (&v)[3]) {
+    if (!kOne)
+      for (int c = 0; c < 3; ++c) dst[3 * (size_t)i + c] = v[c];
+  };
+  auto publish = [&](double* dst, int i, const double (&v)[3]) {
+    for (int c = 0; c < 3; ++c) st<kTeam>(dst + 3 * (size_t)i + c, v[c]);
+  };
+  // the residual is published where blocks span rows, kept otherwise
+  auto keep_r = [&](int i) {
+    if (a.blocks) publish(a.R, i, r);
+    else keep(a.R, i, r);
+  };
+  auto load_r = [&](int i) {
+    if (!kOne)
+      for (int c = 0; c < 3; ++c) r[c] = a.blocks ? ld<kTeam>(a.R + 3 * (size_t)i + c) : a.R[3 * (size_t)i + c];
+  };
+  auto own_z = [&](int i) {
+    if (!kOne)
+      for (int c = 0; c < 3; ++c) z[c] = ld<kTeam>(a.Z + 3 * (size_t)i + c);
+  };
   // r = b - A x
-  cluster_sums(a, a.X, i0, nt);
+  for (int i = i0; i < n; i += nt) {
+    for (int c = 0; c < 3; ++c) x[c] = a.X[3 * (size_t)i + c];
+    publish(a.Z, i, x);
+  }
   team.barrier();
+  if (a.ng) {
+    cluster_sums<kTeam>(a, i0, nt);
+    team.barrier();
+  }
   double v[7] = {0, 0, 0, 0, 0, 0, 0};
   for (int i = i0; i < n; i += nt) {
     double ax[3];
-    apply_row(a, a.X, i, ax);
+    load(a.X, i, x);
+    apply_row<kTeam>(a, i, x, ax);
     for (int c = 0; c < 3; ++c) {
-      const double b = a.B[3 * i + c];
-      const double r = b - ax[c];
-      a.R[3 * i + c] = r;
+      const double b = a.B[3 * (size_t)i + c];
+      r[c] = b - ax[c];
       v[3 + c] += b * b;
-      v[6] = fmax(v[6], fabs(r));
+      v[6] = fmax(v[6], fabs(r[c]));
     }
+    keep_r(i);
   }
   team.barrier();
-  // z = M^-1 r, p = z
   for (int i = i0; i < n; i += nt) {
-    double z[3];
-    precond_row(a, a.R, i, z);
+    load_r(i);
+    precond_row<kTeam>(a, i, r, z);
     for (int c = 0; c < 3; ++c) {
-      a.Z[3 * i + c] = z[c];
-      a.P[3 * i + c] = z[c];
-      v[c] += a.R[3 * i + c] * z[c];
+      p[c] = q[c] = 0.0;
+      v[c] += r[c] * z[c];
     }
+    keep(a.P, i, p);
+    keep(a.Q, i, q);
+    publish(a.Z, i, z);
   }
-  team.template reduce<6, 1>(v, red, sel);
-  double rz[3] = {v[0], v[1], v[2]};
+  team.template reduce<6, 1>(v);
+  double rz[3] = {v[0], v[1], v[2]}, beta[3] = {0, 0, 0};
   // one tolerance for the three columns, relative to the largest |b|
   const double tol2 = a.rtol * a.rtol * fmax(v[3], fmax(v[4], v[5]));
   bool done = v[6] == 0.0;
   int it = 0;
   while (!done && it < a.max_iter) {
-    cluster_sums(a, a.P, i0, nt);
-    team.barrier();
+    if (a.ng) {
+      cluster_sums<kTeam>(a, i0, nt);
+      team.barrier();
+    }
     double pq[3] = {0, 0, 0};
     for (int i = i0; i < n; i += nt) {
-      double q[3];
-      apply_row(a, a.P, i, q);
+      double az[3];
+      own_z(i);
+      apply_row<kTeam>(a, i, z, az);
+      load(a.P, i, p);
+      load(a.Q, i, q);
       for (int c = 0; c < 3; ++c) {
-        a.Q[3 * i + c] = q[c];
-        pq[c] += a.P[3 * i + c] * q[c];
+        p[c] = z[c] + beta[c] * p[c];
+        q[c] = az[c] + beta[c] * q[c];
+        pq[c] += p[c] * q[c];
       }
+      keep(a.P, i, p);
+      keep(a.Q, i, q);
     }
-    team.template reduce<3, 0>(pq, red, sel);
+    team.template reduce<3, 0>(pq);
     double alpha[3];
     for (int c = 0; c < 3; ++c) alpha[c] = pq[c] > 0 ? rz[c] / pq[c] : 0.0;
     double w[6] = {0, 0, 0, 0, 0, 0};
-    for (int i = i0; i < n; i += nt)
-      for (int c = 0; c < 3; ++c) {
-        a.X[3 * i + c] += alpha[c] * a.P[3 * i + c];
-        const double r = a.R[3 * i + c] - alpha[c] * a.Q[3 * i + c];
-        a.R[3 * i + c] = r;
-        w[3 + c] += r * r;
-      }
-    team.barrier();
     for (int i = i0; i < n; i += nt) {
-      double z[3];
-      precond_row(a, a.R, i, z);
+      load(a.X, i, x);
+      load(a.P, i, p);
+      load(a.Q, i, q);
+      load_r(i);
       for (int c = 0; c < 3; ++c) {
-        a.Z[3 * i + c] = z[c];
-        w[c] += a.R[3 * i + c] * z[c];
+        x[c] += alpha[c] * p[c];
+        r[c] -= alpha[c] * q[c];
+        w[3 + c] += r[c] * r[c];
       }
+      keep(a.X, i, x);
+      keep_r(i);
     }
-    team.template reduce<6, 0>(w, red, sel);
+    if (a.blocks) team.barrier();
+    for (int i = i0; i < n; i += nt) {
+      load_r(i);
+      precond_row<kTeam>(a, i, r, z);
+      for (int c = 0; c < 3; ++c) w[c] += r[c] * z[c];
+      publish(a.Z, i, z);
+    }
+    team.template reduce<6, 0>(w);
     ++it;
     done = w[3] <= tol2 && w[4] <= tol2 && w[5] <= tol2;
-    if (done) break;
-    double beta[3];
     for (int c = 0; c < 3; ++c) {
       beta[c] = rz[c] > 0 ? w[c] / rz[c] : 0.0;
       rz[c] = w[c];
     }
-    for (int i = i0; i < n; i += nt)
-      for (int c = 0; c < 3; ++c) a.P[3 * i + c] = a.Z[3 * i + c] + beta[c] * a.P[3 * i + c];
-    team.barrier();
   }
+  if (kOne && i0 < n)
+    for (int c = 0; c < 3; ++c) a.X[3 * (size_t)i0 + c] = x[c];
   if (tid == 0 && team.leader()) {
     a.info[0] = it;
     a.info[1] = done ? 1 : 0;
   }
 }
 
-__global__ void k_zero_words(int* p, int n) {
-  if ((int)threadIdx.x < n) p[threadIdx.x] = 0;
+__global__ void k_zero_words(unsigned long long* p, int n) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
 }
 
-__global__ __launch_bounds__(kCGThreads) void k_cg3(CGArgs a) {
-  __shared__ double red[2 * 8 * kMaxWaves];
-  SoloTeam team;
-  cg3_body(a, team, red);
-}
-
-__global__ __launch_bounds__(kCGThreads) void k_cg3_team(CGArgs a, unsigned* cnt, double* part, int* abort_flag,
-                                                          long long limit) {
-  __shared__ double red[2 * 8 * kMaxWaves];
-  GridTeam team{(int)blockIdx.x, (int)gridDim.x, cnt, part, abort_flag, limit, 0u, 0};
-  cg3_body(a, team, red);
+template <bool kTeam, bool kOne>
+__global__ __launch_bounds__(kTeam ? kCGTeamThreads : kCGThreads) void k_cg3(CGArgs a, unsigned long long* slots,
+                                                                             int* abort_flag, long long limit) {
+  __shared__ double red[kTagRed];
+  TagTeam team{kTeam ? (int)blockIdx.x : 0, kTeam ? (int)gridDim.x : 1, slots, abort_flag, limit, red, 0u, 0};
+  cg3_body<kTeam, kOne>(a, team);
 }
 
 struct System {
@@ -510,7 +586,7 @@ int run_cg(const System& S, double* X, int max_iter, double rtol, int* iteration
   const size_t nn = (size_t)S.n, ng = (size_t)S.ng, nnz = S.ci.size(), nb = S.bmem.size(), ni = S.binv.size();
   const size_t bytes = al((nn + 1) * 4) + al(nnz * 4) + al(nnz * 8) + al(nn * 4) + al((ng + 1) * 4) + al(nn * 4) +
                        al(ng * 8) + 3 * al(nn * 4) + al(nb * 4) + al(ni * 8) + 5 * al(nn * 24) + al(ng * 24) +
-                       al(32) + al(nn * 8) + al(2 * kMaxTeam * 8 * 8);
+                       al(nn * 8) + al((kTagSlotWords + 4) * 8);
   char* ws = nullptr;
   MO_HIP(hipMallocAsync((void**)&ws, bytes, s));
   char* w = ws;
@@ -541,9 +617,10 @@ int run_cg(const System& S, double* X, int max_iter, double rtol, int* iteration
   a.P = (double*)take(nn * 24);
   a.Q = (double*)take(nn * 24);
   a.S = (double*)take(ng * 24);
-  a.info = (int*)take(32);   // info[0..1]; team counter [4], abort flag [5]
   double* d_dg = (double*)take(S.dg.size() * 8);
-  double* d_part = (double*)take(2 * kMaxTeam * 8 * 8);   // team partials [2][kMaxTeam][8]
+  unsigned long long* d_slots = (unsigned long long*)take((kTagSlotWords + 4) * 8);   // team slots, then info, abort flag
+  a.info = (int*)(d_slots + kTagSlotWords);   // info[0..1]; abort flag [2]
+  a.blocks = S.bmem.size() == S.binv.size() ? 0 : 1;
   a.dg = S.dg.empty() ? nullptr : d_dg;
   a.rp = d_rp; a.ci = d_ci; a.w = d_w; a.cid = d_cid; a.cp = d_cp; a.cm = d_cm; a.cw2 = d_cw2;
   a.pstart = d_ps; a.psize = d_pz; a.prow = d_pr; a.bmem = d_bm; a.binv = d_bi; a.B = d_B;
@@ -570,57 +647,52 @@ int run_cg(const System& S, double* X, int max_iter, double rtol, int* iteration
       break;
     }
     // Systems of at least kTeamRows rows run on a cooperative grid of
-    // ceil(n / kCGThreads) workgroups (at most lm_team_max(), at most what is
-    // co-resident), one such launch at a time in the process.
+    // ceil(n / kCGTeamThreads) workgroups (at most kMaxTeam, at most what is
+    // co-resident), one such launch at a time in the process.  21982 rows:
+    // 6.9 ms on 22 workgroups with fenced barriers and the vectors in memory,
+    // 2.1 ms on 43.
+    hipLaunchKernelGGL(k_zero_words, dim3(8), dim3(256), 0, s, d_slots, kTagSlotWords + 4);
+    int* abort_flag = a.info + 2;
+    int dev = 0, khz = 0, cus = 0, per = 0;
+    if (hipGetLastError() != hipSuccess || hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess) {
+      rc = fail(MO_ERR_HIP, "%s: clear or device query failed", who);
+      break;
+    }
+    long long limit = (long long)std::max(khz, 1) * 1000LL * 20;   // a 20 s bound on any one wait
+    if (const char* wv = getenv("MO_LM_TEAM_WAIT_US")) limit = atoll(wv) * (long long)std::max(khz, 1) / 1000LL;
     int team = 1;
-    if (S.n >= kTeamRows) {
-      int dev = 0, cus = 0, per = 0;
-      if (hipGetDevice(&dev) == hipSuccess &&
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
-          hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_cg3_team, kCGThreads, 0) == hipSuccess)
-        team = std::min({(S.n + kCGThreads - 1) / kCGThreads, lm_team_max(), per * cus});
-      team = std::max(team, 1);
+    const bool one = S.n <= kCGTeamThreads * kMaxTeam;
+    const void* kern = one ? (const void*)k_cg3<true, true> : (const void*)k_cg3<true, false>;
+    if (S.n >= kTeamRows &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess &&
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, kCGTeamThreads, 0) == hipSuccess) {
+      team = std::min((S.n + kCGTeamThreads - 1) / kCGTeamThreads, kMaxTeam);
+      if (team > per * cus) team = 1;
     }
     std::unique_lock<std::mutex> team_lock(team_launch_mutex(), std::defer_lock);
+    void* args[] = {(void*)&a, (void*)&d_slots, (void*)&abort_flag, (void*)&limit};
     if (team > 1) {
-      int dev = 0, khz = 0;
-      if (hipGetDevice(&dev) != hipSuccess ||
-          hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess) {
-        rc = fail(MO_ERR_HIP, "%s: device query failed", who);
-        break;
-      }
-      long long limit = (long long)std::max(khz, 1) * 1000LL * 20;   // a 20 s bound on any one wait
-      if (const char* wv = getenv("MO_LM_TEAM_WAIT_US")) limit = atoll(wv) * (long long)std::max(khz, 1) / 1000LL;
-      unsigned* cnt = (unsigned*)a.info + 4;                  // counter + abort flag after info[0..1]
-      int* abort_flag = (int*)a.info + 5;
-      double* part = d_part;
-      hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s, a.info, 8);
-      if (hipGetLastError() != hipSuccess) {
-        rc = fail(MO_ERR_HIP, "%s: clear failed", who);
-        break;
-      }
-      void* args[] = {(void*)&a, (void*)&cnt, (void*)&part, (void*)&abort_flag, (void*)&limit};
       team_lock.lock();
-      if (hipLaunchCooperativeKernel((const void*)k_cg3_team, dim3(team), dim3(kCGThreads), args, 0, s) !=
-          hipSuccess) {
+      if (hipLaunchCooperativeKernel(kern, dim3(team), dim3(kCGTeamThreads), args, 0, s) != hipSuccess) {
         (void)hipGetLastError();   // refused: nothing was launched; solve on one workgroup
         team = 1;
       }
     }
     if (team == 1) {
-      hipLaunchKernelGGL(k_cg3, dim3(1), dim3(kCGThreads), 0, s, a);
-      if (hipGetLastError() != hipSuccess) {
+      const void* solo = S.n <= kCGThreads ? (const void*)k_cg3<false, true> : (const void*)k_cg3<false, false>;
+      if (hipLaunchKernel(solo, dim3(1), dim3(kCGThreads), args, 0, s) != hipSuccess) {
         rc = fail(MO_ERR_HIP, "%s: launch failed", who);
         break;
       }
     }
-    int info[6] = {0, 0, 0, 0, 0, 0};
-    if (hipMemcpyAsync(info, a.info, 24, hipMemcpyDeviceToHost, s) != hipSuccess ||
+    int info[3] = {0, 0, 0};
+    if (hipMemcpyAsync(info, a.info, 12, hipMemcpyDeviceToHost, s) != hipSuccess ||
         hipStreamSynchronize(s) != hipSuccess) {
       rc = fail(MO_ERR_HIP, "%s: solve failed", who);
       break;
     }
-    if (team > 1 && info[5]) {
+    if (team > 1 && info[2]) {
       rc = fail(MO_ERR_HIP, "%s: a team barrier wait exceeded its bound (result invalid)", who);
       break;
     }
