@@ -71,3 +71,33 @@ def test_linear_estimation_rot_rigid_motion(gpu, n):
     cad.linear_estimation_rot(x, torch.from_numpy(F).to(gpu), torch.from_numpy(TV).to(gpu), 1.0)
     # scale = s / (s + 1e-8) with s > 1e-2, the sum of a vertex's edge lengths
     assert np.abs(x.cpu().numpy() - TV).max() <= 1e-5
+
+
+@pytest.mark.parametrize("spokes", [31, 32, 33, 100])
+def test_linear_estimation_merged_edges(gpu, spokes):
+    """A fan around vertex 0 (its edges past a short insertion sort), in both
+    orders of the faces' corners, some faces repeated: the parallel edges'
+    weights add up, and vertices in no face stay alone."""
+    print(f"[linear merge] {spokes}", flush=True)
+    rng = np.random.default_rng(spokes)
+    n = spokes + 3
+    V = rng.random((n, 3))
+    order = rng.permutation(spokes) + 1
+    F = np.array([[0, order[i], order[(i + 1) % spokes]] for i in range(spokes)])
+    F[::2] = F[::2, ::-1]
+    F = np.concatenate([F, F[3:9, [1, 2, 0]], F[5:6]]).astype(np.int32)
+    w = lambda d: (2.0 * 2e-2 / (d + 1e-8)) ** 2                       # noqa: E731
+    GV = V + 0.05 * rng.normal(size=V.shape)
+    a, b = np.concatenate([F[:, 0], F[:, 1], F[:, 2]]), np.concatenate([F[:, 1], F[:, 2], F[:, 0]])
+    r = w(np.linalg.norm(V[a] - V[b], axis=1))[:, None] * (V[a] - V[b])
+    B = (1.0 + 1e-6) * GV
+    np.add.at(B, a, r)
+    np.add.at(B, b, -r)
+    W = np.zeros((n, n))
+    np.add.at(W, (a, b), w(np.linalg.norm(V[a] - V[b], axis=1)))
+    W += W.T
+    want = np.linalg.solve(np.diag(W.sum(1) + 1.0 + 1e-6) - W, B)
+    x = torch.from_numpy(V.copy()).to(gpu)
+    cad.linear_estimation(x, torch.from_numpy(F).to(gpu), torch.zeros(0, 2, dtype=torch.int32, device=gpu),
+                          torch.arange(n, dtype=torch.int32, device=gpu), torch.from_numpy(GV).to(gpu), 2.0)
+    assert np.linalg.norm(x.cpu().numpy() - want) <= 1e-10 * np.linalg.norm(want)
