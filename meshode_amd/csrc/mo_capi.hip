@@ -844,7 +844,11 @@ int lm_core(const std::vector<CorePair>& pairs, const mo_lm_options& opt, mo_lm_
   hipLaunchKernelGGL(k_make_x0, io_grid, dim3(256), 0, ts, d_io, deg, x0, u);
   MO_HIP(hipGetLastError());
   // per pair and register/LDS team shape: the largest chunk's adjacency entries
-  if ((rc = lm_lds_chunk_entries(d_pairs, adj, np, d_chunk, ts))) return rc;
+  const size_t lds_cap = (size_t)std::max(0, device_lds_limit() - 4096);
+  const LMArrays A{x0, u, adj, raw, work, wt};
+  if ((rc = lm_lds_chunk_entries(d_pairs, A, np, nvalloc, opt.kernel_variant == 0 ? (int)max_nv : 0, lds_cap, d_chunk,
+                                 ts)))
+    return rc;
   std::vector<int> pstat(2 * np), hchunk(4 * np);
   int herr = 0;
   {
@@ -867,7 +871,6 @@ int lm_core(const std::vector<CorePair>& pairs, const mo_lm_options& opt, mo_lm_
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return pairs[a].nv > pairs[b].nv; });
   const int nb = lm_lds_buckets();
-  const size_t lds_cap = (size_t)std::max(0, device_lds_limit() - 4096);
   std::vector<std::vector<int>> bucket(nb + 1);
   std::vector<size_t> bucket_lds(nb + 1, 0);
   for (int p : order) {
@@ -876,9 +879,10 @@ int lm_core(const std::vector<CorePair>& pairs, const mo_lm_options& opt, mo_lm_
     // the register/LDS kernel packs a vertex's LDS adjacency offset and count
     // into 16 bits each and a neighbour index (or the zero slot, index nv)
     // into 15: a pair qualifies only when all of them fit
-    const int padded = hchunk[4 * p + 3];   // entries with every count rounded up to even
+    // entries with every count rounded up to even (negative: a team's pair)
+    const int padded = hchunk[4 * p + 3];
     if (opt.kernel_variant == 0 && c.kind != 2 && c.nv > 0 && c.nv <= 32767 && pstat[2 * p + 1] <= 2 &&
-        padded < 65536) {
+        padded >= 0 && padded < 65536) {
       b = lm_lds_bucket_for((int)c.nv);
       if (b >= 0 && lm_lds_bytes((int)c.nv, padded) > lds_cap) b = -1;
     }
@@ -894,7 +898,6 @@ int lm_core(const std::vector<CorePair>& pairs, const mo_lm_options& opt, mo_lm_
   }
   start[nb + 1] = (int)plist.size();
   if ((rc = chain_h2d(d_plist, plist.data(), np * sizeof(int), s))) return rc;
-  LMArrays A{x0, u, adj, raw, work, wt};
   const LMOptionsDev dopt = to_dev_options(opt);
   MO_CHECK(nb <= kMaxLdsLaunches, MO_ERR_STATE, "%d register/LDS shapes exceed the %d work counters", nb,
            kMaxLdsLaunches);
@@ -958,11 +961,16 @@ int lm_core(const std::vector<CorePair>& pairs, const mo_lm_options& opt, mo_lm_
       const long long ent = hchunk[4 * p + b];
       return c <= lm_lds_team_max() && ent < 65536 && lm_lds_team_bytes((int)ch, ent) <= lds_cap;
     };
+    // ... the halo kernel first: its chunks' LDS was counted with the topology
+    auto halo_fits = [&](int p) {
+      const int need = hchunk[4 * p + 3];
+      return need < 0 && (size_t)-(long long)need <= lds_cap;
+    };
     for (int p : bucket[nb]) {
       const CorePair& c = pairs[p];
       bool ok = opt.kernel_variant == 0 && c.kind != 2 && c.nv > 0 && pstat[2 * p + 1] <= 2;
       if (ok) {
-        ok = false;
+        ok = halo_fits(p);
         for (int b : lm_lds_team_order()) ok = ok || lds_team_fits(p, b);
       }
       (ok ? lds_cand : rest).push_back(p);
@@ -976,6 +984,12 @@ int lm_core(const std::vector<CorePair>& pairs, const mo_lm_options& opt, mo_lm_
     std::vector<size_t> lds_of(nls, 0);
     for (size_t k = 0; k < lds_cand.size(); ++k) {
       const int p = lds_cand[k];
+      if (halo_fits(p)) {
+        int ch = 0, c = 0;
+        pshape[k] = lm_lds_halo_shape((int)pairs[p].nv, &ch, &c);
+        lds_of[pshape[k]] = std::max(lds_of[pshape[k]], (size_t)-(long long)hchunk[4 * p + 3]);
+        continue;
+      }
       for (int b : lm_lds_team_order())
         if (pshape[k] < 0 && lds_team_fits(p, b)) {
           int T = 0, V = 0;

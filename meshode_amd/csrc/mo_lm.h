@@ -109,9 +109,12 @@ int lm_lds_launch(int bucket, const LMPairDesc* pairs_dev, const int* plist, int
 // Multi-workgroup register/LDS kernel (k_lm_solve_lds_team) for pairs
 // above one workgroup's capacity with multiplicities <= 2: workgroup r of a
 // team owns a contiguous chunk of the pair's vertices.  Team shape b (0..2)
-// holds 4096, 3072 or 2048 vertices per workgroup; lm_lds_chunk_entries
-// writes, per pair, the largest chunk's adjacency entry count for each
-// shape (3 ints per pair); lm_lds_team_bytes gives the dynamic LDS of a
+// holds 4096, 3072 or 2048 vertices per workgroup; shapes 3 and 4 are the
+// halo kernel's (k_lm_solve_lds_halo).  lm_lds_chunk_entries writes, per
+// pair, the largest chunk's adjacency entry count for shapes 0..2, then the
+// one-workgroup kernel's padded entry count or, for a pair that only a team
+// can hold and whose halo was counted, minus the halo kernel's LDS bytes
+// (4 ints per pair); lm_lds_team_bytes gives the dynamic LDS of a
 // chunk; wg_dev entries are (team, rank, team size, chunk); cnt / part /
 // abort_flag as for lm_team_launch.  Returns kCoopRefused like
 // lm_team_launch.
@@ -123,7 +126,12 @@ int lm_lds_team_max();   // largest team of the register/LDS team kernel
 int lm_lds_team_shape(int b, int* threads, int* vertices_per_thread);
 size_t lm_lds_team_bytes(int chunk, long long entries);
 int lm_lds_team_capacity(int b, size_t lds_bytes);
-int lm_lds_chunk_entries(const LMPairDesc* pairs_dev, const int2* adj, int np, int* out_dev, hipStream_t s);
+// max_nv: the batch's largest pair; lds_cap: dynamic LDS a workgroup may use.
+int lm_lds_chunk_entries(const LMPairDesc* pairs_dev, const LMArrays& arrays, int np, long long total_vertices,
+                         int max_nv, size_t lds_cap, int* out_dev, hipStream_t s);
+// Team shape, chunk and workgroups of the halo kernel for a pair of nv
+// vertices (-1: too large).
+int lm_lds_halo_shape(int nv, int* chunk, int* workgroups);
 int lm_lds_team_launch(int b, const LMPairDesc* pairs_dev, const int* plist, const int4* wg_dev, int nwg,
                        const LMArrays& arrays, const LMOptionsDev& opt, LMResultDev* results_dev,
                        long long total_vertices, size_t lds_bytes, unsigned* cnt, double* part, int* abort_flag,

@@ -43,7 +43,11 @@ namespace mo {
 
 namespace {
 
-enum GSlot { gGR = 1, gS = 2, gDG = 3, gZ = 4 };   // global slots of LMArrays::work used here
+// global slots of LMArrays::work used here; gOrder: a large pair's spatial
+// order (int perm[nv], inv[nv] and the sort's scratch), gSlots: a pair's
+// TagTeam words
+enum GSlot { gGR = 1, gS = 2, gDG = 3, gZ = 4, gOrder = 5, gSlots = 6 };
+static_assert(gSlots < kLMWorkSlots, "work slots");
 
 // Block-wide exclusive scan of one int per thread (T <= 1024).
 __device__ inline int block_exclusive_scan(int x, int* buf, int& total) {
@@ -86,14 +90,22 @@ __device__ inline int opaque(int x) {
   return x;
 }
 
-// The solver body, shared by the one-workgroup kernel (Team = LdsSolo: the
-// workgroup owns all nv vertices, neighbours come from its LDS array) and
-// the multi-workgroup kernel (Team = LdsTeam: workgroup r owns the
-// contiguous chunk [lo, hi) of the pair's vertices; a neighbour in another
-// chunk is read from the pair's global publication array, which every
-// owner writes next to its LDS copy before the team barrier).  Entry: an
-// adjacency entry type (uint16 local indices for the solo kernel, uint32
-// pair indices for the team kernel).
+// First record of a halo team's copies of neighbours: behind the own
+// vertices and behind the set-up's bitmap (a bit per vertex of the pair and
+// a 16-bit count per word).
+__host__ __device__ inline int halo_base(int own, int nv) {
+  const int words = (nv + 31) / 32, overlay = (words * 6 + 15) / 16;
+  return own > overlay ? own : overlay;
+}
+
+// The solver body, shared by the one-workgroup kernel (LdsSolo: all nv
+// vertices in the workgroup's LDS array), the halo team (LdsHalo: a
+// workgroup owns a range of the pair's vertices and keeps copies of the
+// neighbours outside it behind them, read from the pair's publication array
+// once per publication) and the team for meshes whose
+// halo does not fit (LdsTeam: every access to such a neighbour reads the
+// publication array).  Entry: an adjacency entry type (uint16 local indices,
+// uint32 pair indices for LdsTeam).
 template <int T, int VPT, class Team, class Entry>
 __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const LMArrays& A,
                                  const LMOptionsDev& opt, LMResultDev* __restrict__ res, long long totalV,
@@ -103,8 +115,7 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
   const bool o_pcg_warm = kPcgWarmStart;
   const int o_pcg_max = opt.pcg_max_iterations;
   const int tid = threadIdx.x;
-  const int lo = team.lo;                  // owned vertices: lo + t + k T < hi
-  const int own = team.hi - team.lo;
+  const int own = team.hi - team.lo;       // owned vertices: local index t + k T < own
   const long long vb = P.vbase;
   const float l2 = P.lambda * P.lambda;
   const float* __restrict__ grid = P.grid;
@@ -117,13 +128,11 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
   float4* __restrict__ S = A.work + (size_t)gS * totalV + vb;
   float4* __restrict__ DG = A.work + (size_t)gDG * totalV + vb;
   float4* __restrict__ ZG = A.work + (size_t)gZ * totalV + vb;   // team: published vectors
-  // paired layout (one workgroup per pair): a zero vector at VEC[own], and
-  // every vertex's entry list padded to even length with it, so the PCG
-  // product reads two entries per 32-bit LDS word
+  // paired layout: a zero vector behind the vertex records, and every
+  // vertex's entry list padded to even length with it, so the PCG product
+  // reads two entries per 32-bit LDS word
   constexpr bool kPaired = Team::kPaired;
-  constexpr int kZeroSlots = kPaired ? 1 : 0;
-  float4* VEC = (float4*)smem;                                      // own vertices, local index
-  Entry* LCSR = (Entry*)(smem + (size_t)(own + kZeroSlots) * sizeof(float4));
+  float4* VEC = (float4*)smem;             // own vertices at their local index, then a halo team's copies of neighbours
   int sel = 0;
   const long long clock_start = wall_clock64();
 
@@ -131,46 +140,116 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
   // each own vertex's (LDS offset << 16) | count lives in VEC[il].w for the
   // whole solve (publications write x, y, z only), so it costs no register
   float uniform_m = 0.f;   // paired layout: the pair's multiplicity when all entries share it, else 0
+  Entry* LCSR;
   {
     int cnt[VPT], gst[VPT], mine = 0;
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const int il = opaque(tid + k * T), i = lo + il;
+      const int il = opaque(tid + k * T);
       cnt[k] = 0;
       gst[k] = 0;
       if (il < own) {
-        const int2 a = ADJ[i];
+        const int2 a = ADJ[team.index(il)];
         gst[k] = a.x;
         cnt[k] = a.y;
         mine += kPaired ? a.y + (a.y & 1) : a.y;
       }
     }
+    if constexpr (Team::kHalo) {
+      // distinct neighbours owned elsewhere: a bitmap over the pair's ranks
+      // (at the LDS' start, dead before the own records are written), its
+      // words' prefix counts, and each one's rank in the w of its record
+      unsigned* bm = (unsigned*)smem;
+      const int nwords = (P.nv + 31) >> 5;
+      unsigned short* pre = (unsigned short*)(bm + nwords);
+      if ((size_t)halo_base(own, P.nv) * sizeof(float4) > lds_bytes) {
+        team.give_up();
+        return;
+      }
+      for (int q = tid; q < nwords; q += blockDim.x) bm[q] = 0u;
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < VPT; ++k)
+        for (int e = 0; e < cnt[k]; ++e) {
+          const int q = team.rank(nb_index(NB[gst[k] + e]));
+          if ((unsigned)(q - team.lo) < (unsigned)own) continue;
+          team.shared |= 1u << k;
+          atomicOr(&bm[q >> 5], 1u << (q & 31));
+        }
+      __syncthreads();
+      const int per = (nwords + (int)blockDim.x - 1) / (int)blockDim.x;
+      const int q0 = min(nwords, tid * per), q1 = min(nwords, q0 + per);
+      int bits = 0;
+      for (int q = q0; q < q1; ++q) bits += __popc(bm[q]);
+      int nh;
+      int h = block_exclusive_scan(bits, scan_buf, nh);
+      team.nhalo = nh;
+      team.hbase = halo_base(own, P.nv);
+      for (int q = q0; q < q1; ++q) {
+        pre[q] = (unsigned short)h;
+        const int n = __popc(bm[q]);
+        if ((size_t)(team.hbase + h + n) * sizeof(float4) <= lds_bytes) {
+          int r = team.hbase + h;
+          for (unsigned m = bm[q]; m; m &= m - 1) reinterpret_cast<int*>(VEC + r++)[3] = q * 32 + __ffs((int)m) - 1;
+        }
+        h += n;
+      }
+      __syncthreads();
+    }
+    const int zero = team.hbase + team.nhalo;   // the zero vector's index
+    const int records = zero + (kPaired ? 1 : 0);
+    LCSR = (Entry*)(smem + (size_t)records * sizeof(float4));
     int total;
     int off = block_exclusive_scan(mine, scan_buf, total);
     // the launch's LDS was sized from the same adjacency; a mismatch (a
     // replayed graph whose inputs' faces changed) leaves the pair unsolved
     // and is reported by the host, never written past the allocation
-    if ((size_t)(own + kZeroSlots) * sizeof(float4) + (size_t)total * sizeof(Entry) > lds_bytes) return;
+    if ((size_t)records * sizeof(float4) + (size_t)total * sizeof(Entry) > lds_bytes ||
+        (Team::kHalo && (records > 32767 || total > 65535))) {
+      team.give_up();
+      return;
+    }
     int has1 = 0, has2 = 0;
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      {
-        const int il = opaque(tid + k * T);
-        if (il < own) reinterpret_cast<float*>(VEC + il)[3] = __uint_as_float(((unsigned)off << 16) | (unsigned)cnt[k]);
-      }
-      for (int e = 0; e < cnt[k]; ++e) {
+      int o = off;
+      for (int e = 0; e < cnt[k]; ++e, ++o) {
         const unsigned en = NB[gst[k] + e];
         has1 |= (en >> 24) == 1u;
         has2 |= (en >> 24) == 2u;
-        LCSR[off + e] = (Entry)((nb_index(en) << 1) | ((en >> 24) - 1u));
+        int j = team.rank(nb_index(en));
+        if constexpr (Team::kHalo) {
+          if ((unsigned)(j - team.lo) < (unsigned)own) {
+            j -= team.lo;
+          } else {
+            const unsigned* bm = (const unsigned*)smem;
+            const unsigned short* pre = (const unsigned short*)(bm + ((P.nv + 31) >> 5));
+            j = team.hbase + (int)pre[j >> 5] + __popc(bm[j >> 5] & ((1u << (j & 31)) - 1u));
+          }
+        }
+        LCSR[o] = (Entry)(((unsigned)j << 1) | ((en >> 24) - 1u));
       }
-      if (kPaired && (cnt[k] & 1)) LCSR[off + cnt[k]] = (Entry)((unsigned)own << 1);
+      if (kPaired && (cnt[k] & 1)) LCSR[o] = (Entry)((unsigned)zero << 1);
+      off += kPaired ? cnt[k] + (cnt[k] & 1) : cnt[k];
+    }
+    if constexpr (Team::kHalo) __syncthreads();   // the bitmap is dead from here
+    off -= mine;
+#pragma unroll
+    for (int k = 0; k < VPT; ++k) {
+      const int il = opaque(tid + k * T);
+      if (il < own) reinterpret_cast<float*>(VEC + il)[3] = __uint_as_float(((unsigned)off << 16) | (unsigned)cnt[k]);
       off += kPaired ? cnt[k] + (cnt[k] & 1) : cnt[k];
     }
     if constexpr (kPaired) {
-      const int any1 = __syncthreads_or(has1), any2 = __syncthreads_or(has2);
+      int any1 = __syncthreads_or(has1), any2 = __syncthreads_or(has2);
+      if constexpr (Team::kHalo) {
+        double any[2] = {any1 ? 1.0 : 0.0, any2 ? 1.0 : 0.0};
+        team.template reduce<0, 2>(any, red, sel);
+        any1 = any[0] > 0.0;
+        any2 = any[1] > 0.0;
+      }
       uniform_m = any1 && !any2 ? 1.f : (any2 && !any1 ? 2.f : 0.f);
-      if (tid == 0) VEC[own] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (tid == 0) VEC[zero] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
   }
 
@@ -215,7 +294,12 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
           const unsigned w = *pw;
           const float4 a = VEC[opaque((int)__builtin_amdgcn_ubfe(w, 1, 15))];
           const float4 b = VEC[opaque((int)__builtin_amdgcn_ubfe(w, 17, 15))];
-          sx += a.x + b.x; sy += a.y + b.y; sz += a.z + b.z;
+          if constexpr (Team::kInOrder) {
+            sx += a.x; sy += a.y; sz += a.z;
+            sx += b.x; sy += b.y; sz += b.z;
+          } else {
+            sx += a.x + b.x; sy += a.y + b.y; sz += a.z + b.z;
+          }
         }
         sx *= uniform_m; sy *= uniform_m; sz *= uniform_m;
       } else {
@@ -225,7 +309,12 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
           const float4 a = VEC[opaque((int)__builtin_amdgcn_ubfe(w, 1, 15))];
           const float4 b = VEC[opaque((int)__builtin_amdgcn_ubfe(w, 17, 15))];
           const float ma = (float)((w & 1u) + 1u), mb = (float)(((w >> 16) & 1u) + 1u);
-          sx += ma * a.x + mb * b.x; sy += ma * a.y + mb * b.y; sz += ma * a.z + mb * b.z;
+          if constexpr (Team::kInOrder) {
+            sx += ma * a.x; sy += ma * a.y; sz += ma * a.z;
+            sx += mb * b.x; sy += mb * b.y; sz += mb * b.z;
+          } else {
+            sx += ma * a.x + mb * b.x; sy += ma * a.y + mb * b.y; sz += ma * a.z + mb * b.z;
+          }
         }
       }
     } else {
@@ -242,15 +331,16 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
   auto eval = [&](bool first, double& cv, double& ce, double& gmax) {
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const int il = opaque(tid + k * T), i = lo + il;
-      if (il < own) team.publish(VEC, ZG, il, i, U[i]);
+      const int il = opaque(tid + k * T);
+      if (il < own) team.publish(VEC, ZG, k, il, U[team.index(il)]);
     }
-    team.sync();
+    team.sync(VEC, ZG);
     double v[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const int il = opaque(tid + k * T), i = lo + il;
+      const int il = opaque(tid + k * T);
       if (il >= own) continue;
+      const int i = team.index(il);
       const float4 x0 = X0[i];
       const float4 ui = VEC[il];
       const int cs = __float_as_int(ui.w);
@@ -302,12 +392,13 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
     double v[3] = {0.0, 0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const int il = opaque(tid + k * T), i = lo + il;
+      const int il = opaque(tid + k * T);
       px[k] = py[k] = pz[k] = 0.f;
       qx[k] = qy[k] = qz[k] = 0.f;
       if (!warm) ex[k] = ey[k] = ez[k] = 0.f;
       dx[k] = dy[k] = dz[k] = 1.f;
       if (il >= own) continue;
+      const int i = team.index(il);
       const float4 s = S[i];
       const float ldk = l2 * X0[i].w;
       float4 dg;
@@ -333,24 +424,24 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
       dy[k] = ldk + fminf(dg.y * __builtin_amdgcn_rcpf(s.y * s.y) * finv_radius, 1e30f);
       dz[k] = ldk + fminf(dg.z * __builtin_amdgcn_rcpf(s.z * s.z) * finv_radius, 1e30f);
       if (warm) {
-        team.publish(VEC, ZG, il, i, make_float4(ex[k], ey[k], ez[k], 0.f));
+        team.publish(VEC, ZG, k, il, make_float4(ex[k], ey[k], ez[k], 0.f));
         continue;
       }
       const float4 gr = GR[i];
       const float r0 = -gr.x, r1 = -gr.y, r2 = -gr.z;
       float z0, z1, z2;
       precond(k, r0, r1, r2, z0, z1, z2);
-      team.publish(VEC, ZG, il, i, make_float4(z0, z1, z2, 0.f));
+      team.publish(VEC, ZG, k, il, make_float4(z0, z1, z2, 0.f));
       v[0] += (double)(r0 * z0 + r1 * z1 + r2 * z2);
       v[1] += (double)(r0 * r0 + r1 * r1 + r2 * r2);
     }
     if (warm) {
       // A e (into q) and the scaling alpha
-      team.sync();
+      team.sync(VEC, ZG);
       double a2[2] = {0.0, 0.0};
 #pragma unroll
       for (int k = 0; k < VPT; ++k) {
-        const int il = opaque(tid + k * T), i = lo + il;
+        const int il = opaque(tid + k * T);
         if (il >= own) continue;
         const float4 ei = VEC[il];
         float sx, sy, sz;
@@ -359,7 +450,7 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
         qx[k] = gx[k] * gee + dx[k] * ei.x - l2 * sx;
         qy[k] = gy[k] * gee + dy[k] * ei.y - l2 * sy;
         qz[k] = gz[k] * gee + dz[k] * ei.z - l2 * sz;
-        const float4 gr = GR[i];
+        const float4 gr = GR[team.index(il)];
         a2[0] -= (double)(gr.x * qx[k] + gr.y * qy[k] + gr.z * qz[k]);
         a2[1] += (double)(ex[k] * qx[k] + ey[k] * qy[k] + ez[k] * qz[k]);
       }
@@ -367,21 +458,22 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
       const float al = a2[1] > 0.0 ? (float)(a2[0] / a2[1]) : 0.f;
 #pragma unroll
       for (int k = 0; k < VPT; ++k) {
-        const int il = opaque(tid + k * T), i = lo + il;
+        const int il = opaque(tid + k * T);
         if (il >= own) continue;
         ex[k] *= al; ey[k] *= al; ez[k] *= al;
-        const float4 gr = GR[i];
+        const float4 gr = GR[team.index(il)];
         const float r0 = -gr.x - al * qx[k], r1 = -gr.y - al * qy[k], r2 = -gr.z - al * qz[k];
         qx[k] = qy[k] = qz[k] = 0.f;
         float z0, z1, z2;
         precond(k, r0, r1, r2, z0, z1, z2);
-        team.publish(VEC, ZG, il, i, make_float4(z0, z1, z2, 0.f));
+        team.publish(VEC, ZG, k, il, make_float4(z0, z1, z2, 0.f));
         v[0] += (double)(r0 * z0 + r1 * z1 + r2 * z2);
         v[1] += (double)(r0 * r0 + r1 * r1 + r2 * r2);
         v[2] += (double)(gr.x * gr.x + gr.y * gr.y + gr.z * gr.z);
       }
     }
-    team.template reduce<3, 0>(v, red, sel);   // also publishes z
+    team.template reduce<3, 0>(v, red, sel);
+    team.refresh(VEC, ZG);   // z is published
     double rz = v[0];
     const double rr0 = warm ? v[2] : v[1];     // |b|^2
     if (!(rr0 > 0.0)) return 0;
@@ -393,7 +485,7 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
       double w1[1] = {0.0};
 #pragma unroll
       for (int k = 0; k < VPT; ++k) {
-        const int il = opaque(tid + k * T), i = lo + il;
+        const int il = opaque(tid + k * T);
         if (il >= own) continue;
         const float4 zi = VEC[il];
         float sx, sy, sz;
@@ -413,7 +505,7 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
       double w2[2] = {0.0, 0.0};
 #pragma unroll
       for (int k = 0; k < VPT; ++k) {
-        const int il = opaque(tid + k * T), i = lo + il;
+        const int il = opaque(tid + k * T);
         if (il >= own) continue;
         ex[k] += fa * px[k]; ey[k] += fa * py[k]; ez[k] += fa * pz[k];
         // the residual is not kept: r = M z for the z still published
@@ -425,13 +517,14 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
         const float r2 = gz[k] * gzo + dz[k] * zo.z - fa * qz[k];
         float z0, z1, z2;
         precond(k, r0, r1, r2, z0, z1, z2);
-        team.publish(VEC, ZG, il, i, make_float4(z0, z1, z2, 0.f));
+        team.publish(VEC, ZG, k, il, make_float4(z0, z1, z2, 0.f));
         w2[0] += (double)(r0 * z0 + r1 * z1 + r2 * z2);
         w2[1] += (double)(r0 * r0 + r1 * r1 + r2 * r2);
       }
-      team.template reduce<2, 0>(w2, red, sel);   // also publishes z
+      team.template reduce<2, 0>(w2, red, sel);
       ++it;
       if (w2[1] <= tol2) break;
+      team.refresh(VEC, ZG);   // z is published
       beta = (float)(w2[0] / rz);
       rz = w2[0];
     }
@@ -442,18 +535,19 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
   auto candidate = [&]() -> LMCandidate {
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const int il = opaque(tid + k * T), i = lo + il;
+      const int il = opaque(tid + k * T);
       if (il < own) {
-        const float4 ui = U[i];
-        team.publish(VEC, ZG, il, i, make_float4(ui.x + ex[k], ui.y + ey[k], ui.z + ez[k], 0.f));
+        const float4 ui = U[team.index(il)];
+        team.publish(VEC, ZG, k, il, make_float4(ui.x + ex[k], ui.y + ey[k], ui.z + ez[k], 0.f));
       }
     }
-    team.sync();
+    team.sync(VEC, ZG);
     double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const int il = opaque(tid + k * T), i = lo + il;
+      const int il = opaque(tid + k * T);
       if (il >= own) continue;
+      const int i = team.index(il);
       const float4 x0 = X0[i];
       const float dres = GR[i].w;
       const float gd = gx[k] * ex[k] + gy[k] * ey[k] + gz[k] * ez[k];
@@ -492,10 +586,10 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
     // u <- u + delta: exactly the candidate published to LDS
 #pragma unroll
     for (int k = 0; k < VPT; ++k) {
-      const int il = opaque(tid + k * T), i = lo + il;
+      const int il = opaque(tid + k * T);
       if (il < own) {
         const float4 v = VEC[il];
-        U[i] = make_float4(v.x, v.y, v.z, 0.f);
+        U[team.index(il)] = make_float4(v.x, v.y, v.z, 0.f);
       }
     }
   };
@@ -505,14 +599,19 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
 
 // One workgroup per pair.
 struct LdsSolo {
-  static constexpr bool kPaired = true;
-  int lo, hi;
+  static constexpr bool kPaired = true, kHalo = false, kInOrder = false;
+  int lo, hi, hbase, nhalo;
+  __device__ explicit LdsSolo(int nv) : lo(0), hi(nv), hbase(nv), nhalo(0) {}
   __device__ bool leader() const { return true; }
-  __device__ void sync() { __syncthreads(); }
+  __device__ void give_up() {}
+  __device__ int index(int il) const { return il; }
+  __device__ int rank(int j) const { return j; }
+  __device__ void sync(float4*, const float4*) { __syncthreads(); }
+  __device__ void refresh(float4*, const float4*) {}
   template <int K, int M>
   __device__ void reduce(double (&v)[K + M], double* red, int& sel) { block_reduce_dpp<K, M>(v, red, sel); }
   __device__ float4 neighbour(const float4* VEC, const float4* ZG, unsigned j) const { return VEC[j]; }
-  __device__ void publish(float4* VEC, float4* ZG, int il, int i, float4 v) const { store_xyz(VEC + il, v); }
+  __device__ void publish(float4* VEC, float4* ZG, int k, int il, float4 v) const { store_xyz(VEC + il, v); }
 };
 
 // A team of workgroups per pair (co-resident: cooperative launch).
@@ -521,21 +620,71 @@ struct LdsSolo {
 // reductions are CoherentTeam's, so no barrier writes back or invalidates
 // the L2.
 struct LdsTeam {
-  static constexpr bool kPaired = false;
+  static constexpr bool kPaired = false, kHalo = false;
   CoherentTeam g;
-  int lo, hi;
+  int lo, hi, hbase, nhalo;
+  __device__ LdsTeam(const CoherentTeam& team, int l, int h) : g(team), lo(l), hi(h), hbase(h - l), nhalo(0) {}
   __device__ bool leader() const { return g.leader(); }
-  __device__ void sync() { g.barrier(); }
+  __device__ void give_up() {}
+  __device__ int index(int il) const { return lo + il; }
+  __device__ int rank(int j) const { return j; }
+  __device__ void sync(float4*, const float4*) { g.barrier(); }
+  __device__ void refresh(float4*, const float4*) {}
   template <int K, int M>
   __device__ void reduce(double (&v)[K + M], double* red, int& sel) { g.template reduce_dpp<K, M>(v, red, sel); }
   __device__ float4 neighbour(const float4* VEC, const float4* ZG, unsigned j) const {
     const unsigned jl = j - (unsigned)lo;
     return jl < (unsigned)(hi - lo) ? VEC[jl] : load_coherent(ZG + j);
   }
-  __device__ void publish(float4* VEC, float4* ZG, int il, int i, float4 v) const {
+  __device__ void publish(float4* VEC, float4* ZG, int k, int il, float4 v) const {
     store_xyz(VEC + il, v);
-    store_coherent(ZG + i, v);
+    store_coherent(ZG + lo + il, v);
   }
+};
+
+// A large pair's team: workgroup r owns the ranks [lo, hi) of the pair's
+// vertices in the spatial order that k_chunk_plan made (perm: rank ->
+// vertex, inv: vertex -> rank), which keeps halos short whatever the mesh's
+// numbering.  Records hbase .. hbase + nhalo of VEC are copies of the
+// neighbours owned elsewhere, each with its rank in w; only vertices that
+// have such a neighbour (bit k of `shared` for slot k) are written to ZG,
+// and refresh() copies the halo after the exchange that follows a
+// publication.  A vertex's neighbours are then LDS reads as in LdsSolo:
+// reading ZG in the gather cost a remote round trip per neighbour.
+struct LdsHalo {
+  static constexpr bool kPaired = true, kHalo = true, kInOrder = true;
+  TagTeam g;
+  int lo, hi, hbase, nhalo;
+  unsigned shared;
+  const int* perm;
+  const int* inv;
+  __device__ LdsHalo(const TagTeam& team, int l, int h, const int* p, const int* i)
+      : g(team), lo(l), hi(h), hbase(h - l), nhalo(0), shared(0u), perm(p), inv(i) {}
+  __device__ float4 neighbour(const float4* VEC, const float4* ZG, unsigned j) const { return VEC[j]; }
+  __device__ void publish(float4* VEC, float4* ZG, int k, int il, float4 v) const {
+    store_xyz(VEC + il, v);
+    if (shared >> k & 1u) store_coherent(ZG + lo + il, v);
+  }
+  __device__ void refresh(float4* VEC, const float4* ZG) const {
+    float4* rec = VEC + hbase;
+    for (int h = threadIdx.x; h < nhalo; h += 2 * blockDim.x) {
+      const int h2 = h + blockDim.x;
+      const bool two = h2 < nhalo;
+      const int r1 = reinterpret_cast<const int*>(rec + h)[3];
+      const int r2 = two ? reinterpret_cast<const int*>(rec + h2)[3] : r1;
+      const float4 a = load_coherent(ZG + r1), b = load_coherent(ZG + r2);
+      store_xyz(rec + h, a);
+      if (two) store_xyz(rec + h2, b);
+    }
+    __syncthreads();
+  }
+  __device__ bool leader() const { return g.leader(); }
+  __device__ void give_up() { __hip_atomic_store(g.abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+  __device__ int index(int il) const { return perm[lo + il]; }
+  __device__ int rank(int j) const { return inv[j]; }
+  __device__ void sync(float4* VEC, const float4* ZG) { g.barrier(); refresh(VEC, ZG); }
+  template <int K, int M>
+  __device__ void reduce(double (&v)[K + M], double*, int&) { g.template reduce<K, M>(v); }
 };
 
 // A resident grid of workgroups (as many as the chip holds at once) works
@@ -558,7 +707,7 @@ __global__ void __launch_bounds__(T) k_lm_solve_lds(const LMPairDesc* __restrict
   while (w < count) {
     const int pid = plist[w];
     const LMPairDesc P = pairs[pid];
-    LdsSolo team{0, P.nv};
+    LdsSolo team(P.nv);
     lds_solve<T, VPT, LdsSolo, unsigned short>(P, pid, team, A, opt, res, totalV, smem, red, scan_buf, lds_bytes);
     __syncthreads();   // every thread is done with this pair's LDS
     if (threadIdx.x == 0) s_item = (int)gridDim.x + atomicAdd(next, 1);
@@ -582,9 +731,92 @@ __global__ void __launch_bounds__(T) k_lm_solve_lds_team(const LMPairDesc* __res
   const int pid = plist[m.x];
   const LMPairDesc P = pairs[pid];
   const int lo = min(P.nv, m.y * m.w), hi = min(P.nv, lo + m.w);
-  LdsTeam team{CoherentTeam{m.y, m.z, cnt + (size_t)m.x * 32, part + (size_t)m.x * 2 * kMaxTeam * 8, abort_flag, limit, 0u, 0},
-               lo, hi};
+  LdsTeam team(CoherentTeam{m.y, m.z, cnt + (size_t)m.x * 32, part + (size_t)m.x * 2 * kMaxTeam * 8, abort_flag, limit,
+                            0u, 0},
+               lo, hi);
   lds_solve<T, VPT, LdsTeam, unsigned>(P, pid, team, A, opt, res, totalV, smem, red, scan_buf, lds_bytes);
+}
+
+__device__ inline unsigned long long* pair_slots(const LMArrays& A, long long totalV, long long vbase) {
+  return (unsigned long long*)(A.work + (size_t)gSlots * totalV + vbase);
+}
+
+// Large pairs with their halo in LDS; wg as for k_lm_solve_lds_team.  Bound
+// by the two exchanges and the halo copy of a PCG iteration (about 10 us at
+// three vertices per thread).  Twelve icospheres each of 10242 and 40962
+// vertices, 50 steps of 30 PCG iterations: 55.7 ms on k_lm_solve_lds_team,
+// whose gather waits for a remote read per neighbour, 14.9 ms here.
+template <int T, int VPT>
+__global__ void __launch_bounds__(T) k_lm_solve_lds_halo(const LMPairDesc* __restrict__ pairs,
+                                                         const int* __restrict__ plist, const int4* __restrict__ wg,
+                                                         LMArrays A, LMOptionsDev opt, LMResultDev* __restrict__ res,
+                                                         long long totalV, int* abort_flag, long long limit,
+                                                         unsigned lds_bytes) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  __shared__ double red[kTagRed];
+  __shared__ int scan_buf[kMaxWaves];
+  const int4 m = wg[blockIdx.x];
+  const int pid = plist[m.x];
+  const LMPairDesc P = pairs[pid];
+  const int lo = min(P.nv, m.y * m.w), hi = min(P.nv, lo + m.w);
+  const int* perm = (const int*)(A.work + (size_t)gOrder * totalV + P.vbase);
+  LdsHalo team(TagTeam{m.y, m.z, pair_slots(A, totalV, P.vbase), abort_flag, limit, red, 0u, 0}, lo, hi, perm,
+               perm + P.nv);
+  lds_solve<T, VPT, LdsHalo, unsigned short>(P, pid, team, A, opt, res, totalV, smem, red, scan_buf, lds_bytes);
+}
+
+// Bound on any one wait of a team, in device clock ticks.
+int team_wait_limit(long long* limit) {
+  int dev = 0, khz = 0;
+  MO_HIP(hipGetDevice(&dev));
+  MO_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+  *limit = (long long)std::max(khz, 1) * 1000LL * 20;   // 20 s
+  if (const char* w = getenv("MO_LM_TEAM_WAIT_US")) *limit = atoll(w) * (long long)std::max(khz, 1) / 1000LL;
+  return MO_OK;
+}
+
+bool coop_refused_by_host() {
+  const char* f = getenv("MO_LM_COOP_REFUSE");
+  return f && f[0] == '1';
+}
+
+// kCoopRefused when the runtime refuses the cooperative grid (nothing was
+// launched then).
+int launch_coop(const void* kern, int nwg, int threads, void** args, size_t lds_bytes, hipStream_t s) {
+  if (coop_refused_by_host()) return kCoopRefused;
+  if (hipLaunchCooperativeKernel(kern, dim3(nwg), dim3(threads), args, (unsigned)lds_bytes, s) != hipSuccess) {
+    (void)hipGetLastError();
+    return kCoopRefused;
+  }
+  return MO_OK;
+}
+
+int coop_capacity(const void* kern, int threads, size_t lds_bytes) {
+  int dev = 0, cus = 0, per = 0;
+  if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess ||
+      hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, threads, lds_bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    return 0;
+  }
+  return per * cus;
+}
+
+template <int T, int VPT>
+int launch_halo_bucket(const LMPairDesc* pairs_dev, const int* plist, const int4* wg_dev, int nwg, const LMArrays& A,
+                       const LMOptionsDev& opt, LMResultDev* res, long long totalV, size_t lds_bytes, int* abort_flag,
+                       hipStream_t s) {
+  auto kern = k_lm_solve_lds_halo<T, VPT>;
+  MO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
+  long long limit = 0;
+  if (int rc = team_wait_limit(&limit)) return rc;
+  LMArrays a = A;
+  LMOptionsDev o = opt;
+  unsigned lb = (unsigned)lds_bytes;
+  void* args[] = {(void*)&pairs_dev, (void*)&plist,  (void*)&wg_dev,     (void*)&a,     (void*)&o,
+                  (void*)&res,       (void*)&totalV, (void*)&abort_flag, (void*)&limit, (void*)&lb};
+  return launch_coop((const void*)kern, nwg, T, args, lds_bytes, s);
 }
 
 // Team launch of the register/LDS kernel: nwg workgroups (wg_dev entries)
@@ -595,13 +827,8 @@ int launch_team_bucket(const LMPairDesc* pairs_dev, const int* plist, const int4
                        double* part, int* abort_flag, hipStream_t s) {
   auto kern = k_lm_solve_lds_team<T, VPT>;
   MO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-  int dev = 0, khz = 0;
-  MO_HIP(hipGetDevice(&dev));
-  MO_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
-  long long limit = (long long)std::max(khz, 1) * 1000LL * 20;   // a 20 s bound on any one wait
-  if (const char* w = getenv("MO_LM_TEAM_WAIT_US")) limit = atoll(w) * (long long)std::max(khz, 1) / 1000LL;
-  if (const char* f = getenv("MO_LM_COOP_REFUSE"))
-    if (f[0] == '1') return kCoopRefused;
+  long long limit = 0;
+  if (int rc = team_wait_limit(&limit)) return rc;
   LMArrays a = A;
   LMOptionsDev o = opt;
   long long tv = totalV;
@@ -609,23 +836,11 @@ int launch_team_bucket(const LMPairDesc* pairs_dev, const int* plist, const int4
   void* args[] = {(void*)&pairs_dev, (void*)&plist, (void*)&wg_dev, (void*)&a,           (void*)&o,
                   (void*)&res,       (void*)&tv,    (void*)&cnt,    (void*)&part,        (void*)&abort_flag,
                   (void*)&limit,     (void*)&lb};
-  if (hipLaunchCooperativeKernel((const void*)kern, dim3(nwg), dim3(T), args, (unsigned)lds_bytes, s) != hipSuccess) {
-    (void)hipGetLastError();   // the runtime refused the cooperative grid: nothing was launched
-    return kCoopRefused;
-  }
-  return MO_OK;
+  return launch_coop((const void*)kern, nwg, T, args, lds_bytes, s);
 }
 
-template <int T, int VPT>
-int team_bucket_capacity(size_t lds_bytes) {
-  auto kern = k_lm_solve_lds_team<T, VPT>;
-  int dev = 0, cus = 0, per = 0;
-  if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes) != hipSuccess ||
-      hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)kern, T, lds_bytes) != hipSuccess)
-    return 0;
-  return per * cus;
+__host__ __device__ inline size_t lm_lds_bytes_dev(int nv, long long padded_entries) {
+  return (((size_t)nv * 16 + 16 + (size_t)padded_entries * 2) + 15) & ~(size_t)15;
 }
 
 // Per pair: for each team shape b, the largest chunk's adjacency entries
@@ -678,6 +893,153 @@ __global__ void __launch_bounds__(256) k_chunk_entries(const LMPairDesc* __restr
     out[4 * p + b] = mx;
   }
   if (threadIdx.x == 3) out[4 * p + 3] = padded;
+}
+
+// Chunks of a halo team: 3072 vertices per workgroup, 4096 beyond
+// kMaxTeam of those (0: too large for either).
+__host__ __device__ inline int halo_chunk(int nv, int* chunk) {
+  for (int cap = 3072; cap <= 4096; cap += 1024) {
+    const int c = (nv + cap - 1) / cap;
+    if (c > kMaxTeam) continue;
+    *chunk = (nv + c - 1) / c;
+    return c;
+  }
+  return 0;
+}
+
+// Pairs that can't be solved by one register/LDS workgroup (lds_cap: its
+// LDS) but by a halo team: the vertices' spatial order (work slot gOrder:
+// perm, inv) and minus the team's LDS bytes in out[4 p + 3], which keeps
+// the one-workgroup kernel's entry count otherwise.  The order is that of a
+// 32^3 grid's Morton codes over the mesh's box, ties by index (a stable
+// radix sort).  An icosphere's numbering gives chunks of 2926 vertices up to
+// 16154 neighbours elsewhere (every old vertex's are midpoints far behind
+// it), this order at most 442; of a 41000-vertex box mesh 416 and 358.  One
+// workgroup per pair; runs beside the grid builds.
+constexpr int kPlanThreads = 512;
+static_assert(3072 * 2 >= kTagSlotWords, "a pair's team words fit its work slot");
+__device__ inline unsigned spread3(unsigned x) {   // bits 0..4 to 0, 3, .. 12
+  unsigned r = 0;
+  for (int b = 0; b < 5; ++b) r |= (x >> b & 1u) << (3 * b);
+  return r;
+}
+__global__ void __launch_bounds__(kPlanThreads) k_chunk_plan(const LMPairDesc* __restrict__ pairs, LMArrays A,
+                                                             long long totalV, int lds_cap, int* __restrict__ out) {
+  __shared__ int buf[16 * kPlanThreads];
+  __shared__ int scan_buf[kMaxWaves];
+  __shared__ double red[2 * 8 * kMaxWaves];
+  const int p = blockIdx.x, tid = threadIdx.x;
+  const LMPairDesc P = pairs[p];
+  const int nv = P.nv;
+  int chunk = 0;
+  const int c = halo_chunk(nv, &chunk);
+  const int padded = out[4 * p + 3];
+  if ((P.flags & 1) || c < 2 || (nv <= 8192 && padded < 65536 && lm_lds_bytes_dev(nv, padded) <= (size_t)lds_cap)) return;
+  unsigned long long* slots = pair_slots(A, totalV, P.vbase);   // the team's words start at zero
+  for (int k = tid; k < kTagSlotWords; k += kPlanThreads) slots[k] = 0ull;
+  const float4* X0 = A.x0 + P.vbase;
+  int* perm = (int*)(A.work + (size_t)gOrder * totalV + P.vbase);
+  int* inv = perm + nv;
+  int* code = inv + nv;
+  int* tmp = code + nv;
+  // box, codes
+  double box[6];
+  for (int k = 0; k < 6; ++k) box[k] = -INFINITY;
+  for (int i = tid; i < nv; i += kPlanThreads) {
+    const float4 x = X0[i];
+    box[0] = fmax(box[0], (double)-x.x); box[1] = fmax(box[1], (double)-x.y); box[2] = fmax(box[2], (double)-x.z);
+    box[3] = fmax(box[3], (double)x.x); box[4] = fmax(box[4], (double)x.y); box[5] = fmax(box[5], (double)x.z);
+  }
+  int sel = 0;
+  block_reduce_dpp<0, 6>(box, red, sel);
+  const float ext = (float)fmax(fmax(box[3] + box[0], box[4] + box[1]), box[5] + box[2]);
+  const float sc = ext > 0.f && ext < INFINITY ? 32.f / ext : 0.f;
+  for (int i = tid; i < nv; i += kPlanThreads) {
+    const float4 x = X0[i];
+    const float f[3] = {(x.x + (float)box[0]) * sc, (x.y + (float)box[1]) * sc, (x.z + (float)box[2]) * sc};
+    unsigned m = 0;
+    for (int a = 0; a < 3; ++a) m |= spread3((unsigned)fminf(fmaxf(f[a], 0.f), 31.f)) << a;   // NaN: 0
+    code[i] = (int)m;
+    tmp[i] = i;
+  }
+  __syncthreads();
+  // four passes of a 4-bit radix sort; thread t moves items [t per, (t + 1) per)
+  const int per = (nv + kPlanThreads - 1) / kPlanThreads;
+  const int i0 = min(nv, tid * per), i1 = min(nv, i0 + per);
+  int* src = tmp;
+  int* dst = perm;
+  for (int pass = 0; pass < 4; ++pass) {
+    for (int d = 0; d < 16; ++d) buf[d * kPlanThreads + tid] = 0;
+    // (blocks of 8: the loads of a block are in flight together)
+    for (int i = i0; i < i1; i += 8) {
+      int d[8];
+      for (int q = 0; q < 8; ++q) d[q] = code[src[min(i + q, i1 - 1)]];
+      for (int q = 0; q < 8; ++q)
+        if (i + q < i1) buf[(d[q] >> (4 * pass) & 15) * kPlanThreads + tid]++;
+    }
+    __syncthreads();
+    int sum = 0;
+    for (int q = 0; q < 16; ++q) sum += buf[tid * 16 + q];
+    int total;
+    int at = block_exclusive_scan(sum, scan_buf, total);
+    for (int q = 0; q < 16; ++q) {
+      const int n = buf[tid * 16 + q];
+      buf[tid * 16 + q] = at;
+      at += n;
+    }
+    __syncthreads();
+    for (int i = i0; i < i1; i += 8) {
+      int v[8], d[8];
+      for (int q = 0; q < 8; ++q) v[q] = src[min(i + q, i1 - 1)];
+      for (int q = 0; q < 8; ++q) d[q] = code[v[q]];
+      for (int q = 0; q < 8; ++q)
+        if (i + q < i1) dst[buf[(d[q] >> (4 * pass) & 15) * kPlanThreads + tid]++] = v[q];
+    }
+    __syncthreads();
+    int* t = src;
+    src = dst;
+    dst = t;
+  }
+  // four passes: the order is back in tmp
+  for (int i = tid; i < nv; i += kPlanThreads) {
+    const int v = src[i];
+    perm[i] = v;
+    inv[v] = i;
+  }
+  __syncthreads();
+  // the largest LDS of the chunks: records and entries
+  const int2* ADJ = A.adj + P.vbase;
+  const unsigned* NB = A.nbr + P.ebase;
+  unsigned* bm = (unsigned*)buf;   // nv <= 32 * 16 * kPlanThreads
+  const int nwords = (nv + 31) >> 5;
+  int bytes = 0;
+  bool ok = true;
+  for (int r = 0; r < c; ++r) {
+    const int lo = min(nv, r * chunk), own = min(nv, lo + chunk) - lo;
+    for (int q = tid; q < nwords; q += kPlanThreads) bm[q] = 0u;
+    __syncthreads();
+    int ent = 0;
+    for (int il = tid; il < own; il += kPlanThreads) {
+      const int2 a = ADJ[perm[lo + il]];
+      ent += a.y + (a.y & 1);
+      for (int e = 0; e < a.y; e += 8) {
+        int r8[8];
+        for (int q = 0; q < 8; ++q) r8[q] = inv[nb_index(NB[a.x + min(e + q, a.y - 1)])];
+        for (int q = 0; q < 8; ++q)
+          if ((unsigned)(r8[q] - lo) >= (unsigned)own) atomicOr(&bm[r8[q] >> 5], 1u << (r8[q] & 31));
+      }
+    }
+    __syncthreads();
+    int halo = 0;
+    for (int q = tid; q < nwords; q += kPlanThreads) halo += __popc(bm[q]);
+    int nh, ne;
+    block_exclusive_scan(halo, scan_buf, nh);
+    block_exclusive_scan(ent, scan_buf, ne);
+    const int records = halo_base(own, nv) + nh + 1;
+    ok = ok && records <= 32767 && ne <= 65535;
+    bytes = max(bytes, records * 16 + (ne + 7) / 8 * 16);
+  }
+  if (tid == 0 && ok) out[4 * p + 3] = -bytes;
 }
 
 template <int T, int VPT>
@@ -781,8 +1143,9 @@ int lm_lds_bucket_for(int nv) {
 // workgroup), in preference order: the largest chunk whose LDS fits.
 static const int kTeamT[] = {1024, 1024, 1024};
 static const int kTeamVPT[] = {4, 3, 2};
+constexpr int kHaloShape = 3;   // then the halo teams of 1024x3 and 1024x4
 
-int lm_lds_team_shapes() { return 3; }
+int lm_lds_team_shapes() { return kHaloShape + 2; }
 
 // Preference order of the team shapes: 1024x3, then 1024x4 (only for pairs
 // whose 3072-vertex team would exceed kMaxTeam), then 1024x2 (chunks whose
@@ -814,9 +1177,9 @@ const std::vector<int>& lm_lds_team_order() {
 int lm_lds_team_max() { return kMaxTeam; }
 
 int lm_lds_team_shape(int b, int* threads, int* vpt) {
-  MO_CHECK(b >= 0 && b < 3, MO_ERR_ARG, "team shape %d out of range", b);
-  *threads = kTeamT[b];
-  *vpt = kTeamVPT[b];
+  MO_CHECK(b >= 0 && b < lm_lds_team_shapes(), MO_ERR_ARG, "team shape %d out of range", b);
+  *threads = 1024;
+  *vpt = b < kHaloShape ? kTeamVPT[b] : 3 + (b - kHaloShape);
   return MO_OK;
 }
 
@@ -826,19 +1189,32 @@ size_t lm_lds_team_bytes(int chunk, long long entries) {
 
 int lm_lds_team_capacity(int b, size_t lds_bytes) {
   switch (b) {
-    case 0: return team_bucket_capacity<1024, 4>(lds_bytes);
-    case 1: return team_bucket_capacity<1024, 3>(lds_bytes);
-    case 2: return team_bucket_capacity<1024, 2>(lds_bytes);
+    case 0: return coop_capacity((const void*)k_lm_solve_lds_team<1024, 4>, 1024, lds_bytes);
+    case 1: return coop_capacity((const void*)k_lm_solve_lds_team<1024, 3>, 1024, lds_bytes);
+    case 2: return coop_capacity((const void*)k_lm_solve_lds_team<1024, 2>, 1024, lds_bytes);
+    case kHaloShape: return coop_capacity((const void*)k_lm_solve_lds_halo<1024, 3>, 1024, lds_bytes);
+    case kHaloShape + 1: return coop_capacity((const void*)k_lm_solve_lds_halo<1024, 4>, 1024, lds_bytes);
     default: return 0;
   }
 }
 
-int lm_lds_chunk_entries(const LMPairDesc* pairs_dev, const int2* adj, int np, int* out_dev, hipStream_t s) {
+int lm_lds_chunk_entries(const LMPairDesc* pairs_dev, const LMArrays& A, int np, long long totalV, int max_nv,
+                         size_t lds_cap, int* out_dev, hipStream_t s) {
   if (np <= 0) return MO_OK;
-  hipLaunchKernelGGL(k_chunk_entries, dim3(np), dim3(256), 0, s, pairs_dev, adj, np,
+  hipLaunchKernelGGL(k_chunk_entries, dim3(np), dim3(256), 0, s, pairs_dev, A.adj, np,
                      kTeamT[0] * kTeamVPT[0], kTeamT[1] * kTeamVPT[1], kTeamT[2] * kTeamVPT[2], out_dev);
   MO_HIP(hipGetLastError());
+  // pairs below 3073 vertices are never split
+  if (max_nv > 3072) {
+    hipLaunchKernelGGL(k_chunk_plan, dim3(np), dim3(kPlanThreads), 0, s, pairs_dev, A, totalV, (int)lds_cap, out_dev);
+    MO_HIP(hipGetLastError());
+  }
   return MO_OK;
+}
+
+int lm_lds_halo_shape(int nv, int* chunk, int* workgroups) {
+  *workgroups = halo_chunk(nv, chunk);
+  return *workgroups == 0 ? -1 : *chunk <= 3072 ? kHaloShape : kHaloShape + 1;
 }
 
 int lm_lds_team_launch(int b, const LMPairDesc* pairs, const int* plist, const int4* wg_dev, int nwg,
@@ -852,12 +1228,16 @@ int lm_lds_team_launch(int b, const LMPairDesc* pairs, const int* plist, const i
                                                abort_flag, s);
     case 2: return launch_team_bucket<1024, 2>(pairs, plist, wg_dev, nwg, A, opt, res, totalV, lds_bytes, cnt, part,
                                                abort_flag, s);
+    case kHaloShape: return launch_halo_bucket<1024, 3>(pairs, plist, wg_dev, nwg, A, opt, res, totalV, lds_bytes,
+                                                        abort_flag, s);
+    case kHaloShape + 1: return launch_halo_bucket<1024, 4>(pairs, plist, wg_dev, nwg, A, opt, res, totalV, lds_bytes,
+                                                            abort_flag, s);
     default: return fail(MO_ERR_ARG, "bad register/LDS team shape %d", b);
   }
 }
 
 size_t lm_lds_bytes(int nv, long long padded_entries) {
-  return (((size_t)nv * 16 + 16 + (size_t)padded_entries * 2) + 15) & ~(size_t)15;
+  return lm_lds_bytes_dev(nv, padded_entries);
 }
 
 int lm_lds_launch(int bucket, const LMPairDesc* pairs, const int* plist, int count, int* next, const LMArrays& A,

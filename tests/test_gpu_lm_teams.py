@@ -1,0 +1,66 @@
+"""Large pairs on teams of register/LDS workgroups (k_lm_solve_lds_halo:
+spatial order, neighbours' copies in LDS).  The result must not depend on
+the mesh's numbering (up to the rounding of sums), agrees with the
+one-workgroup kernel on global memory, and a mesh whose halo does not fit
+the LDS is still solved.  Sizes: just above one workgroup's 8192 vertices
+(3 chunks), chunks with one vertex more and less than their neighbours, and
+border edges (multiplicity 1 beside 2).  The oracle's exact-step LM checks
+the same kernel in test_gpu_lm (12000 vertices).
+"""
+import numpy as np
+import pytest
+import torch
+
+from meshode_amd import deform, synth
+
+pytestmark = pytest.mark.gpu
+
+ENERGY_RTOL = 1e-3   # energies of the same steps on different kernels
+
+
+def _pair(n, open_faces=0, seed=3):
+    V, F, tV, tF = synth.box_union_pair(seed, n_boxes=5, n_verts=n // 2 * 2)
+    if n % 2:                       # one vertex in no face
+        V = np.concatenate([V, [[0.31, 0.2, 0.1]]])
+    if open_faces:                  # border edges: multiplicity 1 beside 2
+        F = F[open_faces:]
+    return V, F, tV, tF
+
+
+@pytest.mark.parametrize("mesh", ["ico5", "boxes8194", "boxes12289"])
+def test_halo_team_any_numbering(gpu, mesh):
+    print(f"[lm halo] {mesh}", flush=True)
+    V, F, tV, tF = (synth.displaced_sphere_pair(4, src_level=5, tgt_level=4) if mesh == "ico5"
+                    else _pair(int(mesh[5:]), open_faces=3))
+    perm = np.random.default_rng(1).permutation(len(V))
+    inv = np.argsort(perm)
+    # few steps: later ones of a box pair's non-smooth problem part ways over
+    # the last bits of the FP32 neighbour sums, whichever kernel runs
+    opt = deform.default_options(max_num_iterations=3)
+    out, st = deform.rigid_deform_batch([(V, F, tV, tF), (V[perm], inv[F].astype(np.int32), tV, tF)],
+                                        grid_resolution=32, options=opt)
+    assert all(s["solver_path_name"] == "lds_team" for s in st)
+    assert abs(st[0]["initial_cost"] - st[1]["initial_cost"]) <= 1e-9 * st[0]["initial_cost"]
+    assert abs(st[0]["final_cost"] - st[1]["final_cost"]) <= ENERGY_RTOL * st[0]["final_cost"]
+    # one workgroup on global memory solves the same problem
+    _, one = deform.rigid_deform_batch([(V, F, tV, tF)], grid_resolution=32,
+                                       options=deform.default_options(max_num_iterations=3, kernel_variant=1))
+    assert abs(st[0]["final_cost"] - one[0]["final_cost"]) <= ENERGY_RTOL * one[0]["final_cost"]
+
+
+def test_halo_too_long_for_the_lds(gpu):
+    """Random triangles: nearly every neighbour is in another chunk, so the
+    pair stays on the kernel that reads such neighbours where they are."""
+    print("[lm halo] random triangles", flush=True)
+    rng = np.random.default_rng(5)
+    n = 30000
+    V, _, tV, tF = _pair(1000)
+    V = rng.random((n, 3)) * (V.max(0) - V.min(0)) + V.min(0)
+    F = rng.permutation(np.repeat(np.arange(n, dtype=np.int32), 2)).reshape(-1, 3)
+    F = F[(F[:, 0] != F[:, 1]) & (F[:, 1] != F[:, 2]) & (F[:, 2] != F[:, 0])]
+    opt = dict(max_num_iterations=3)
+    _, st = deform.rigid_deform_batch([(V, F, tV, tF)], grid_resolution=32, options=deform.default_options(**opt))
+    _, one = deform.rigid_deform_batch([(V, F, tV, tF)], grid_resolution=32,
+                                       options=deform.default_options(kernel_variant=1, **opt))
+    assert st[0]["solver_path_name"] == "lds_team"
+    assert abs(st[0]["final_cost"] - one[0]["final_cost"]) <= ENERGY_RTOL * one[0]["final_cost"]
