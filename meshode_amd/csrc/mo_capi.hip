@@ -909,8 +909,8 @@ int lm_core(const std::vector<CorePair>& pairs, const mo_lm_options& opt, mo_lm_
   if ((rc = timer.mark(2))) return rc;
   for (int b = 0; b < nb; ++b)
     if (!bucket[b].empty())
-      if ((rc = lm_lds_launch(b, d_pairs, d_plist + start[b], (int)bucket[b].size(), d_next + b, A, dopt, d_res,
-                              nvalloc, bucket_lds[b], s)))
+      if ((rc = lm_lds_launch(b, d_pairs, d_plist + start[b], (int)bucket[b].size(), (int)pairs[bucket[b][0]].nv,
+                              d_next + b, A, dopt, d_res, nvalloc, bucket_lds[b], s)))
         return rc;
   // Pairs the register/LDS kernel does not take.  A pair of nv vertices
   // gets a team of ceil(nv / team_vertices) co-resident workgroups (at most

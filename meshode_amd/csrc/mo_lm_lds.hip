@@ -288,7 +288,40 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
       // (the entry indices pass through opaque() so each address is one
       // bit-field extract and one shift-add)
       const unsigned* const L2e = L2 + n2;
-      if (uniform_m != 0.f) {
+      // With few vertices per thread nothing else covers the two LDS round
+      // trips of a word, and there are registers for three words at once (a
+      // closed triangle mesh's vertex), entries past the list's end being the
+      // zero vector.  With the launch trimmed to the waves in use: one 642-vertex
+      // pair at 64^3 3.14 -> 3.03 ms.
+      if constexpr (VPT <= 2 && !Team::kInOrder) {
+        const unsigned none = (unsigned)(team.hbase + team.nhalo) * 0x20002u;
+        #pragma unroll 1
+        for (const unsigned* pw = L2; pw < L2e; pw += 3) {
+          unsigned w[3];
+          float4 v[6];
+          w[0] = pw[0];
+          w[1] = pw + 1 < L2e ? pw[1] : none;
+          w[2] = pw + 2 < L2e ? pw[2] : none;
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            v[2 * q] = VEC[__builtin_amdgcn_ubfe(w[q], 1, 15)];
+            v[2 * q + 1] = VEC[__builtin_amdgcn_ubfe(w[q], 17, 15)];
+          }
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            const float4 a = v[2 * q], b = v[2 * q + 1];
+            if (uniform_m != 0.f) {
+              sx += a.x + b.x; sy += a.y + b.y; sz += a.z + b.z;
+            } else {
+              const float ma = (float)((w[q] & 1u) + 1u), mb = (float)(((w[q] >> 16) & 1u) + 1u);
+              sx += ma * a.x + mb * b.x; sy += ma * a.y + mb * b.y; sz += ma * a.z + mb * b.z;
+            }
+          }
+        }
+        if (uniform_m != 0.f) {
+          sx *= uniform_m; sy *= uniform_m; sz *= uniform_m;
+        }
+      } else if (uniform_m != 0.f) {
         #pragma unroll 1
         for (const unsigned* pw = L2; pw < L2e; ++pw) {
           const unsigned w = *pw;
@@ -1043,17 +1076,20 @@ __global__ void __launch_bounds__(kPlanThreads) k_chunk_plan(const LMPairDesc* _
 }
 
 template <int T, int VPT>
-int launch_bucket(const LMPairDesc* pairs, const int* plist, int count, int* next, const LMArrays& A,
+int launch_bucket(const LMPairDesc* pairs, const int* plist, int count, int max_nv, int* next, const LMArrays& A,
                   const LMOptionsDev& opt, LMResultDev* res, long long totalV, size_t lds_bytes, hipStream_t s) {
   auto kern = k_lm_solve_lds<T, VPT>;
+  // one vertex per thread: no more waves than the largest pair needs (idle
+  // ones would still take part in every reduction)
+  const int threads = VPT == 1 ? std::min(T, std::max(64, (max_nv + 63) / 64 * 64)) : T;
   MO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
   // one wave of workgroups: the chip's capacity for this shape and LDS size
   int dev = 0, cus = 0, per = 0;
   MO_HIP(hipGetDevice(&dev));
   MO_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  MO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)kern, T, lds_bytes));
+  MO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)kern, threads, lds_bytes));
   const int nwg = std::max(1, std::min(count, std::max(per, 1) * std::max(cus, 1)));
-  hipLaunchKernelGGL(kern, dim3(nwg), dim3(T), lds_bytes, s, pairs, plist, count, next, A, opt, res, totalV,
+  hipLaunchKernelGGL(kern, dim3(nwg), dim3(threads), lds_bytes, s, pairs, plist, count, next, A, opt, res, totalV,
                      (unsigned)lds_bytes);
   MO_HIP(hipGetLastError());
   return MO_OK;
@@ -1240,12 +1276,12 @@ size_t lm_lds_bytes(int nv, long long padded_entries) {
   return lm_lds_bytes_dev(nv, padded_entries);
 }
 
-int lm_lds_launch(int bucket, const LMPairDesc* pairs, const int* plist, int count, int* next, const LMArrays& A,
+int lm_lds_launch(int bucket, const LMPairDesc* pairs, const int* plist, int count, int max_nv, int* next, const LMArrays& A,
                   const LMOptionsDev& opt, LMResultDev* res, long long totalV, size_t lds_bytes, hipStream_t s) {
   if (count <= 0) return MO_OK;
   switch (bucket) {
 #define MO_SHAPE(ID, T, V) \
-    case ID: return launch_bucket<T, V>(pairs, plist, count, next, A, opt, res, totalV, lds_bytes, s);
+    case ID: return launch_bucket<T, V>(pairs, plist, count, max_nv, next, A, opt, res, totalV, lds_bytes, s);
     MO_SHAPE(0, 1024, 1) MO_SHAPE(1, 1024, 2) MO_SHAPE(2, 1024, 4) MO_SHAPE(3, 1024, 5)
     MO_SHAPE(4, 512, 8) MO_SHAPE(5, 512, 10) MO_SHAPE(6, 512, 12) MO_SHAPE(7, 512, 16)
     MO_SHAPE(8, 256, 20) MO_SHAPE(9, 256, 24) MO_SHAPE(10, 256, 32) MO_SHAPE(11, 768, 6) MO_SHAPE(12, 768, 7)

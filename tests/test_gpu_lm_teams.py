@@ -6,6 +6,9 @@ the LDS is still solved.  Sizes: just above one workgroup's 8192 vertices
 (3 chunks), chunks with one vertex more and less than their neighbours, and
 border edges (multiplicity 1 beside 2).  The oracle's exact-step LM checks
 the same kernel in test_gpu_lm (12000 vertices).
+
+Small pairs: a launch has as many waves as its largest pair needs, so a
+pair's result must not depend on which pairs share the launch.
 """
 import numpy as np
 import pytest
@@ -64,3 +67,16 @@ def test_halo_too_long_for_the_lds(gpu):
                                        options=deform.default_options(kernel_variant=1, **opt))
     assert st[0]["solver_path_name"] == "lds_team"
     assert abs(st[0]["final_cost"] - one[0]["final_cost"]) <= ENERGY_RTOL * one[0]["final_cost"]
+
+
+def test_small_pairs_any_launch_width(gpu):
+    """1 to 16 waves per workgroup and both sides of a wave's 64 vertices;
+    an open mesh (mixed multiplicities, odd lists) among them."""
+    print("[lm small] launch widths", flush=True)
+    pairs = [_pair(n, k % 2 * 5, seed=3 + k) for k, n in enumerate((126, 128, 130, 640, 642, 1022, 1024, 2048))]
+    opt = deform.default_options(max_num_iterations=10)
+    out, st = deform.rigid_deform_batch(pairs, grid_resolution=32, options=opt)
+    for k, p in enumerate(pairs):
+        alone, sa = deform.rigid_deform_batch([p], grid_resolution=32, options=opt)
+        assert torch.equal(alone[0], out[k]), k
+        assert sa[0]["final_cost"] == st[k]["final_cost"] and sa[0]["pcg_iterations"] == st[k]["pcg_iterations"]
