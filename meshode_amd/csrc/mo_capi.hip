@@ -1984,14 +1984,18 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
     L.lds = 0;
     const size_t ent0 = c_ent.size(), halo0 = c_halo.size();
     std::vector<int> seen(n, -1), at(n, 0), record(n, -1);
+    // whole chunks: with c capped at kRotChipTeam some of c chunks of ch
+    // vertices can be empty (65 vertices, team_vertices 1), and the kernel
+    // takes every workgroup to own a vertex
     const int ch = (n + c - 1) / c;
+    c = (n + ch - 1) / ch;
     bool fits = true;
     for (int r = 0; r < c && fits; ++r) {
       RotChunk k{};
       k.pid = p;
       k.rank = r;
       k.size = c;
-      k.lo = std::min(n, r * ch);
+      k.lo = r * ch;
       k.own = std::min(n, k.lo + ch) - k.lo;
       k.ent = (long long)c_ent.size();
       k.halo = (long long)c_halo.size();

@@ -48,7 +48,7 @@ struct RotChunk {
   int pid;             // problem
   int team;            // its slots and, in a launch, its team number
   int rank, size;      // this workgroup in the team
-  int lo, own;         // vertices [lo, lo + own) of the problem
+  int lo, own;         // vertices [lo, lo + own) of the problem, own >= 1
   int nhalo, nent;
   long long halo;      // first halo entry
   long long ent;       // first adjacency entry

@@ -56,6 +56,29 @@ def test_chip_energy_parity(gpu, oracle, name, workgroups):
     assert abs(eg - so["final_cost"]) <= 1e-3 * so["final_cost"]
 
 
+@pytest.mark.parametrize("n,team_vertices,workgroups", [(65, 1, 33), (130, 2, 44), (1000, 15, 63), (1000, 16, 63),
+                                                        (64, 1, 64), (128, 2, 64), (129, 2, 43)])
+def test_no_empty_chunk(gpu, oracle, n, team_vertices, workgroups):
+    """team_vertices asking for more chunks than a team has workgroups: chunks
+    of ceil(n / 64) vertices, and as many as the vertices fill."""
+    print(f"[rot chip] {n} vertices, team_vertices {team_vertices}", flush=True)
+    sV, sF = _fan(n - 1)
+    _, _, tV, tF = synth.displaced_sphere_pair(5, src_level=1, tgt_level=2)
+    pid = deform.template_f64(tV, tF, 16)
+    _, scale, trans = pyDeform.TemplateInfo(pid)
+    grid = pyDeform.TemplateGrid(pid)[0].cpu().numpy().reshape(-1)
+    sn = (sV - trans) / scale
+    V = torch.from_numpy(sn).to(gpu).contiguous()
+    opt = deform.default_options(pcg_relative_tolerance=1e-6, team_vertices=team_vertices)
+    st, W = deform.deform_rot(pid, V, sF, 1.0, options=opt)
+    assert st["workgroups"] == workgroups
+    eg = oracle.lm_rot_cost(grid, 16, V.cpu().numpy(), W.cpu().numpy(), sn, sF, 1.0)[0]
+    assert st["final_cost"] == pytest.approx(eg, rel=1e-3)
+    one = torch.from_numpy(sn).to(gpu).contiguous()
+    s1, _ = deform.deform_rot(pid, one, sF, 1.0)
+    assert st["final_cost"] == pytest.approx(s1["final_cost"], rel=1e-3)
+
+
 def test_hub_beyond_lds(gpu):
     """A hub of 6000 neighbours does not fit a chunk's LDS: one workgroup."""
     print("[rot chip] fan6000", flush=True)
