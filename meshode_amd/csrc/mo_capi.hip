@@ -2048,7 +2048,7 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
     if (!plan[p].chunks.empty()) order.push_back(p);
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return nv[a] > nv[b]; });
   if (!order.empty()) {
-    struct Launch { int threads; size_t lds; bool coop; size_t c0, c1, p0; };
+    struct Launch { int threads; size_t lds; bool coop; size_t c0, c1; };
     std::vector<Launch> launches;
     std::vector<RotChunk> chunks;
     int cap = 0;
@@ -2071,7 +2071,7 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
           rot_wgs[order[q]] = 1;
           continue;
         }
-        launches.push_back(Launch{L.threads, 0, false, chunks.size(), chunks.size(), q});
+        launches.push_back(Launch{L.threads, 0, false, chunks.size(), chunks.size()});
         cur = &launches.back();
       }
       for (RotChunk k : L.chunks) {
@@ -2104,21 +2104,24 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
                            d_chip[kPub].as<unsigned long long>()};
     unsigned long long* slots = d_chip[kSlots].as<unsigned long long>();
     d_abort = (int*)(slots + words);
-    for (size_t k = 0; k < launches.size(); ++k) {
-      const Launch& L = launches[k];
+    int coop = 0;
+    for (const Launch& L : launches) {
       if (L.coop && !team_lock.owns_lock()) team_lock.lock();
       rc = lm_rot_chip_launch(d_pair.as<RotPairDesc>(), d_chip[kChunks].as<RotChunk>() + L.c0, (int)(L.c1 - L.c0), CA,
-                              to_dev_options(o), d_res.as<LMResultDev>(), L.threads, L.lds, L.coop, slots, d_abort, s);
-      if (rc == kCoopRefused && k == 0) {
-        // the runtime refused the cooperative grid before any problem ran:
-        // one workgroup per problem instead
-        solo.resize(npairs);
-        std::iota(solo.begin(), solo.end(), 0);
-        std::fill(path.begin(), path.end(), MO_PATH_COOP_REFUSED);
-        std::fill(rot_wgs.begin(), rot_wgs.end(), 1);
-        break;
+                              to_dev_options(o), d_res.as<LMResultDev>(), L.threads, L.lds, L.coop ? ++coop : 0, slots,
+                              d_abort, s);
+      if (rc == kCoopRefused) {
+        // the runtime refused this cooperative grid, first or later: none of
+        // its problems has run, each goes to one workgroup
+        for (size_t q = L.c0; q < L.c1; ++q)
+          if (chunks[q].rank == 0) {
+            const int p = chunks[q].pid;
+            solo.push_back(p);
+            path[p] = MO_PATH_COOP_REFUSED;
+            rot_wgs[p] = 1;
+          }
+        rc = MO_OK;
       }
-      if (rc == kCoopRefused) return fail(MO_ERR_HIP, "DeformWithRot: cooperative launch refused after %zu chunks", k);
       if (rc) return rc;
     }
   }

@@ -71,12 +71,12 @@ constexpr int kRotPubWords = 5;
 // dynamic LDS of a chunk: records (own and halo), then entries
 size_t lm_rot_chip_lds(int threads, int nhalo, int nent);
 int lm_rot_chip_capacity(int threads, size_t lds_bytes);   // co-resident workgroups, 0: cannot launch
-// slots: kTagSlotWords zeroed 64-bit words per team; cooperative when
-// `coop` (some team has more than one workgroup).  Returns kCoopRefused
-// when the runtime refused the cooperative grid.
+// slots: kTagSlotWords zeroed 64-bit words per team; coop: 0 when every team
+// has one workgroup, else the launch is cooperative, the coop-th such one of
+// the call.  Returns kCoopRefused when the runtime refused the grid.
 int lm_rot_chip_slot_words();
 int lm_rot_chip_launch(const RotPairDesc* pairs_dev, const RotChunk* chunks_dev, int nchunks, const RotChipArrays& a,
-                       const LMOptionsDev& opt, LMResultDev* results_dev, int threads, size_t lds_bytes, bool coop,
+                       const LMOptionsDev& opt, LMResultDev* results_dev, int threads, size_t lds_bytes, int coop,
                        unsigned long long* slots, int* abort_flag, hipStream_t s);
 
 }  // namespace mo

@@ -882,7 +882,7 @@ int lm_rot_chip_capacity(int threads, size_t lds_bytes) {
 }
 
 int lm_rot_chip_launch(const RotPairDesc* pairs_dev, const RotChunk* chunks_dev, int nchunks, const RotChipArrays& a,
-                       const LMOptionsDev& opt, LMResultDev* results_dev, int threads, size_t lds_bytes, bool coop,
+                       const LMOptionsDev& opt, LMResultDev* results_dev, int threads, size_t lds_bytes, int coop,
                        unsigned long long* slots, int* abort_flag, hipStream_t s) {
   if (nchunks <= 0) return MO_OK;
   MO_HIP(hipFuncSetAttribute(chip_kernel(threads), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
@@ -899,11 +899,11 @@ int lm_rot_chip_launch(const RotPairDesc* pairs_dev, const RotChunk* chunks_dev,
     MO_HIP(hipLaunchKernel(chip_kernel(threads), dim3(nchunks), dim3(threads), args, lds_bytes, s));
     return MO_OK;
   }
-  // MO_LM_COOP_REFUSE=1 treats the launch as refused without trying it (the
-  // fallback path's test hook; the runtime refuses cooperative grids while
-  // another process holds the GPU)
+  // MO_LM_COOP_REFUSE=k treats the call's k-th and later cooperative launches
+  // as refused without trying them (the fallback path's test hook; the
+  // runtime refuses cooperative grids while another process holds the GPU)
   if (const char* f = getenv("MO_LM_COOP_REFUSE"))
-    if (f[0] == '1') return kCoopRefused;
+    if (atoi(f) > 0 && coop >= atoi(f)) return kCoopRefused;
   if (hipLaunchCooperativeKernel(chip_kernel(threads), dim3(nchunks), dim3(threads), args, (unsigned)lds_bytes, s) !=
       hipSuccess) {
     (void)hipGetLastError();   // the runtime refused the cooperative grid: nothing was launched

@@ -89,3 +89,38 @@ def test_hub_beyond_lds(gpu):
     opt = deform.default_options(max_num_iterations=2, pcg_max_iterations=20)
     st, _ = deform.deform_rot(pid, V, sF, 1.0, options=opt)
     assert st["workgroups"] == 1 and st["final_cost"] <= st["initial_cost"]
+
+
+def test_refused_after_the_first_launch(gpu, monkeypatch):
+    """A batch that fills the chip twice over takes several cooperative
+    launches.  When the runtime refuses a later one, its problems go to one
+    workgroup each and the earlier ones keep their results.  Each launch is
+    as many problems as are co-resident, so the refused ones are the last of
+    the order of sizes; 1100 problems of 2 workgroups are more than fit on
+    256 CUs at 4 workgroups each."""
+    print("[rot chip] second launch refused", flush=True)
+    sV, sF, tV, tF = _case("boxes258")
+    pid = deform.template_f64(tV, tF, 16)
+    _, scale, trans = pyDeform.TemplateInfo(pid)
+    sn = torch.from_numpy((sV - trans) / scale).to(gpu).contiguous()
+    Fd = torch.from_numpy(sF).to(gpu)
+    opt = deform.default_options(max_num_iterations=2, pcg_max_iterations=10, pcg_relative_tolerance=1e-6)
+    n = 1100
+
+    def solve():
+        Vs = [sn.clone() for _ in range(n)]
+        st, W = deform.deform_rot_batch([pid] * n, Vs, [Fd] * n, [1.0] * n, options=opt)
+        return st, Vs
+
+    want_st, want = solve()
+    assert all(s["solver_path_name"] == "team" for s in want_st)
+    monkeypatch.setenv("MO_LM_COOP_REFUSE", "2")
+    st, got = solve()
+    monkeypatch.delenv("MO_LM_COOP_REFUSE")
+    ran = [s["solver_path_name"] == "team" for s in st]
+    k = sum(ran)
+    assert 0 < k < n and all(ran[:k])
+    assert all(s["solver_path_name"] == "one_workgroup_coop_refused" and s["workgroups"] == 1 for s in st[k:])
+    assert all(torch.equal(a, b) for a, b in zip(got[:k], want[:k]))
+    for s in st[k:]:
+        assert s["final_cost"] == pytest.approx(want_st[0]["final_cost"], rel=1e-3)
