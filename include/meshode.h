@@ -176,7 +176,9 @@ typedef struct mo_lm_options {
                                             workgroup of a pair's team (0: 4 * block_threads);
                                             mo_deform_rot(_batch): largest chunk of a problem per
                                             workgroup, at most 256 (512 above 16384 vertices; 0:
-                                            that) */
+                                            that); > 0 also puts a problem that the on-chip solver
+                                            does not hold on a team of workgroups of that many
+                                            vertices (0: on one workgroup) */
 } mo_lm_options;
 
 typedef struct mo_lm_stats {
@@ -435,10 +437,12 @@ int mo_linear_estimation(double* V, int64_t nv, const int32_t* F, int64_t nf, co
  * solution out.  rot [nv,3] FP64 device array or null: the start rotations
  * (zeros when null, as the reference) in, the final ones out.  F [nf,3]
  * device.  A problem of up to 32768 vertices is solved on chip by one
- * workgroup per chunk of 256 (512 above 16384) vertices; larger ones, hubs
- * whose adjacency exceeds a chunk's LDS and devices that refuse a
- * cooperative grid take one workgroup of opt.block_threads (at most 256)
- * threads.  Synchronizes `stream`. */
+ * workgroup per chunk of 256 (512 above 16384) vertices in the mesh's order.
+ * Larger ones and those with a chunk whose adjacency or neighbours in other
+ * chunks exceed its LDS (hubs, vertices numbered at random) keep their
+ * vectors in global memory: on teams of workgroups of opt.block_threads (at
+ * most 256) threads if opt.team_vertices > 0, else on one, as does what a
+ * refused cooperative grid leaves.  Synchronizes `stream`. */
 int mo_deform_rot(int32_t param_id, double* V, int64_t nv, const int32_t* F, int64_t nf, double lambda,
                   const mo_lm_options* opt, double* rot, mo_lm_stats* stats, void* stream);
 

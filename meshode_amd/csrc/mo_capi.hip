@@ -1935,17 +1935,17 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
   } team_drain{team_lock, s};
   std::vector<int> path(npairs, MO_PATH_ONE_WORKGROUP);
   std::vector<int> rot_wgs(npairs, 1);   // workgroups that solve each problem
-  std::vector<int> solo;                 // problems for the one-workgroup kernel in global memory
+  std::vector<int> solo;                 // problems for the kernels with vectors in global memory
   DevPtr d_chip[9];
   int* d_abort = nullptr;
-  int rc;
+  int rc, coop = 0;                      // coop: cooperative launches tried
 
   // On-chip solver: chunks of at most 256 vertices (512 where 64 of those
   // are not enough; options.team_vertices > 0 asks for smaller ones), one
   // workgroup each.  A problem's chunks depend on the problem alone, so its
   // result is the same in any batch.  A chunk whose records and adjacency
   // do not fit the LDS (a halo or a vertex degree of thousands), or a
-  // problem above 64 x 512 vertices, takes the one-workgroup kernel.
+  // problem above 64 x 512 vertices, takes the kernels in global memory.
   const size_t lds_cap = 150 * 1024;
   std::vector<int2> c_row((size_t)vtot);
   std::vector<unsigned> c_ent;
@@ -2104,7 +2104,6 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
                            d_chip[kPub].as<unsigned long long>()};
     unsigned long long* slots = d_chip[kSlots].as<unsigned long long>();
     d_abort = (int*)(slots + words);
-    int coop = 0;
     for (const Launch& L : launches) {
       if (L.coop && !team_lock.owns_lock()) team_lock.lock();
       rc = lm_rot_chip_launch(d_pair.as<RotPairDesc>(), d_chip[kChunks].as<RotChunk>() + L.c0, (int)(L.c1 - L.c0), CA,
@@ -2125,8 +2124,22 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
       if (rc) return rc;
     }
   }
-  DevPtr d_adj, d_list, d_hab, d_vw, d_hw, d_pair1, d_res1;
+  // What is left runs with its vectors in global memory: with
+  // options.team_vertices > 0 on a team of ceil(nv / team_vertices) workgroups
+  // (at most lm_team_max(), packed largest first into cooperative launches),
+  // else, and where the runtime refuses such a launch, on one workgroup.
+  DevPtr d_adj, d_list, d_hab, d_vw, d_hw, d_pair1, d_res1, d_team;
   if (!solo.empty()) {
+    const int rbt = std::min(o.block_threads, 256);
+    const int rcap = o.team_vertices > 0 ? lm_rot_team_capacity(rbt) : 0;
+    int nteam = 0;   // solo[0, nteam): problems for teams
+    if (rcap >= lm_team_max()) {
+      std::stable_sort(solo.begin(), solo.end(), [&](int a, int b) {
+        const bool ra = path[a] == MO_PATH_COOP_REFUSED, rb = path[b] == MO_PATH_COOP_REFUSED;
+        return ra != rb ? rb : nv[a] > nv[b];
+      });
+      while (nteam < (int)solo.size() && path[solo[nteam]] != MO_PATH_COOP_REFUSED) ++nteam;
+    }
     // half-edges in residual order (face, j) and each vertex's outgoing then
     // incoming half-edges
     std::vector<int2> hab;
@@ -2179,8 +2192,57 @@ MO_EXPORT int mo_deform_rot_batch(int32_t npairs, const int32_t* param_ids, doub
     MO_HIP(hipStreamSynchronize(s));   // host vectors above go out of scope
     RotArrays A{d_x0.as<float4>(), d_u.as<float4>(), d_w.as<float4>(), d_adj.as<int4>(), d_list.as<int>(),
                 d_hab.as<int2>(), d_vw.as<float4>(), d_hw.as<float4>()};
-    rc = lm_rot_launch(d_pair1.as<RotPairDesc>(), (int)spd.size(), A, to_dev_options(o), d_res1.as<LMResultDev>(), vtot,
-                       hslots, std::min(o.block_threads, 256), s);
+    int done = 0;    // solo[0, done) launched
+    if (nteam) {
+      std::vector<int> order(nteam), tc(nteam);
+      std::iota(order.begin(), order.end(), 0);
+      std::vector<int4> wg;
+      std::vector<int> pack_team{0}, pack_wg{0};
+      int used = 0;
+      for (int t = 0; t < nteam; ++t) {
+        tc[t] = (int)std::min<long long>((nv[solo[t]] + o.team_vertices - 1) / o.team_vertices, lm_team_max());
+        if (used + tc[t] > rcap) {
+          pack_team.push_back(t);
+          pack_wg.push_back((int)wg.size());
+          used = 0;
+        }
+        for (int r = 0; r < tc[t]; ++r) wg.push_back(make_int4(t - pack_team.back(), r, tc[t], 0));
+        used += tc[t];
+      }
+      pack_team.push_back(nteam);
+      pack_wg.push_back((int)wg.size());
+      const int per = lm_team_part_doubles();
+      const size_t b_tp = al(nteam * sizeof(int)), b_wg = al(wg.size() * sizeof(int4)),
+                   b_cnt = al(((size_t)nteam * 32 + 1) * sizeof(unsigned)), b_part = al((size_t)nteam * per * 8);
+      if (int e_ = d_team.alloc(b_tp + b_wg + b_cnt + b_part)) return e_;
+      char* base = d_team.as<char>();
+      int* d_tp = (int*)base;
+      int4* d_wg = (int4*)(base + b_tp);
+      unsigned* d_cnt = (unsigned*)(base + b_tp + b_wg);
+      double* d_part = (double*)(base + b_tp + b_wg + b_cnt);
+      if (!d_abort) d_abort = (int*)(d_cnt + (size_t)nteam * 32);
+      if ((rc = zero_fill(d_cnt, ((size_t)nteam * 32 + 1) * sizeof(unsigned), s))) return rc;
+      MO_HIP(hipMemcpyAsync(d_tp, order.data(), nteam * sizeof(int), hipMemcpyHostToDevice, s));
+      MO_HIP(hipMemcpyAsync(d_wg, wg.data(), wg.size() * sizeof(int4), hipMemcpyHostToDevice, s));
+      MO_HIP(hipStreamSynchronize(s));   // host vectors above go out of scope
+      if (!team_lock.owns_lock()) team_lock.lock();
+      for (size_t k = 0; k + 1 < pack_team.size(); ++k) {
+        const int t0 = pack_team[k], t1 = pack_team[k + 1];
+        rc = lm_rot_team_launch(d_pair1.as<RotPairDesc>(), d_tp + t0, d_wg + pack_wg[k], pack_wg[k + 1] - pack_wg[k],
+                                A, to_dev_options(o), d_res1.as<LMResultDev>(), vtot, hslots, rbt, ++coop,
+                                d_cnt + (size_t)t0 * 32, d_part + (size_t)t0 * per, d_abort, s);
+        if (rc == kCoopRefused) break;   // this pack and the rest: one workgroup each
+        if (rc) return rc;
+        for (int t = t0; t < t1; ++t) {
+          path[solo[t]] = MO_PATH_TEAM;
+          rot_wgs[solo[t]] = tc[t];
+        }
+        done = t1;
+      }
+      for (int t = done; t < nteam; ++t) path[solo[t]] = MO_PATH_COOP_REFUSED;
+    }
+    rc = lm_rot_launch(d_pair1.as<RotPairDesc>() + done, (int)solo.size() - done, A, to_dev_options(o),
+                       d_res1.as<LMResultDev>() + done, vtot, hslots, rbt, s);
     if (rc) return rc;
     for (size_t q = 0; q < solo.size(); ++q)
       MO_HIP(hipMemcpyAsync(d_res.as<LMResultDev>() + solo[q], d_res1.as<LMResultDev>() + q, sizeof(LMResultDev),

@@ -36,6 +36,16 @@ int lm_rot_launch(const RotPairDesc* pairs_dev, int npairs, const RotArrays& arr
                   LMResultDev* results_dev, long long total_vertices, long long total_half_edges, int block_threads,
                   hipStream_t s);
 
+// Multi-workgroup variant (k_lm_rot_team), laid out as lm_team_launch
+// (mo_lm.h): wg_dev entries (team, rank, size, -), team t solves problem
+// plist[t]; cnt / part / abort_flag as there; coop as for
+// lm_rot_chip_launch.
+int lm_rot_team_capacity(int block_threads);
+int lm_rot_team_launch(const RotPairDesc* pairs_dev, const int* plist, const int4* wg_dev, int nwg,
+                       const RotArrays& arrays, const LMOptionsDev& opt, LMResultDev* results_dev,
+                       long long total_vertices, long long total_half_edges, int block_threads, int coop,
+                       unsigned* cnt, double* part, int* abort_flag, hipStream_t s);
+
 // On-chip solver (k_lm_rot_chip): a problem's vertices are split into chunks
 // of at most kRotChip, one workgroup per chunk with one vertex per thread;
 // the workgroups of a problem (at most kRotChipTeam) are its team.  A chunk

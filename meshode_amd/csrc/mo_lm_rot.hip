@@ -2,8 +2,8 @@
 // on gfx950: the whole trust-region loop in one persistent kernel (the loop
 // of mo_lm_util.h), on chip on one workgroup per 256-vertex chunk of the
 // problem (k_lm_rot_chip below), or, for problems that kernel does not hold
-// and where the runtime refuses a cooperative grid, on one workgroup with
-// its vectors in global memory (k_lm_rot).
+// and where the runtime refuses a cooperative grid, with its vectors in
+// global memory, on one workgroup (k_lm_rot) or on a team (k_lm_rot_team).
 //
 // Unknowns per vertex i: the position p_i = x0_i + u_i and an angle-axis
 // rotation w_i (zero at the start, deformer.cc:114).  Residuals:
@@ -457,6 +457,23 @@ __global__ void __launch_bounds__(256) k_lm_rot(const RotPairDesc* __restrict__ 
   lm_rot_pair(pairs[pid], res + pid, A, opt, totalV, totalH, team, red);
 }
 
+// The same on a team of workgroups, for problems the on-chip solver below
+// does not hold when the caller asks for teams (options.team_vertices).
+// 33024 vertices, 5 steps of 40 PCG iterations: 343 ms on one workgroup of
+// 256 threads, 18.2 on 32 of them (46.4 on 32 of 64 threads, 1131 on one).
+// wg[b] = (team, rank, team size, -): team t solves problem plist[t].
+__global__ void __launch_bounds__(256) k_lm_rot_team(const RotPairDesc* __restrict__ pairs,
+                                                      const int* __restrict__ plist, const int4* __restrict__ wg,
+                                                      RotArrays A, LMOptionsDev opt, LMResultDev* __restrict__ res,
+                                                      long long totalV, long long totalH, unsigned* cnt, double* part,
+                                                      int* abort_flag, long long limit) {
+  __shared__ double red[2 * 8 * kMaxWaves];
+  const int4 m = wg[blockIdx.x];
+  const int pid = plist[m.x];
+  GridTeam team{m.y, m.z, cnt + (size_t)m.x * 32, part + (size_t)m.x * 2 * kMaxTeam * 8, abort_flag, limit, 0u, 0};
+  lm_rot_pair(pairs[pid], res + pid, A, opt, totalV, totalH, team, red);
+}
+
 // ---------------------------------------------------------------------------
 // The on-chip solver.  With R = A_a (a rotation: A^T A = I) and J = the right
 // Jacobian of the exponential map at w_a, dq/dw x = R ((J x) x e), so for a
@@ -858,6 +875,57 @@ int lm_rot_launch(const RotPairDesc* pairs_dev, int npairs, const RotArrays& arr
   return MO_OK;
 }
 
+// Bound on any one wait of a team, in device clock ticks.
+static int team_wait_limit(long long* limit) {
+  int dev = 0, khz = 0;
+  MO_HIP(hipGetDevice(&dev));
+  MO_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
+  *limit = (long long)std::max(khz, 1) * 1000LL * 20;   // 20 s
+  if (const char* w = getenv("MO_LM_TEAM_WAIT_US")) *limit = atoll(w) * (long long)std::max(khz, 1) / 1000LL;
+  return MO_OK;
+}
+
+// MO_LM_COOP_REFUSE=k treats the call's k-th and later cooperative launches
+// as refused without trying them (the fallback path's test hook; the
+// runtime refuses cooperative grids while another process holds the GPU)
+static bool refused_by_host(int coop) {
+  const char* f = getenv("MO_LM_COOP_REFUSE");
+  return f && atoi(f) > 0 && coop >= atoi(f);
+}
+
+int lm_rot_team_capacity(int block_threads) {
+  int dev = 0, cus = 0, per = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)k_lm_rot_team, block_threads, 0) != hipSuccess)
+    return 0;
+  return per * cus;
+}
+
+int lm_rot_team_launch(const RotPairDesc* pairs_dev, const int* plist, const int4* wg_dev, int nwg,
+                       const RotArrays& arrays, const LMOptionsDev& opt, LMResultDev* results_dev,
+                       long long total_vertices, long long total_half_edges, int block_threads, int coop,
+                       unsigned* cnt, double* part, int* abort_flag, hipStream_t s) {
+  if (nwg <= 0) return MO_OK;
+  MO_CHECK(block_threads >= 64 && block_threads <= 256 && block_threads % 64 == 0, MO_ERR_ARG,
+           "block_threads must be a multiple of 64 in [64, 256] (got %d)", block_threads);
+  long long limit = 0;
+  if (int rc = team_wait_limit(&limit)) return rc;
+  RotArrays a = arrays;
+  LMOptionsDev o = opt;
+  LMResultDev* r = results_dev;
+  long long tv = total_vertices, th = total_half_edges;
+  void* args[] = {(void*)&pairs_dev, (void*)&plist, (void*)&wg_dev, (void*)&a, (void*)&o, (void*)&r, (void*)&tv,
+                  (void*)&th, (void*)&cnt, (void*)&part, (void*)&abort_flag, (void*)&limit};
+  if (refused_by_host(coop)) return kCoopRefused;
+  if (hipLaunchCooperativeKernel((const void*)k_lm_rot_team, dim3(nwg), dim3(block_threads), args, 0, s) !=
+      hipSuccess) {
+    (void)hipGetLastError();   // the runtime refused the cooperative grid: nothing was launched
+    return kCoopRefused;
+  }
+  return MO_OK;
+}
+
 size_t lm_rot_chip_lds(int threads, int nhalo, int nent) {
   return 48 * ((size_t)threads + (size_t)nhalo) + 16 * (size_t)nent;
 }
@@ -886,11 +954,8 @@ int lm_rot_chip_launch(const RotPairDesc* pairs_dev, const RotChunk* chunks_dev,
                        unsigned long long* slots, int* abort_flag, hipStream_t s) {
   if (nchunks <= 0) return MO_OK;
   MO_HIP(hipFuncSetAttribute(chip_kernel(threads), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-  int dev = 0, khz = 0;
-  MO_HIP(hipGetDevice(&dev));
-  MO_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev));
-  long long limit = (long long)std::max(khz, 1) * 1000LL * 20;   // a 20 s bound on any one wait
-  if (const char* w = getenv("MO_LM_TEAM_WAIT_US")) limit = atoll(w) * (long long)std::max(khz, 1) / 1000LL;
+  long long limit = 0;
+  if (int rc = team_wait_limit(&limit)) return rc;
   RotChipArrays arr = a;
   LMOptionsDev o = opt;
   void* args[] = {(void*)&pairs_dev, (void*)&chunks_dev, (void*)&arr,        (void*)&o,
@@ -899,11 +964,7 @@ int lm_rot_chip_launch(const RotPairDesc* pairs_dev, const RotChunk* chunks_dev,
     MO_HIP(hipLaunchKernel(chip_kernel(threads), dim3(nchunks), dim3(threads), args, lds_bytes, s));
     return MO_OK;
   }
-  // MO_LM_COOP_REFUSE=k treats the call's k-th and later cooperative launches
-  // as refused without trying them (the fallback path's test hook; the
-  // runtime refuses cooperative grids while another process holds the GPU)
-  if (const char* f = getenv("MO_LM_COOP_REFUSE"))
-    if (atoi(f) > 0 && coop >= atoi(f)) return kCoopRefused;
+  if (refused_by_host(coop)) return kCoopRefused;
   if (hipLaunchCooperativeKernel(chip_kernel(threads), dim3(nchunks), dim3(threads), args, (unsigned)lds_bytes, s) !=
       hipSuccess) {
     (void)hipGetLastError();   // the runtime refused the cooperative grid: nothing was launched

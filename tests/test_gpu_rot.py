@@ -163,7 +163,7 @@ def test_rigid_rot_deform_cli(gpu, oracle, tmp_path):
     pid = deform.template_f64(tV2, tF2, N)
     _, scale, trans = pyDeform.TemplateInfo(pid)
     V = torch.from_numpy((sV2 - trans) / scale).to(gpu).contiguous()
-    # the CLI solves its one problem on a team (64-thread workgroups, 512 vertices each)
+    # the CLI's options: what the on-chip solver does not hold goes to 64-thread workgroups, 512 vertices each
     st, _ = deform.deform_rot(pid, V, sF2, 1.0,
                               options=deform.default_options(pcg_relative_tolerance=1e-6, block_threads=64,
                                                              team_vertices=512))

@@ -123,4 +123,74 @@ def test_refused_after_the_first_launch(gpu, monkeypatch):
     assert all(s["solver_path_name"] == "one_workgroup_coop_refused" and s["workgroups"] == 1 for s in st[k:])
     assert all(torch.equal(a, b) for a, b in zip(got[:k], want[:k]))
     for s in st[k:]:
-        assert s["final_cost"] == pytest.approx(want_st[0]["final_cost"], rel=1e-3)
+        assert s["final_cost"] == pytest.approx(want_st[0]["final_cost"], rel=1e-6)
+
+
+TEAM = dict(pcg_relative_tolerance=1e-6, team_vertices=16, block_threads=64)
+
+
+@pytest.mark.parametrize("name", ["boxes254", "boxes600", "repeated", "fan300"])
+def test_one_workgroup_energy_parity(gpu, oracle, monkeypatch, name):
+    """The kernel a refused cooperative launch leaves its problems to."""
+    print(f"[rot one workgroup] {name}", flush=True)
+    sV, sF, tV, tF = _case(name)
+    pid = deform.template_f64(tV, tF, 16)
+    _, scale, trans = pyDeform.TemplateInfo(pid)
+    grid = pyDeform.TemplateGrid(pid)[0].cpu().numpy().reshape(-1)
+    sn = (sV - trans) / scale
+    V = torch.from_numpy(sn).to(gpu).contiguous()
+    monkeypatch.setenv("MO_LM_COOP_REFUSE", "1")
+    st, W = deform.deform_rot(pid, V, sF, 1.0, options=deform.default_options(**TEAM))
+    monkeypatch.delenv("MO_LM_COOP_REFUSE")
+    assert st["solver_path_name"] == "one_workgroup_coop_refused" and st["workgroups"] == 1
+    _, _, so = oracle.lm_rot_solve(grid, 16, sn, sF, 1.0)
+    eg = oracle.lm_rot_cost(grid, 16, V.cpu().numpy(), W.cpu().numpy(), sn, sF, 1.0)[0]
+    assert st["initial_cost"] == pytest.approx(so["initial_cost"], rel=1e-4)
+    assert abs(eg - so["final_cost"]) <= 1e-3 * so["final_cost"]
+
+
+def _sheet(a, b, shuffle=False):
+    """A wavy sheet of a x b vertices, numbered by rows or at random."""
+    i, j = np.meshgrid(np.arange(a), np.arange(b), indexing="ij")
+    V = np.stack([0.1 + 0.8 * i / a, 0.1 + 0.8 * j / b, 0.5 + 0.1 * np.sin(9.0 * i / a + 5.0 * j / b)], -1).reshape(-1, 3)
+    k = (i * b + j)[:-1, :-1].reshape(-1)
+    F = np.concatenate([np.stack([k, k + b, k + 1], 1), np.stack([k + 1, k + b, k + b + 1], 1)]).astype(np.int32)
+    if shuffle:
+        perm = np.random.default_rng(2).permutation(len(V))
+        V, F = V[perm], np.argsort(perm)[F].astype(np.int32)
+    return V, F
+
+
+@pytest.mark.parametrize("name,team_vertices,workgroups,solver", [
+    ("rows16500", 0, 33, "team"),                 # 512 vertices per workgroup, on chip
+    ("rows33024", 0, 1, "one_workgroup"),         # more than 64 workgroups of 512
+    ("rows33024", 2048, 17, "team"),              # the same on a team in global memory
+    ("random16900", 0, 1, "one_workgroup"),       # neighbours everywhere: no chunk fits
+    ("random16900", 512, 32, "team"),             # (34 workgroups asked for, 32 given)
+    ("fan6000", 512, 12, "team"),
+])
+def test_large_problems(gpu, monkeypatch, name, team_vertices, workgroups, solver):
+    """A few steps on every kernel a large problem can take, against the same
+    steps on one workgroup in global memory."""
+    print(f"[rot large] {name} team_vertices={team_vertices}", flush=True)
+    sV, sF = {"rows16500": lambda: _sheet(165, 100), "rows33024": lambda: _sheet(258, 128),
+              "random16900": lambda: _sheet(130, 130, True), "fan6000": lambda: _fan(6000)}[name]()
+    _, _, tV, tF = synth.displaced_sphere_pair(5, src_level=1, tgt_level=2)
+    pid = deform.template_f64(tV, tF, 16)
+    _, scale, trans = pyDeform.TemplateInfo(pid)
+    lo, hi = tV.min(0), tV.max(0)
+    sn = torch.from_numpy((lo + (hi - lo) * sV - trans) / scale).to(gpu).contiguous()
+    steps = dict(max_num_iterations=2, pcg_max_iterations=15, pcg_relative_tolerance=1e-6, block_threads=256)
+    V = sn.clone()
+    st, _ = deform.deform_rot(pid, V, sF, 1.0, options=deform.default_options(team_vertices=team_vertices, **steps))
+    assert st["workgroups"] == workgroups and st["solver_path_name"] == solver
+    one = sn.clone()
+    monkeypatch.setenv("MO_LM_COOP_REFUSE", "1")
+    ref, _ = deform.deform_rot(pid, one, sF, 1.0, options=deform.default_options(team_vertices=256, **steps))
+    monkeypatch.delenv("MO_LM_COOP_REFUSE")
+    assert ref["solver_path_name"] == "one_workgroup_coop_refused"
+    print(f"[rot large]   {st['final_cost']:.9e} / {ref['final_cost']:.9e} ({st['pcg_iterations']} pcg)", flush=True)
+    assert st["initial_cost"] == pytest.approx(ref["initial_cost"], rel=1e-6)
+    assert st["final_cost"] == pytest.approx(ref["final_cost"], rel=1e-6)
+    assert st["final_cost"] < st["initial_cost"]
+    assert st["iterations"] == ref["iterations"] and st["pcg_iterations"] == ref["pcg_iterations"]
