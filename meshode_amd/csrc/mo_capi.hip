@@ -1229,6 +1229,7 @@ MO_EXPORT int mo_template_grid(int32_t param_id, double* dist64, float* dist32, 
 MO_EXPORT int mo_grid_build(const double* Vn, int64_t nv, const int32_t* F, int64_t nf, int32_t grid_resolution,
                             double* dist64, float* dist32, int32_t* nearest, void* stream) {
   MO_CHECK(Vn && F && nv > 0 && nf > 0, MO_ERR_ARG, "grid build needs vertices and faces");
+  if (int e_ = grid_check_resolution(grid_resolution)) return e_;
   hipStream_t s = as_stream(stream);
   GridSpec gs{Vn, nv, F, nf, grid_resolution, dist64, dist32, nearest};
   const size_t gws = grid_batch_workspace_bytes(&gs, 1);

@@ -86,6 +86,8 @@ struct GridJob {
   unsigned long long* stats;
 };
 
+// (the workspace grows with N^3: the resolutions are checked before it is sized)
+int grid_check_resolution(int N);
 size_t grid_batch_workspace_bytes(const GridSpec* specs, int n);
 
 // Builds every grid of the batch with one launch per stage.  err_dev: device

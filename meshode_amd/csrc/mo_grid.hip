@@ -836,6 +836,11 @@ static long long brick_total(long long N) {
 }
 static size_t queue_bytes(long long bricks) { return al256(sizeof(GridQueue) + (size_t)bricks * sizeof(int2)); }
 
+int grid_check_resolution(int N) {
+  MO_CHECK(N >= 2 && N <= 2048, MO_ERR_ARG, "grid resolution %d out of range [2, 2048]", N);
+  return MO_OK;
+}
+
 int grid_build_batch_launch(const GridSpec* specs, int n, void* workspace, hipStream_t stream, int* err_dev,
                             hipEvent_t build_after) {
   if (n <= 0) return MO_OK;
@@ -844,13 +849,15 @@ int grid_build_batch_launch(const GridSpec* specs, int n, void* workspace, hipSt
   GridJob* d_jobs = (GridJob*)w;
   w += al256((size_t)n * sizeof(GridJob));
   long long bricks = 0;
-  for (int q = 0; q < n; ++q) bricks += brick_total(specs[q].N);
+  for (int q = 0; q < n; ++q) {
+    if (int rc = grid_check_resolution(specs[q].N)) return rc;
+    bricks += brick_total(specs[q].N);
+  }
   GridQueue* queue = (GridQueue*)w;
   w += queue_bytes(bricks);
   long long max_nf = 0, max_tiles = 0, max_bricks = 0;
   for (int q = 0; q < n; ++q) {
     const GridSpec& sp = specs[q];
-    MO_CHECK(sp.N >= 2 && sp.N <= 2048, MO_ERR_ARG, "grid resolution %d out of range [2, 2048]", sp.N);
     MO_CHECK(sp.nf >= 1, MO_ERR_ARG, "distance field needs at least one triangle (got %lld)", sp.nf);
     GridJob& J = jobs[q];
     J.V = sp.Vn; J.F = sp.F; J.nv = sp.nv; J.nf = sp.nf; J.N = sp.N;
