@@ -224,14 +224,18 @@ __global__ void __launch_bounds__(256, 8) k_face_prep(const GridJob* __restrict_
   q.nx = q.ny = q.nz = q.c = q.e = q.pad = 0.f;
   // FP32 error of n . q - c for |q_i| <= 1: 3 products and sums of terms
   // below 3 + |c|, their operands rounded to 2^-24: under 1e-6 (1 + |c|).
-  // n itself is good to 1e-10 where the triangle's sine exceeds 1e-6.
+  // n itself is good to 1e-9 where the triangle's sine exceeds 1e-6, and c
+  // sums terms as large as the coordinates m: 1e-9 m more, which counts
+  // where a face's vertices lie far from the box that its plane crosses.
   if (nn > 1e-12 * g.d00 * g.d11) {
     const double inv = 1.0 / sqrt(nn);
     const double ux = g.nx * inv, uy = g.ny * inv, uz = g.nz * inv;
     const double c = ux * g.ax + uy * g.ay + uz * g.az;
     q.nx = (float)ux; q.ny = (float)uy; q.nz = (float)uz;
     q.c = (float)c;
-    q.e = (float)(1e-6 * (1.0 + (c < 0.0 ? -c : c)));
+    const double m = dmax(dmax(dmax(-(double)q.lox, (double)q.hix), dmax(-(double)q.loy, (double)q.hiy)),
+                          dmax(-(double)q.loz, (double)q.hiz));
+    q.e = (float)(1e-6 * (1.0 + (c < 0.0 ? -c : c)) + 1e-9 * m);
   }
   J.cull[pos] = q;
   }
