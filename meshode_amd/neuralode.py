@@ -109,25 +109,29 @@ class RK4Adjoint(Function):
 
     @staticmethod
     def forward(ctx, y0, steps, func, *params):
+        return RK4Adjoint._integrate(ctx, y0, steps, func, any(ctx.needs_input_grad))
+
+    @staticmethod
+    def _integrate(ctx, y0, steps, func, keep):
+        """y1; keep: what backward needs stays in ctx."""
         h = 1.0 / steps
         y = y0.detach()
+        saved = []
         with torch.no_grad():
             packed = flow256_pack(func) if _fused_field(func, y) else None
             if packed is not None:
                 # the fused adjoint starts from the stage inputs: 48 B a point and step
-                keep = any(ctx.needs_input_grad)
-                saved = [torch.empty((steps, 4) + tuple(y.shape), dtype=torch.float32, device=y.device)] if keep else []
+                if keep:
+                    saved = [torch.empty((steps, 4) + tuple(y.shape), dtype=torch.float32, device=y.device)]
                 for k in range(steps):
                     y = flow256_step(packed, y, h, saved[0][k] if keep else None)
             else:
-                saved = [y]
                 for _ in range(steps):
+                    if keep:
+                        saved.append(y)
                     y = rk4_step(func, y, h)
-                    saved.append(y)
-                saved.pop()
         ctx.func, ctx.steps, ctx.h, ctx.packed = func, steps, h, packed
         ctx.save_for_backward(*saved)
-        ctx.n_params = len(params)
         return y
 
     @staticmethod
@@ -176,9 +180,20 @@ class RK4Adjoint(Function):
         return (gy, None, None, *gp)
 
 
+class _RK4Inference(RK4Adjoint):
+    """RK4Adjoint where no gradient can be asked for.  (needs_input_grad says
+    which inputs require one whatever the grad mode, and inside a Function's
+    forward the mode is always off.)"""
+
+    @staticmethod
+    def forward(ctx, y0, steps, func, *params):
+        return RK4Adjoint._integrate(ctx, y0, steps, func, False)
+
+
 def odeint_rk4(func: nn.Module, y0, steps=16):
     """Integrate dy/dt = func(y) over [0, 1] with ``steps`` RK4 steps."""
-    return RK4Adjoint.apply(y0, steps, func, *func.parameters())
+    f = RK4Adjoint if torch.is_grad_enabled() else _RK4Inference
+    return f.apply(y0, steps, func, *func.parameters())
 
 
 class _DistanceLoss(Function):

@@ -91,6 +91,36 @@ def test_adjoint_central_differences():
         assert g[i, j].item() == pytest.approx((lp - lm) / (2 * eps), rel=1e-6, abs=1e-10)
 
 
+@pytest.mark.parametrize("mode", ["grad", "no_grad", "inference", "frozen"])
+def test_stage_inputs_are_kept_for_a_backward_only(monkeypatch, mode):
+    """The fused step's stage inputs (48 B a point and step) are asked for
+    when a gradient can be: not under no_grad or inference_mode, whose
+    parameters still require one, and not for frozen parameters."""
+    m = NO.VelocityMLP(hidden=8, seed=3, dtype=torch.float64)
+    y0 = torch.rand(5, 3, dtype=torch.float64)
+    want = y0
+    with torch.no_grad():
+        for _ in range(3):
+            want = NO.rk4_step(m, want, 1.0 / 3)
+    asked = []
+
+    def step(packed, y, h, stages=None):
+        asked.append(stages is not None)
+        return NO.rk4_step(m, y, h)
+
+    monkeypatch.setattr(NO, "_fused_field", lambda func, y: True)
+    monkeypatch.setattr(NO, "flow256_pack", lambda func: "packed")
+    monkeypatch.setattr(NO, "flow256_step", step)
+    if mode == "frozen":
+        m.requires_grad_(False)
+    off = {"no_grad": torch.no_grad, "inference": torch.inference_mode}.get(mode, torch.enable_grad)
+    with off():
+        y = NO.odeint_rk4(m, y0, steps=3)
+    assert torch.equal(y, want)
+    assert asked == [mode == "grad"] * 3
+    assert y.requires_grad == (mode == "grad")
+
+
 @pytest.mark.gpu
 def test_gpu_flow_and_loss_against_fp64(gpu, oracle):
     from meshode_amd import pyDeform, synth
