@@ -761,7 +761,7 @@ using namespace mo;
 
 MO_EXPORT int mo_flow256_step_stages(const float* y0, int64_t n, const float* packed, float h, float* y1, float* Zs,
                                      void* stream) {
-  MO_CHECK(packed && n >= 0 && n <= (1LL << 30) / 12 && (n == 0 || (y0 && y1)), MO_ERR_ARG,
+  MO_CHECK(packed && n >= 0 && n <= (1LL << 30) && (n == 0 || (y0 && y1)), MO_ERR_ARG,
            "mo_flow256_step_stages: bad arguments");
   MO_CHECK(((uintptr_t)packed & 15) == 0, MO_ERR_ARG, "mo_flow256_step_stages: packed not 16-byte aligned");
   if (n == 0) return MO_OK;

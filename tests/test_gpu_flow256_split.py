@@ -85,3 +85,27 @@ def test_fp32_mfma_adjoint_step(gpu, n):
     errs = [_rel(y1, out.detach())] + [_rel(a, b) for a, b in zip(got, want)]
     print("[flow256 fp32]  ", " ".join(f"{e:.1e}" for e in errs), flush=True)
     assert max(errs) <= 2e-6
+
+
+def test_step_beyond_2_30_floats(gpu):
+    """As many points as mo_flow256_step takes are taken with the stage
+    inputs too: beyond 2^30 floats of them (here by one point), where every
+    index into them needs 64 bits."""
+    n, k = (1 << 30) // 12 + 1, 4096
+    print(f"[flow256 split] n={n}", flush=True)
+    m, y0, _ = _problem(k, gpu)
+    y = y0.repeat(n // k + 1, 1)[:n].contiguous()
+    P = NO.flow256_pack(m)
+    want_z = torch.empty(4, k, 3, device=gpu)
+    want = NO.flow256_step(P, y0, 1.0 / STEPS, want_z)
+    got = NO.flow256_step(P, y, 1.0 / STEPS)
+    z = torch.empty(4, n, 3, device=gpu)
+    again = NO.flow256_step(P, y, 1.0 / STEPS, z)
+    assert torch.equal(got, again)
+    # a point's place in its block moves its last bits: the bar of the file
+    for lo in (0, k * (n // k // 2), k * (n // k - 1)):
+        assert _rel(got[lo:lo + k], want.double()) <= 2e-6
+        assert _rel(z[:, lo:lo + k], want_z.double()) <= 2e-6
+    tail = n - k * (n // k)
+    assert _rel(got[-tail:], want[:tail].double()) <= 2e-6
+    assert _rel(z[:, -tail:], want_z[:, :tail].double()) <= 2e-6
