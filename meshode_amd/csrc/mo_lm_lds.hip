@@ -288,40 +288,7 @@ __device__ inline void lds_solve(const LMPairDesc& P, int pid, Team& team, const
       // (the entry indices pass through opaque() so each address is one
       // bit-field extract and one shift-add)
       const unsigned* const L2e = L2 + n2;
-      // With few vertices per thread nothing else covers the two LDS round
-      // trips of a word, and there are registers for three words at once (a
-      // closed triangle mesh's vertex), entries past the list's end being the
-      // zero vector.  With the launch trimmed to the waves in use: one 642-vertex
-      // pair at 64^3 3.14 -> 3.03 ms.
-      if constexpr (VPT <= 2 && !Team::kInOrder) {
-        const unsigned none = (unsigned)(team.hbase + team.nhalo) * 0x20002u;
-        #pragma unroll 1
-        for (const unsigned* pw = L2; pw < L2e; pw += 3) {
-          unsigned w[3];
-          float4 v[6];
-          w[0] = pw[0];
-          w[1] = pw + 1 < L2e ? pw[1] : none;
-          w[2] = pw + 2 < L2e ? pw[2] : none;
-#pragma unroll
-          for (int q = 0; q < 3; ++q) {
-            v[2 * q] = VEC[__builtin_amdgcn_ubfe(w[q], 1, 15)];
-            v[2 * q + 1] = VEC[__builtin_amdgcn_ubfe(w[q], 17, 15)];
-          }
-#pragma unroll
-          for (int q = 0; q < 3; ++q) {
-            const float4 a = v[2 * q], b = v[2 * q + 1];
-            if (uniform_m != 0.f) {
-              sx += a.x + b.x; sy += a.y + b.y; sz += a.z + b.z;
-            } else {
-              const float ma = (float)((w[q] & 1u) + 1u), mb = (float)(((w[q] >> 16) & 1u) + 1u);
-              sx += ma * a.x + mb * b.x; sy += ma * a.y + mb * b.y; sz += ma * a.z + mb * b.z;
-            }
-          }
-        }
-        if (uniform_m != 0.f) {
-          sx *= uniform_m; sy *= uniform_m; sz *= uniform_m;
-        }
-      } else if (uniform_m != 0.f) {
+      if (uniform_m != 0.f) {
         #pragma unroll 1
         for (const unsigned* pw = L2; pw < L2e; ++pw) {
           const unsigned w = *pw;
@@ -948,7 +915,14 @@ __host__ __device__ inline int halo_chunk(int nv, int* chunk) {
 // radix sort).  An icosphere's numbering gives chunks of 2926 vertices up to
 // 16154 neighbours elsewhere (every old vertex's are midpoints far behind
 // it), this order at most 442; of a 41000-vertex box mesh 416 and 358.  One
-// workgroup per pair; runs beside the grid builds.
+// workgroup per pair; runs beside the grid builds (1.1 ms for 24
+// icospheres).  Every such pair is planned, whatever its numbering: also
+// where nothing hides it (templates that are there already) it costs no more
+// than the halo kernel gives back in the first LM iteration.  Direct kernel
+// and halo kernel with its plan, whole calls of one iteration and of a solve:
+// 1 pair of 20000 box vertices 2.08 -> 2.09 and 23.2 -> 20.0 ms, 16 of 8200
+// 2.24 -> 2.02 and 21.8 -> 17.8, 2 icospheres of 40962 5.02 -> 2.24 and 73.6
+// -> 20.5.
 constexpr int kPlanThreads = 512;
 static_assert(3072 * 2 >= kTagSlotWords, "a pair's team words fit its work slot");
 __device__ inline unsigned spread3(unsigned x) {   // bits 0..4 to 0, 3, .. 12
@@ -1080,7 +1054,9 @@ int launch_bucket(const LMPairDesc* pairs, const int* plist, int count, int max_
                   const LMOptionsDev& opt, LMResultDev* res, long long totalV, size_t lds_bytes, hipStream_t s) {
   auto kern = k_lm_solve_lds<T, VPT>;
   // one vertex per thread: no more waves than the largest pair needs (idle
-  // ones would still take part in every reduction)
+  // ones would still take part in every reduction).  One pair's whole call at
+  // 32^3 on 16 waves and trimmed: 128 vertices 3.21 -> 2.53 ms, 258 vertices
+  // 4.31 -> 3.70, 642 vertices 4.26 -> 4.03, 770 and more the same.
   const int threads = VPT == 1 ? std::min(T, std::max(64, (max_nv + 63) / 64 * 64)) : T;
   MO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
   // one wave of workgroups: the chip's capacity for this shape and LDS size
