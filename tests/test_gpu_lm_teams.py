@@ -51,6 +51,33 @@ def test_halo_team_any_numbering(gpu, mesh):
     assert abs(st[0]["final_cost"] - one[0]["final_cost"]) <= ENERGY_RTOL * one[0]["final_cost"]
 
 
+@pytest.mark.parametrize("side,workgroups", [(443, 64), (444, 49), (512, 64)])
+def test_halo_team_largest(gpu, side, workgroups):
+    """Sheets of side^2 vertices on either side of 64 workgroups of 3072
+    (196608), where the chunks grow to 4096, and the largest that 64 of those
+    hold (262144), against the one-workgroup kernel."""
+    print(f"[lm halo] {side} x {side}", flush=True)
+    i, j = np.meshgrid(np.arange(side), np.arange(side), indexing="ij")
+    V = np.stack([i / side, j / side, 0.1 * np.sin(9.0 * i / side + 5.0 * j / side)], -1).reshape(-1, 3)
+    k = (i * side + j)[:-1, :-1].reshape(-1)
+    F = np.concatenate([np.stack([k, k + side, k + 1], 1), np.stack([k + 1, k + side, k + side + 1], 1)]).astype(np.int32)
+    _, _, tV, tF = _pair(1000)
+    lo, hi = tV.min(0), tV.max(0)
+    pair = (lo + (hi - lo) * V * [1.0, 1.0, 0.5] + (hi - lo) * [0.0, 0.0, 0.4], F, tV, tF)
+    opt = dict(max_num_iterations=1, pcg_max_iterations=30)
+    _, st = deform.rigid_deform_batch([pair], grid_resolution=32, options=deform.default_options(**opt))
+    _, one = deform.rigid_deform_batch([pair], grid_resolution=32, options=deform.default_options(kernel_variant=1, **opt))
+    assert st[0]["solver_path_name"] == "lds_team" and st[0]["workgroups"] == workgroups
+    assert one[0]["solver_path_name"] == "one_workgroup"
+    print(f"[lm halo]   {st[0]['final_cost']:.9e} / {one[0]['final_cost']:.9e}", flush=True)
+    # the same FP32 positions and residuals, summed in FP64
+    assert abs(st[0]["initial_cost"] - one[0]["initial_cost"]) <= 1e-6 * one[0]["initial_cost"]
+    # one step cut off after 30 PCG iterations: 4e-6 apart on every size (the
+    # register/LDS kernels take hardware reciprocals in the LM diagonal, 1e-7
+    # each, which an unconverged step carries on)
+    assert abs(st[0]["final_cost"] - one[0]["final_cost"]) <= 1e-4 * one[0]["final_cost"]
+
+
 def test_halo_too_long_for_the_lds(gpu):
     """Random triangles: nearly every neighbour is in another chunk, so the
     pair stays on the kernel that reads such neighbours where they are."""
