@@ -30,11 +30,4 @@ constexpr int kSplitLayer = 3 * kSplitPlane;     // floats of one matrix
 constexpr int kPacked = kPSplit + 4 * kSplitLayer;
 static_assert(kPSplit % 4 == 0, "fragments are read as 16-byte words");
 
-// dW0 [256][3], db0, db1, db2, dW3 [3][256], db3 [3]
-constexpr int kSmallGrad = 3 * kH + 3 * kH + 3 * kH + 3;   // 2307
-
-// out[y][e] = sum over the nblocks rows of partial[y][b][e], in a fixed
-// order in FP64 (mo_flow256.hip)
-void flow256_rows_reduce(const float* partial, int nblocks, int len, int ny, float* out, hipStream_t s);
-
 }  // namespace mo

@@ -157,14 +157,14 @@ __device__ __forceinline__ void mfma_layer(const float* __restrict__ Wf, const f
   }
 }
 
-// Tout = softplus(Tin W^T + b) (forward hidden layer); with kStore Tin is
-// also copied to dst (see mfma_layer)
-template <bool kTwo, bool kStore = false>
+// Tout = softplus(Tin W^T + b) (forward hidden layer); Tin is also copied to
+// dst (see mfma_layer)
+template <bool kTwo>
 __device__ __forceinline__ void hidden_layer(const float* __restrict__ Wf, const float* __restrict__ bias,
                                              const float* __restrict__ Tin, float* __restrict__ Tout, int w,
-                                             int l, float* __restrict__ dst = nullptr, int nvalid = 0) {
+                                             int l, float* __restrict__ dst, int nvalid) {
   v16f acc0, acc1;
-  mfma_layer<kTwo, kStore>(Wf, Tin, w, l, acc0, acc1, dst, nvalid);
+  mfma_layer<kTwo, true>(Wf, Tin, w, l, acc0, acc1, dst, nvalid);
   const int u = 32 * w + (l & 31), hi = l >> 5;
   const float bu = bias[u];
 #pragma unroll
@@ -262,14 +262,14 @@ __global__ __launch_bounds__(kThreads) void k_flow256_step_save(const float* __r
       __syncthreads();
       {
         float* d1 = Hs + (0 * 4 + s) * plane + (size_t)base * kH;
-        if (nvalid > 32) hidden_layer<true, true>(P + kPW1, P + kPB1, TA, TB, w, l, d1, nvalid);
-        else hidden_layer<false, true>(P + kPW1, P + kPB1, TA, TB, w, l, d1, nvalid);
+        if (nvalid > 32) hidden_layer<true>(P + kPW1, P + kPB1, TA, TB, w, l, d1, nvalid);
+        else hidden_layer<false>(P + kPW1, P + kPB1, TA, TB, w, l, d1, nvalid);
       }
       __syncthreads();
       {
         float* d2 = Hs + (1 * 4 + s) * plane + (size_t)base * kH;
-        if (nvalid > 32) hidden_layer<true, true>(P + kPW2, P + kPB2, TB, TA, w, l, d2, nvalid);
-        else hidden_layer<false, true>(P + kPW2, P + kPB2, TB, TA, w, l, d2, nvalid);
+        if (nvalid > 32) hidden_layer<true>(P + kPW2, P + kPB2, TB, TA, w, l, d2, nvalid);
+        else hidden_layer<false>(P + kPW2, P + kPB2, TB, TA, w, l, d2, nvalid);
       }
       __syncthreads();
       store_tile(TA, Hs + (2 * 4 + s) * plane + (size_t)base * kH, nvalid);
@@ -427,6 +427,7 @@ __global__ __launch_bounds__(kThreads) void k_flow256_step_bwd(int n, const floa
 // workgroup b sums rows [R b / G, R (b + 1) / G) for unit u (coalesced rows
 // of dA1, dA2, dA3, H3) and writes the workgroup's partial row;
 // k_flow256_rows_reduce adds the rows in a fixed order (FP64).
+constexpr int kSmallGrad = 3 * kH + 3 * kH + 3 * kH + 3;   // 2307: dW0 [256][3], db0, db1, db2, dW3 [3][256], db3 [3]
 __global__ __launch_bounds__(kH) void k_flow256_grad_small(int rows, const float* __restrict__ dA1,
                                                            const float* __restrict__ dA2,
                                                            const float* __restrict__ dA3,
@@ -572,11 +573,6 @@ int cu_count() {
 }
 
 }  // namespace
-
-void flow256_rows_reduce(const float* partial, int nblocks, int len, int ny, float* out, hipStream_t s) {
-  hipLaunchKernelGGL(k_flow256_rows_reduce, dim3((len + 63) / 64, ny), dim3(512), 0, s, partial, nblocks, len, out);
-}
-
 }  // namespace mo
 
 using namespace mo;
@@ -632,7 +628,8 @@ MO_EXPORT int mo_flow256_small_grads(int64_t n, const float* dAs, const float* H
   const int nb = 256;
   hipLaunchKernelGGL(k_flow256_grad_small, dim3(nb), dim3(kH), 0, s, rows, dAs, dAs + plane4, dAs + 2 * plane4,
                      Hs + 2 * plane4, Xs, Gs, work);
-  flow256_rows_reduce(work, nb, kSmallGrad, 1, out, s);
+  hipLaunchKernelGGL(k_flow256_rows_reduce, dim3((kSmallGrad + 63) / 64, 1), dim3(512), 0, s, work, nb, kSmallGrad,
+                     out);
   MO_HIP(hipGetLastError());
   return MO_OK;
 }
@@ -652,7 +649,7 @@ MO_EXPORT int mo_flow256_dw_grads(int64_t n, const float* dAs, const float* Hs, 
   const int G = cu_count();
   hipLaunchKernelGGL(k_flow256_dw, dim3(G, 2), dim3(kThreads), 0, s, (int)(4 * n), dAs + plane4, Hs,
                      dAs + 2 * plane4, Hs + plane4, work);
-  flow256_rows_reduce(work, G, kH * kH, 2, out, s);
+  hipLaunchKernelGGL(k_flow256_rows_reduce, dim3(kH * kH / 64, 2), dim3(512), 0, s, work, G, kH * kH, out);
   MO_HIP(hipGetLastError());
   return MO_OK;
 }
