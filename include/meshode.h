@@ -516,9 +516,13 @@ int mo_ode_rk4_backward(const float* y0, int64_t n, const float* params, const f
  * b1, W2 [256,256], b2, W3 [3,256], b3 [3]; FP32 device, row-major) into
  * `packed` (mo_flow256_packed_floats() floats, device, 16-byte aligned).
  * mo_flow256_step: y0, y1 [n,3] FP32 device (distinct buffers); the
- * 256 x 256 products on bf16 MFMA with every FP32 number split exactly into
- * three bf16, at the accuracy of FP32 products (a non-finite activation
- * gives NaN). */
+ * 256 x 256 products on bf16 MFMA with every FP32 number split into three
+ * bf16, at the accuracy of FP32 products.  That holds for magnitudes from
+ * 2^-100 on (the parts of smaller ones leave bf16's normal range: output
+ * gradients scaled by 2^-110 give parameter gradients good to 6e-6, by 2^-120
+ * to 8e-3, where FP32 products lose accuracy from 2^-120 on) and below
+ * 3.39e38, bf16's largest; an activation, gradient or weight beyond it, or not
+ * finite, gives NaN. */
 int64_t mo_flow256_packed_floats(void);
 int mo_flow256_pack(const float* W0, const float* b0, const float* W1, const float* b1, const float* W2,
                     const float* b2, const float* W3, const float* b3, float* packed, void* stream);

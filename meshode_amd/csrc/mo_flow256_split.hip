@@ -2,12 +2,16 @@
 // 256 x 256 products on bf16 MFMA at 32-bit accuracy.
 //
 // An FP32 number is the exact sum of three bf16 (high, middle, low: 3 x 8
-// significant bits).  A product of two such sums is formed from the six
-// partial products of order 2^-16 and above (hh, hm, mh, mm, hl, lh); the
-// three left out are below 2^-25 of the product, under the rounding of an
-// FP32 product, and the sums are accumulated in FP32 as before; against FP64
-// the results are nearer than with FP32 MFMA (gradients of 55000 points over
-// 16 steps 3.3e-7, before 3.7e-7).  Six bf16 products cost 6/16 of the one
+// significant bits) if it is below 3.39e38, bf16's largest, and large enough
+// for its low part to be a normal bf16 (the matrix cores drop the bits of
+// others): from 2^-110 on, which the factors along a gradient's way turn into
+// about 2^-100 for dL/dy1 (2^-110 there gives 6e-6, 2^-115 2e-4).  A product
+// of two such sums is formed from the six partial products of order 2^-16 and
+// above (hh, hm, mh, mm, hl, lh); the three left out are below 2^-25 of the
+// product, under the rounding of an FP32 product, and the sums are
+// accumulated in FP32 as before; against FP64 the results are as near as with
+// FP32 MFMA or nearer (parameter gradients of 4000 points over 3 steps 1.8e-7
+// at most, there 3.4e-7).  Six bf16 products cost 6/16 of the one
 // FP32 product they replace (v_mfma_f32_32x32x16_bf16 does 1024 flops a cycle
 // on a SIMD, v_mfma_f32_32x32x2_f32 64), so the bound rises from 157 to
 // 417 TFLOP/s of FP32 work.  The bf16 MFMA drops the bits of an
@@ -34,9 +38,9 @@
 // inputs (48 B a point and step).  Per stage, last first, the backward
 // recomputes the three hidden layers, keeping softplus'(A2) in the registers
 // of the lane that will need it, and walks back through the transposed
-// products; H1, H2, dA2 and dA3 go to memory transposed ([unit][stage point], 128-byte rows of 32 points) for the
-// weight-gradient product over the step's 4 n stage points, and dW0, db0,
-// dW3, db3 are summed on the spot.  The products' partials are kept per
+// products; H1, H2, dA2 and dA3 go to memory transposed ([unit][stage point],
+// 128-byte rows of 32 points) for the weight-gradient product over the step's
+// 4 n stage points, and dW0, db0, dW3, db3 are summed on the spot.  The products' partials are kept per
 // workgroup across the steps of an integration and added in FP64 once.
 //
 // Measured, 55000 points, 16 steps: forward and gradients 54.1 -> 27.0 ms

@@ -59,6 +59,20 @@ def test_split_flow_and_adjoint(gpu, n):
     assert max(errs) <= 2e-6
 
 
+@pytest.mark.parametrize("e", [-100, -60, 60, 90])
+def test_gradient_magnitudes(gpu, e):
+    """The adjoint is linear in dL/dy1: the same bar for gradients scaled by
+    powers of two, as long as the three bf16 parts of what it multiplies are
+    normal (2^-100 leaves ten powers for the factors that make them smaller)
+    and its sums finite."""
+    print(f"[flow256 split] gradients 2^{e}", flush=True)
+    m, y0, w = _problem(300, gpu)
+    y0.requires_grad_(True)
+    got = torch.autograd.grad(NO.odeint_rk4(m, y0, steps=STEPS), [y0, *m.parameters()], w * 2.0 ** e)
+    _, want = _reference(m, y0.detach(), w)
+    assert max(_rel(a.double() * 2.0 ** -e, b) for a, b in zip(got, want)) <= 2e-6
+
+
 @pytest.mark.parametrize("n", [33, 1000])
 def test_fp32_mfma_adjoint_step(gpu, n):
     print(f"[flow256 fp32] n={n}", flush=True)
