@@ -800,12 +800,20 @@ int lm_core(const std::vector<CorePair>& pairs, const mo_lm_options& opt, mo_lm_
   std::vector<TopoPairDesc> h_topo(np);
   std::vector<PairIO> h_io(np);
   long long max_nv_io = 1;
+  const size_t lds_cap = (size_t)std::max(0, device_lds_limit() - 4096);
+  bool plan = false;
   for (int p = 0; p < np; ++p) {
     const CorePair& c = pairs[p];
     h_io[p] = PairIO{c.x0, c.xstart, c.sp, c.out, vbase[p], c.nv};
     max_nv_io = std::max(max_nv_io, c.nv);
     const bool weighted = c.kind == 2;
     h_pairs[p] = LMPairDesc{c.grid, c.N, (int)c.nv, vbase[p], 0, weighted ? 1.0f : (float)c.lambda, weighted ? 1 : 0};
+    // (a closed mesh names each edge in two half-edges, a graph in one)
+    if (opt.kernel_variant == 0 && !weighted &&
+        lm_lds_wants_plan(c.nv, c.kind == 0 ? 3 * c.nidx : 2 * c.nidx, lds_cap)) {
+      h_pairs[p].flags |= kPairPlan;
+      plan = true;
+    }
     h_topo[p] = TopoPairDesc{c.idx, c.kind == 0 ? 3 * c.nidx : c.nidx, vbase[p], (int)c.nv, c.kind == 0 ? 0 : 1};
   }
   // With work to enqueue in between (a batch's grid builds), the topology
@@ -844,11 +852,8 @@ int lm_core(const std::vector<CorePair>& pairs, const mo_lm_options& opt, mo_lm_
   hipLaunchKernelGGL(k_make_x0, io_grid, dim3(256), 0, ts, d_io, deg, x0, u);
   MO_HIP(hipGetLastError());
   // per pair and register/LDS team shape: the largest chunk's adjacency entries
-  const size_t lds_cap = (size_t)std::max(0, device_lds_limit() - 4096);
   const LMArrays A{x0, u, adj, raw, work, wt};
-  if ((rc = lm_lds_chunk_entries(d_pairs, A, np, nvalloc, opt.kernel_variant == 0 ? (int)max_nv : 0, lds_cap, d_chunk,
-                                 ts)))
-    return rc;
+  if ((rc = lm_lds_chunk_entries(d_pairs, A, np, nvalloc, plan, lds_cap, d_chunk, ts))) return rc;
   std::vector<int> pstat(2 * np), hchunk(4 * np);
   int herr = 0;
   {

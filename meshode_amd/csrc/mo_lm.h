@@ -18,8 +18,9 @@ struct LMPairDesc {
   long long vbase;        // offset of this pair in the per-vertex arrays
   long long ebase;        // offset of this pair in the adjacency entry array
   float lambda;           // rigidity weight (EdgeLoss lambda); 1 for weighted pairs
-  int flags;              // bit 0: per-entry edge weights in LMArrays::wt
+  int flags;              // bit 0: per-entry edge weights in LMArrays::wt; kPairPlan
 };
+constexpr int kPairPlan = 2;   // LMPairDesc::flags: lm_lds_wants_plan
 
 // Solver options; defaults restate Ceres' Solver::Options defaults that
 // deformer.cc:55-59 leaves untouched (max_num_iterations = 100).
@@ -127,9 +128,12 @@ int lm_lds_team_max();   // largest team of the register/LDS team kernel
 int lm_lds_team_shape(int b, int* threads, int* vertices_per_thread);
 size_t lm_lds_team_bytes(int chunk, long long entries);
 int lm_lds_team_capacity(int b, size_t lds_bytes);
-// max_nv: the batch's largest pair; lds_cap: dynamic LDS a workgroup may use.
+// Whether a pair of nv vertices and about `entries` adjacency entries is
+// planned for the halo kernel; lds_cap: dynamic LDS a workgroup may use.
+bool lm_lds_wants_plan(long long nv, long long entries, size_t lds_cap);
+// plan: some pair is marked kPairPlan.
 int lm_lds_chunk_entries(const LMPairDesc* pairs_dev, const LMArrays& arrays, int np, long long total_vertices,
-                         int max_nv, size_t lds_cap, int* out_dev, hipStream_t s);
+                         bool plan, size_t lds_cap, int* out_dev, hipStream_t s);
 // Team shape, chunk and workgroups of the halo kernel for a pair of nv
 // vertices (-1: too large).
 int lm_lds_halo_shape(int nv, int* chunk, int* workgroups);

@@ -895,6 +895,8 @@ __global__ void __launch_bounds__(256) k_chunk_entries(const LMPairDesc* __restr
   if (threadIdx.x == 3) out[4 * p + 3] = padded;
 }
 
+constexpr int kSoloVertices = 8192;   // most vertices of a one-workgroup shape
+
 // Chunks of a halo team: 3072 vertices per workgroup, 4096 beyond
 // kMaxTeam of those (0: too large for either).
 __host__ __device__ inline int halo_chunk(int nv, int* chunk) {
@@ -907,8 +909,8 @@ __host__ __device__ inline int halo_chunk(int nv, int* chunk) {
   return 0;
 }
 
-// Pairs that can't be solved by one register/LDS workgroup (lds_cap: its
-// LDS) but by a halo team: the vertices' spatial order (work slot gOrder:
+// The pairs marked kPairPlan that can't be solved by one register/LDS
+// workgroup (lds_cap: its LDS) but by a halo team: the vertices' spatial order (work slot gOrder:
 // perm, inv) and minus the team's LDS bytes in out[4 p + 3], which keeps
 // the one-workgroup kernel's entry count otherwise.  The order is that of a
 // 32^3 grid's Morton codes over the mesh's box, ties by index (a stable
@@ -916,7 +918,7 @@ __host__ __device__ inline int halo_chunk(int nv, int* chunk) {
 // 16154 neighbours elsewhere (every old vertex's are midpoints far behind
 // it), this order at most 442; of a 41000-vertex box mesh 416 and 358.  One
 // workgroup per pair; runs beside the grid builds (1.1 ms for 24
-// icospheres).  Every such pair is planned, whatever its numbering: also
+// icospheres).  They are planned whatever their numbering: also
 // where nothing hides it (templates that are there already) it costs no more
 // than the halo kernel gives back in the first LM iteration.  Direct kernel
 // and halo kernel with its plan, whole calls of one iteration and of a solve:
@@ -941,7 +943,7 @@ __global__ void __launch_bounds__(kPlanThreads) k_chunk_plan(const LMPairDesc* _
   int chunk = 0;
   const int c = halo_chunk(nv, &chunk);
   const int padded = out[4 * p + 3];
-  if ((P.flags & 1) || c < 2 || (nv <= 8192 && padded < 65536 && lm_lds_bytes_dev(nv, padded) <= (size_t)lds_cap)) return;
+  if (!(P.flags & kPairPlan) || (nv <= kSoloVertices && padded < 65536 && lm_lds_bytes_dev(nv, padded) <= (size_t)lds_cap)) return;
   unsigned long long* slots = pair_slots(A, totalV, P.vbase);   // the team's words start at zero
   for (int k = tid; k < kTagSlotWords; k += kPlanThreads) slots[k] = 0ull;
   const float4* X0 = A.x0 + P.vbase;
@@ -1210,14 +1212,29 @@ int lm_lds_team_capacity(int b, size_t lds_bytes) {
   }
 }
 
-int lm_lds_chunk_entries(const LMPairDesc* pairs_dev, const LMArrays& A, int np, long long totalV, int max_nv,
+// A pair is planned where its vertex count, or the adjacency that its edge
+// count gives a closed mesh (half the vertices' lists padded by one), is more
+// than one workgroup holds.  The counts alone decide, so that a pair's kernel
+// does not depend on the batch, and no plan is launched where none is needed:
+// its workgroups, two waves per SIMD, do not get in between a running grid
+// build's single waves, and for 512 pairs of 5000 vertices, which it leaves
+// alone, it held the solver's launch back to that build's end (pipelined
+// batches of 512 62.3 ms, without it 60.5; of 256 31.6 and 30.3).  A mesh whose adjacency outgrows the
+// estimate takes the direct team kernel.
+bool lm_lds_wants_plan(long long nv, long long entries, size_t lds_cap) {
+  int chunk = 0;
+  const long long padded = entries + nv / 2;
+  return nv > 3072 && nv <= (long long)kMaxTeam * 4096 && halo_chunk((int)nv, &chunk) >= 2 &&
+         (nv > kSoloVertices || padded >= 65536 || lm_lds_bytes_dev((int)nv, padded) > lds_cap);
+}
+
+int lm_lds_chunk_entries(const LMPairDesc* pairs_dev, const LMArrays& A, int np, long long totalV, bool plan,
                          size_t lds_cap, int* out_dev, hipStream_t s) {
   if (np <= 0) return MO_OK;
   hipLaunchKernelGGL(k_chunk_entries, dim3(np), dim3(256), 0, s, pairs_dev, A.adj, np,
                      kTeamT[0] * kTeamVPT[0], kTeamT[1] * kTeamVPT[1], kTeamT[2] * kTeamVPT[2], out_dev);
   MO_HIP(hipGetLastError());
-  // pairs below 3073 vertices are never split
-  if (max_nv > 3072) {
+  if (plan) {
     hipLaunchKernelGGL(k_chunk_plan, dim3(np), dim3(kPlanThreads), 0, s, pairs_dev, A, totalV, (int)lds_cap, out_dev);
     MO_HIP(hipGetLastError());
   }

@@ -96,6 +96,29 @@ def test_halo_too_long_for_the_lds(gpu):
     assert abs(st[0]["final_cost"] - one[0]["final_cost"]) <= ENERGY_RTOL * one[0]["final_cost"]
 
 
+def test_planned_pairs_do_not_depend_on_the_batch(gpu):
+    """Which pairs get a spatial order is decided by their own counts: pairs
+    around what one workgroup's LDS holds (5700 vertices of a closed mesh),
+    and one of unshared edges whose adjacency is twice what its counts
+    suggest, alone and beside pairs that are planned."""
+    print("[lm halo] batches", flush=True)
+    rng = np.random.default_rng(8)
+    V, F, tV, tF = _pair(5000)
+    soup = rng.permutation(np.arange(5000 * 5, dtype=np.int32) % 5000)[:24000].reshape(-1, 3)
+    soup = soup[(soup[:, 0] != soup[:, 1]) & (soup[:, 1] != soup[:, 2]) & (soup[:, 2] != soup[:, 0])]
+    pairs = [_pair(n, seed=n) for n in (3072, 5600, 5800, 8190, 8194)] + [(V, soup, tV, tF)]
+    opt = deform.default_options(max_num_iterations=3)
+    out, st = deform.rigid_deform_batch(pairs, grid_resolution=32, options=opt)
+    assert [s["solver_path_name"] for s in st] == ["lds", "lds", "lds_team", "lds_team", "lds_team", "lds_team"]
+    for k, p in enumerate(pairs):
+        alone, sa = deform.rigid_deform_batch([p], grid_resolution=32, options=opt)
+        assert torch.equal(alone[0], out[k]) and sa[0]["solver_path_name"] == st[k]["solver_path_name"], k
+    # the soup against the one-workgroup kernel
+    _, one = deform.rigid_deform_batch([pairs[-1]], grid_resolution=32,
+                                       options=deform.default_options(kernel_variant=1, max_num_iterations=3))
+    assert abs(st[-1]["final_cost"] - one[0]["final_cost"]) <= ENERGY_RTOL * one[0]["final_cost"]
+
+
 def test_small_pairs_any_launch_width(gpu):
     """1 to 16 waves per workgroup and both sides of a wave's 64 vertices;
     an open mesh (mixed multiplicities, odd lists) among them."""
