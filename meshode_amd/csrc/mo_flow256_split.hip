@@ -47,7 +47,10 @@
 // with the FP32 MFMA kernels before (whose adjoint also moved 3.8 GB a step
 // through memory, now 1.8 GB); a forward step 676 -> 356 us (983 TFLOP/s of
 // bf16 products, where an 8192^3 library product reaches 1118), an adjoint
-// step about 950 + 368 us; 5001 points forward 2980 -> 890 us for 16 steps.
+// step 967 + 390 us (k_flow256_adj spills 33 VGPRs, 132 bytes a lane, and
+// k_flow256_adj_dw 6); 5001 points forward 2980 -> 870 us for 16 steps, on 157
+// workgroups of 32 points (99 CUs have none).  MFMA busy 46, 32 and 37% of the
+// time (forward, adjoint, weight gradients).
 #include <algorithm>
 
 #include "mo_common.h"

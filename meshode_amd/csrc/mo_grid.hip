@@ -12,7 +12,9 @@
 // is compiled with -ffp-contract=off: every FP64 operation is one IEEE
 // rounding, so results are bit-reproducible on the host.
 //
-// Kernel structure (HBM traffic is tiny; the build is FP64-VALU bound):
+// Kernel structure (HBM traffic is small; the build is bound by VALU issue,
+// 73% of the SIMDs' cycles for 512 box-union grids, the FP64 exact tests and
+// the FP32 bounds about half each):
 //   1. k_face_bins   : per face, index check + Morton bin of the centroid
 //                      (16^3 bins).
 //   2. k_bin_sort    : one workgroup counting-sorts face indices by bin (LDS
@@ -42,6 +44,8 @@
 //                      and plane bounds can still improve some lane.  Ties
 //                      keep the lowest face index, so the visiting order
 //                      never changes the result.
+//   6. k_grid_heavy  : the bricks whose walk is long, again on 16 wavefronts
+//                      each.
 #include "mo_common.h"
 #include "mo_grid.h"
 
@@ -167,9 +171,10 @@ __device__ inline float round_up(double x) {
 
 // Pass 3: FP64 face record of face perm[pos] and its FP32 culling record,
 // written at its sorted position.
-// At most 64 VGPRs (8 wavefronts per SIMD): the kernel then fits beside a
-// running grid build's wavefronts (85 VGPRs, 5 per SIMD), so a second
-// batch's face preparation is not held back until that build ends.
+// At most 64 VGPRs and one wavefront per SIMD and workgroup: a running grid
+// build (95 VGPRs, 5 wavefronts per SIMD) leaves room for it whenever one of
+// its wavefronts ends, so a second batch's face preparation is not held back
+// until that build ends.
 __global__ void __launch_bounds__(256, 8) k_face_prep(const GridJob* __restrict__ jobs) {
   const GridJob J = jobs[blockIdx.y];
   const double* __restrict__ V = J.V;
@@ -893,11 +898,13 @@ int grid_build_batch_launch(const GridSpec* specs, int n, void* workspace, hipSt
   // Where a brick is handed over: the tail matters the more the fewer bricks
   // share the chip, the work done twice the more the more there are: a
   // multiple of the square root of the launch's bricks (34 tiles for one 64^3
-  // grid, 96 for one 128^3 grid, 768 for 512 64^3 grids).  Multiples 0.25,
-  // 0.5, 1, 2, 4: a 642-vertex pair 3.15, 3.15, 3.22, 3.43, 3.80 ms, a
-  // 128^3 template 4.90, 5.25, 4.69, 4.87, 5.68 ms, 48 mixed pairs 125, 116,
-  // 114, 115, 116 ms; with 4 or 8 wavefronts in the second kernel each of
-  // the three is slower.
+  // grid, 96 for one 128^3 grid, 768 for 512 64^3 grids).  Multiples 0.5,
+  // 0.75, 1: one 5000-vertex box target at 64^3 0.48, 0.49, 0.54 ms, a
+  // 2562-vertex sphere at 50^3 0.78, 0.85, 0.92, a 642-vertex pair 2.76, 2.81,
+  // 2.84, a 10242-vertex sphere at 128^3 5.12, 4.92, 4.60, 48 mixed pairs
+  // 76.1, 74.7, 73.8: small launches want less, large ones more.  0.25, 2 and
+  // 4 are behind on one side or both, and so are 4 or 8 wavefronts in the
+  // second kernel.
   const int max_tiles_brick = std::max(16, (int)(0.75 * std::sqrt((double)bricks)));
   hipLaunchKernelGGL(k_grid_build, dim3((unsigned)max_bricks, n), dim3(64), 0, stream, d_jobs, queue,
                      max_tiles_brick);

@@ -743,7 +743,8 @@ __device__ inline unsigned long long* pair_slots(const LMArrays& A, long long to
 
 // Large pairs with their halo in LDS; wg as for k_lm_solve_lds_team.  Bound
 // by the two exchanges and the halo copy of a PCG iteration (about 10 us at
-// three vertices per thread).  Twelve icospheres each of 10242 and 40962
+// three vertices per thread).  1024x3 spills 20 registers, 1024x4 44 (76 and
+// 124 bytes of scratch a lane).  Twelve icospheres each of 10242 and 40962
 // vertices, 50 steps of 30 PCG iterations: 55.7 ms on k_lm_solve_lds_team,
 // whose gather waits for a remote read per neighbour, 14.9 ms here.
 template <int T, int VPT>
@@ -1086,7 +1087,7 @@ static const int kShapeT[] = {1024, 1024, 1024, 1024, 512, 512, 512, 512, 256, 2
 static const int kShapeVPT[] = {1, 2, 4, 5, 8, 10, 12, 16, 20, 24, 32, 6, 7};
 constexpr int kNumShapes = 13;
 // built-in preference: 768x7 ahead of 1024x5 (5000-vertex pairs: 36.3 against
-// 37.3 ms per 512-pair launch; both spill < 20 VGPRs), otherwise by capacity
+// 37.3 ms per 512-pair launch; they spill 40 and 46 VGPRs), otherwise by capacity
 static const int kPref[kNumShapes] = {0, 1, 2, 12, 3, 4, 11, 5, 6, 7, 8, 9, 10};
 
 static std::mutex g_shape_mu;
@@ -1164,8 +1165,8 @@ int lm_lds_team_shapes() { return kHaloShape + 2; }
 // Preference order of the team shapes: 1024x3, then 1024x4 (only for pairs
 // whose 3072-vertex team would exceed kMaxTeam), then 1024x2 (chunks whose
 // adjacency does not fit the LDS otherwise) -- 1024x3 solved 12k-100k vertex
-// pairs as fast as 1024x4 and 4% faster on 41k-vertex icospheres (its
-// register allocation spills 6 values against 33) -- or
+// pairs as fast as 1024x4 and 4% faster on 41k-vertex icospheres (it spills
+// no register, 1024x4 20) -- or
 // MO_LM_TEAM_VPT="v,v,..." (vertices per thread, e.g. "2,4") read once.
 const std::vector<int>& lm_lds_team_order() {
   static const std::vector<int> order = [] {

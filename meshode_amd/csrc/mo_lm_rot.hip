@@ -491,13 +491,17 @@ __global__ void __launch_bounds__(256) k_lm_rot_team(const RotPairDesc* __restri
 // records and its halo's, and the adjacency with the edge vectors.  A PCG
 // iteration publishes z = M^-1 r once, loads the halo's records, forms
 // A z, p = z + beta p and A p = A z + beta A p_prev, and needs the two
-// reductions of CG and no other exchange; the team protocol is TagTeam.
+// reductions of CG and no other exchange; the team protocol is TagTeam.  (A p
+// is thus a recurrence, where k_lm_rot forms each product anew.  Whole solves
+// of ten box unions of 300 to 5000 vertices, 2 to 6 thousand PCG iterations,
+// here and there: the same number of PCG iterations within 3%, final costs
+// -3e-6 to 4e-5 apart.)
 // What bounds it: the two exchanges and the halo load of an iteration, each
 // a round trip through memory shared by the XCDs, not arithmetic (about
 // 5.7 us an iteration).  One 5000-vertex problem (20 chunks, 4600 PCG
 // iterations): 26.3 ms, where k_lm_rot takes 990 ms on its one CU.  Chunks
-// of 256 put one wavefront on each SIMD of a CU; 21 VGPRs of the cold parts
-// spill at two workgroups per CU.
+// of 256 put one wavefront on each SIMD of a CU; both instances spill 21 VGPRs
+// (84 bytes a lane).
 __device__ inline float3 cross3(float3 a, float3 b) {
   return make_float3(a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x);
 }
