@@ -51,12 +51,13 @@ def lm_algorithmic_flops(nv, entries, lm_iters, pcg_iters):
                  lm_iters * (LM_ITER_FLOPS_BASE + LM_ITER_FLOPS_PER_ENTRY * ev))
 
 
-# Flop model of the grid build (FP64, no FMA contraction): 60 flops per
+# Flop model of the grid build: 60 FP64 flops (no FMA contraction) per
 # point-triangle distance evaluation (face-region test, or the three
-# canonical edge distances) and 25 per face bound check (point-to-AABB and
-# plane bounds); both counts come live from the kernel (mo_last_grid_stats).
-# rocprofv3's SQ_INSTS_VALU_FLOPS_FP64 on the headline launch reads 9.3e11
-# flops against this model's ~7e11 (the rest: tile scans and seeding).
+# canonical edge distances) and 25 FP32 ones per face bound check
+# (point-to-AABB and plane bounds); both counts come live from the kernel
+# (mo_last_grid_stats).  rocprofv3 counts every lane of an instruction, the
+# idle ones of divergent evaluations too: 3.80e11 FP64 and 2.21e11 FP32 flops
+# on the headline launch (SQ_INSTS_VALU_FLOPS_FP64 / _FP32 x 64).
 GRID_FLOPS_PER_EXACT, GRID_FLOPS_PER_BOUND = 60, 25
 
 
@@ -74,13 +75,15 @@ def adjacency_entries(F):
 # 1.99975 and WRITE_SIZE x 1.0, the factors a plain 256 MiB copy reads) on
 # the default workload; keyed by (kernel, pairs, distinct pairs, source
 # verts, grid); other workloads report null.
-MEASURED_TRAFFIC = {("k_lm_solve_lds", 512, 128, 5000, 64): 28.03e9}
+MEASURED_TRAFFIC = {("k_lm_solve_lds", 512, 128, 5000, 64): 28.03e9,
+                    ("k_grid_build", 512, 128, 5000, 64): 8.28e9}
 # Wavefront VALU instructions per launch (rocprofv3 SQ_INSTS_VALU, same
 # workload and key): with the live launch time they give the fraction of the
 # SIMDs' issue cycles the kernel's VALU work fills (a wave64 VALU
 # instruction occupies a SIMD 4 cycles; 1024 SIMDs at 2.4 GHz), which is
 # what bounds both kernels.
-MEASURED_VALU_INSTS = {("k_lm_solve_lds", 512, 128, 5000, 64): 1.252e10}
+MEASURED_VALU_INSTS = {("k_lm_solve_lds", 512, 128, 5000, 64): 1.252e10,
+                       ("k_grid_build", 512, 128, 5000, 64): 1.405e10}
 SIMDS, ENGINE_HZ = 1024, 2.4e9
 
 
@@ -279,9 +282,10 @@ def main():
             lat.append((s["clock_end"] - tm["clock_start"]) / tm["clock_hz"] * 1e3)
     lat = np.array(lat)
 
-    # rooflines: the grid build (FP64 VALU, work counted live by the
-    # kernel) and the LM solver (FP32 VALU, algorithmic flop model); the one
-    # with the longer live time is the dominant kernel
+    # rooflines: the grid build (FP64 VALU for its exact tests, FP32 for its
+    # bounds, work counted live by the kernel) and the LM solver (FP32 VALU,
+    # algorithmic flop model); the one with the longer live time is the
+    # dominant kernel
     nv = np.array([len(p[0]) for p in pairs])
     ent_d = [adjacency_entries(p[1]) for p in distinct]
     ent = np.array([ent_d[i % len(distinct)] for i in range(len(pairs))])
@@ -293,7 +297,8 @@ def main():
     lm_ms = float(np.mean([t["lm_ms"] for t in timings]))
     grid_ms = float(np.mean([t["grid_ms"] for t in timings]))
     gs = _lib.last_grid_stats()
-    grid_flops = GRID_FLOPS_PER_EXACT * gs["exact_tests"] + GRID_FLOPS_PER_BOUND * gs["bound_checks"]
+    grid_flops = GRID_FLOPS_PER_EXACT * gs["exact_tests"]
+    bound_flops = GRID_FLOPS_PER_BOUND * gs["bound_checks"]
     lm_tf = float(np.mean(lm_flops)) / (lm_ms / 1e3) / 1e12
     grid_tf = grid_flops / (grid_ms / 1e3) / 1e12
     cells = int(sum(args.grid ** 3 for _ in pairs))
@@ -307,7 +312,8 @@ def main():
                  "exact_tests_needed_per_cell": gs["exact_tests_needed"] / cells,
                  "bound_checks_per_cell": gs["bound_checks"] / cells,
                  "tiles_per_64_cells": 64 * gs["tiles"] / max(1, cells),
-                 "bound_check_flop_share": GRID_FLOPS_PER_BOUND * gs["bound_checks"] / max(grid_flops, 1)}
+                 "fp32_bound_tflops": bound_flops / (grid_ms / 1e3) / 1e12,
+                 "bound_check_flop_share": bound_flops / max(grid_flops + bound_flops, 1)}
     roof_lm = {"kernel": "k_lm_solve_lds", "bound": "fp32-valu", "achieved": lm_tf, "peak": FP32_VALU_PEAK_TFLOPS,
                "unit": "TFLOP/s", "frac": lm_tf / FP32_VALU_PEAK_TFLOPS,
                "traffic": MEASURED_TRAFFIC.get(("k_lm_solve_lds",) + wkey),

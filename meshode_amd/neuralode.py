@@ -5,26 +5,27 @@ cad_neural_deform2.py:40-108, in the configuration of the config-3 workload).
   3 -> 256 -> 256 -> 256 -> 3 with softplus, Xavier-uniform weights from a
   seed, zero biases.  The reference centres its input the same way
   (neuralode_fast.py:28-32; it also feeds t, which this field does not use).
-  The 256x256 layers are FP32 GEMMs (hipBLASLt, on the MFMA units).
+  As a module its 256x256 layers are FP32 GEMMs (hipBLASLt, on the MFMA
+  units).
 * ``odeint_rk4``: fixed-grid RK4 over t in [0, 1] with ``steps`` equal steps
   using the 3/8-rule step that torchdiffeq's ``method="rk4"`` applies
   (the reference calls ``odeint(..., method="rk4")``, neuralode_fast.py:55-60):
       k1 = f(y); k2 = f(y + h k1/3); k3 = f(y + h (k2 - k1/3));
       k4 = f(y + h (k1 - k2 + k3)); y' = y + h (k1 + 3 k2 + 3 k3 + k4) / 8.
 * On the GPU, with a 256-wide field in FP32, each forward step of
-  ``odeint_rk4`` is one fused HIP kernel (``mo_flow256_step``: the four
-  stages, the 256 x 256 layers on FP32 MFMA, softplus in their epilogue);
-  the parameters are packed once per call (``mo_flow256_pack``).  The
-  adjoint's recomputation saves each step's activations
-  (``mo_flow256_step_save``), a second kernel runs the backward through the
-  four stages (``mo_flow256_step_backward``, the transposed 256 x 256
-  products on MFMA), and the parameter gradients are GEMMs over the saved
-  tensors.
+  ``odeint_rk4`` is one fused HIP kernel (``mo_flow256_step_stages``: the
+  four stages, the 256 x 256 products on bf16 MFMA with FP32 operands split
+  in three, softplus in their epilogue); the parameters are packed once per
+  call (``mo_flow256_pack``).  Where a gradient may be asked for, a step also
+  writes its four stage inputs; the adjoint (``mo_flow256_adjoint_step``)
+  recomputes a step's activations from them on chip while it goes back
+  through its stages, and adds the parameter gradients to partial sums that
+  ``mo_flow256_adjoint_grads`` adds up once.
 * ``RK4Adjoint``: the gradient of the discretized flow (discrete adjoint).
-  The forward keeps only the state at each step boundary (one checkpoint
-  per step); the backward recomputes one step at a time from its
-  checkpoint and back-propagates through its four stages, so memory is one
-  step's activations instead of all ``4 * steps`` evaluations.
+  The forward keeps the state at each step boundary (the fused one the four
+  stage inputs, 48 B a point and step); the backward recomputes one step at a
+  time from them and back-propagates through its four stages, so memory is
+  one step's activations instead of all ``4 * steps`` evaluations.
 * ``DistanceRigidityLoss``: 1/2 sum d(y)^2 over all pushed points (the
   pyDeform distance kernels) + 1/2 rho^2 sum ||(y_b - y_a) - (y0_b - y0_a)||^2
   over the source mesh edges (the graph-edge kernels).
@@ -105,7 +106,7 @@ def flow256_step(packed, y, h, stages=None):
 
 class RK4Adjoint(Function):
     """y1 = Phi(y0; theta) for ``steps`` RK4 steps; backward by recomputation
-    from per-step checkpoints."""
+    from what each step keeps."""
 
     @staticmethod
     def forward(ctx, y0, steps, func, *params):

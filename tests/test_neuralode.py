@@ -167,8 +167,8 @@ def test_gpu_flow_and_loss_against_fp64(gpu, oracle):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [1, 64, 100, 55000])
 def test_gpu_fused_flow256_step_against_fp64(gpu, n):
-    """mo_flow256_step (the four RK4 stages of the 256-wide field on FP32
-    MFMA) against the FP64 torch step with the same weights: y1 within 1e-5
+    """mo_flow256_step (the four RK4 stages of the 256-wide field on bf16
+    MFMA with split FP32 operands) against the FP64 torch step with the same weights: y1 within 1e-5
     of the FP64 step's increment scale, or within 1.5 times the float32 torch
     step's own error where that is larger; points inside and outside the
     unit box."""
@@ -213,7 +213,7 @@ def test_gpu_odeint_uses_fused_step(gpu, monkeypatch):
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [40, 1000])
 def test_gpu_fused_adjoint_against_fp64(gpu, n):
-    """The fused adjoint (mo_flow256_step_save / _backward + GEMMs) of a
+    """The fused adjoint (mo_flow256_adjoint_step / _grads) of a
     4-step integration against FP64 autograd through the same steps: the
     parameter gradients and dL/dy0 within 1e-4 (relative, in norm); 40
     points exercise the one-block (at most 32 points) path."""
