@@ -1062,11 +1062,18 @@ int launch_bucket(const LMPairDesc* pairs, const int* plist, int count, int max_
   // 4.31 -> 3.70, 642 vertices 4.26 -> 4.03, 770 and more the same.
   const int threads = VPT == 1 ? std::min(T, std::max(64, (max_nv + 63) / 64 * 64)) : T;
   MO_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes));
-  // one wave of workgroups: the chip's capacity for this shape and LDS size
+  // one wave of workgroups: the chip's capacity for this shape and LDS size,
+  // with the waves of a workgroup counted as a multiple of the CU's four
+  // SIMDs.  Ten waves lie 3, 3, 2, 2: a second such workgroup would put a
+  // sixth on a SIMD that holds five of this kernel, so it waits for the CU to
+  // empty, where a resident workgroup takes the next pair as soon as it has
+  // one (280 pairs of 602 vertices, LM: two workgroups counted per CU 9.4 ms,
+  // one 7.2; 512 pairs 9.5 either way).
   int dev = 0, cus = 0, per = 0;
   MO_HIP(hipGetDevice(&dev));
   MO_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-  MO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)kern, threads, lds_bytes));
+  MO_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, (const void*)kern, (threads + 255) / 256 * 256,
+                                                      lds_bytes));
   const int nwg = std::max(1, std::min(count, std::max(per, 1) * std::max(cus, 1)));
   hipLaunchKernelGGL(kern, dim3(nwg), dim3(threads), lds_bytes, s, pairs, plist, count, next, A, opt, res, totalV,
                      (unsigned)lds_bytes);

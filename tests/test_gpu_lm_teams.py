@@ -119,6 +119,19 @@ def test_planned_pairs_do_not_depend_on_the_batch(gpu):
     assert abs(st[-1]["final_cost"] - one[0]["final_cost"]) <= ENERGY_RTOL * one[0]["final_cost"]
 
 
+@pytest.mark.parametrize("n", [200, 258, 514, 602, 770])
+def test_more_small_pairs_than_workgroups(gpu, n):
+    """600 pairs of 4, 5, 9, 10 and 13 waves: more than the chip holds of the
+    wider ones, so workgroups take further pairs; each pair as alone."""
+    print(f"[lm small] 600 pairs of {n}", flush=True)
+    pairs = [_pair(n, seed=3 + k) for k in range(4)]
+    opt = deform.default_options(max_num_iterations=3)
+    out, st = deform.rigid_deform_batch([pairs[k % 4] for k in range(600)], grid_resolution=16, options=opt)
+    for k in range(4):
+        alone, _ = deform.rigid_deform_batch([pairs[k]], grid_resolution=16, options=opt)
+        assert all(torch.equal(alone[0], out[j]) for j in range(k, 600, 4))
+
+
 def test_small_pairs_any_launch_width(gpu):
     """1 to 16 waves per workgroup and both sides of a wave's 64 vertices;
     an open mesh (mixed multiplicities, odd lists) among them."""
