@@ -121,8 +121,8 @@ int lm_lds_launch(int bucket, const LMPairDesc* pairs_dev, const int* plist, int
 // abort_flag as for lm_team_launch.  Returns kCoopRefused like
 // lm_team_launch.
 int lm_lds_team_shapes();
-// Team shapes in preference order (MO_LM_TEAM_VPT overrides the default
-// largest-chunk-first order).
+// Shapes 0..2 in preference order: 1024x3, 1024x4, 1024x2, or
+// MO_LM_TEAM_VPT's (no effect on the halo kernel's pairs).
 const std::vector<int>& lm_lds_team_order();
 int lm_lds_team_max();   // largest team of the register/LDS team kernel
 int lm_lds_team_shape(int b, int* threads, int* vertices_per_thread);
